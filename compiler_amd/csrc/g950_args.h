@@ -136,4 +136,17 @@ struct AttnVarArgs {
   int dtype;   // general kernel: q/k/v/o dtype
 };
 
+// Attention of few queries over long keys (attn_decode.hip).  Records of one
+// (sequence, KV head) pair: rows (query x head of the group), each with
+// `splits` key ranges.
+struct AttnDecArgs {
+  AttnArgs a;
+  VarlenArgs v;
+  float* part;  // splits > 1: [pairs * rows * splits][D] unnormalised O
+  float* ml;    //             [pairs * rows * splits][2] maximum (log2 units), sum
+  int splits;   // key ranges per pair
+  int chunk;    // keys per range but the last, which takes the rest (multiple of 16)
+  int rows;     // seqlen_q * group
+};
+
 }  // namespace g950

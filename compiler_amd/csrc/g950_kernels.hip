@@ -4,4 +4,5 @@
 #include "rowreduce.hip"
 #include "gemm.hip"
 #include "attention.hip"
+#include "attn_decode.hip"
 #include "dequant.hip"

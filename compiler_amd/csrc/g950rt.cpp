@@ -42,6 +42,10 @@ struct g950_module {
   // ordered, so each stream owns one buffer, grown on demand
   std::mutex ws_mu;
   std::unordered_map<void*, std::pair<void*, size_t>> ws;
+  // held by a call from its first use of the workspace until its last launch
+  // is queued, so calls of several threads on one stream do not interleave
+  // their launches on one buffer
+  std::mutex ws_use;
   // device address of the library's static scratch array on this device
   // (g950_launch_noalloc), looked up at open; null with scratch_err set if the
   // lookup failed
@@ -61,6 +65,9 @@ thread_local std::string t_kernel;
 // workspace request instead of hipMalloc.
 thread_local char* t_scratch = nullptr;
 constexpr size_t kScratchWorkspace = G950_NOALLOC_SCRATCH_BYTES;
+// The call's hold on its module's workspace (g950_module::ws_use), taken by
+// workspace() and dropped when the call returns.
+thread_local std::unique_lock<std::mutex> t_ws_use;
 
 int fail(int code, const char* fmt, ...) {
   char buf[512];
@@ -284,6 +291,7 @@ int workspace(g950_module* m, void* stream, size_t bytes, void** out) {
     *out = t_scratch;
     return G950_OK;
   }
+  if (!t_ws_use.owns_lock()) t_ws_use = std::unique_lock<std::mutex>(m->ws_use);
   std::lock_guard<std::mutex> lock(m->ws_mu);
   auto& w = m->ws[stream];
   if (w.second < bytes) {
@@ -1279,6 +1287,64 @@ long long rows_held(long long n, long long rs, long long nh, long long hs, long 
   return rs > 0 ? (long long)((n - fixed) / rs) + 1 : 0x7FFFFFFF;
 }
 
+// Workspace for a route that also works without one (null: take it without).
+// Not from the no-alloc scratch array: such calls may overlap on several
+// streams as long as their routes leave it alone.  Not under stream capture:
+// nothing can be allocated there, and a graph would keep an address that a
+// later, larger call frees.  A capture on another stream is left undisturbed
+// (relaxed mode around the allocation).
+void* optional_workspace(g950_module* m, void* stream, size_t bytes) {
+  if (t_scratch) return nullptr;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  void* ws = nullptr;
+  if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone ||
+      workspace(m, stream, bytes, &ws) != G950_OK) {
+    (void)hipGetLastError();
+    ws = nullptr;
+  }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  return ws;
+}
+
+// Few queries per sequence (attn_decode.hip): `a.rows` query rows per
+// (sequence, KV head) pair, at most 32.  Key ranges: four workgroups per CU
+// (two are resident), so that sequences of different lengths even out, but
+// no range below 256 keys.  Measured on MI355X (bf16, 32/8 heads, d 128, 64-
+// key pages; us at a target of 2 / 4 / 8 / 16 workgroups per CU): 64
+// sequences of 2048 keys 93 / 99 / 107 / 112, 64 of 8000..400 226 / 205 /
+// 221 / 220, 32 of 4096..300 70 / 71 / 69 / 77; ranges from 128 keys up cost
+// one sequence of 8192 keys 29.5 us against 21.8 (256) and 19.8 (512), one
+// of 1024 keys runs 11.7 against 13.6 with 512.
+constexpr long long kDecTarget = 4, kDecMinKeys = 256;
+
+int launch_attn_decode(g950_module* m, AttnDecArgs& a, uint32_t dt, long long D, bool paged, void* stream) {
+  const long long pairs = (long long)a.a.Z * a.a.Hkv;
+  const long long cus = m ? m->cus : 256;
+  long long splits = std::min({(kDecTarget * cus + pairs - 1) / pairs, (long long)(a.a.Sk + kDecMinKeys - 1) / kDecMinKeys, 64ll});
+  splits = std::max(splits, 1ll);
+  if (splits > 1 && m) {
+    const long long recs = pairs * a.rows * splits;
+    a.part = (float*)optional_workspace(m, stream, (size_t)recs * (size_t)(D + 2) * 4);
+    a.ml = a.part + recs * D;
+    if (!a.part) splits = 1;
+  }
+  a.chunk = (int)(((a.a.Sk + splits - 1) / splits + 63) / 64 * 64);
+  a.splits = (int)splits;
+  const char* ty = dt == G950_DTYPE_BFLOAT16 ? "bf16" : "f16";
+  char name[64];
+  snprintf(name, sizeof name, "g950_attn_dec_%s_d%lld_r%d%s", ty, D, a.rows <= 16 ? 16 : 32, paged ? "_pg" : "");
+  if (pairs * splits > 0x7FFFFFFF) return fail(G950_USAGE, "flash_varlen: grid too large");
+  if (int rc = launch(m, name, (unsigned)(pairs * splits), 256u, a, stream)) return rc;
+  if (splits == 1) return G950_OK;
+  snprintf(name, sizeof name, "g950_attn_dec_%s_d%lld_merge", ty, D);
+  return launch(m, name, (unsigned)((pairs * a.rows + 3) / 4), 256u, a, stream);
+}
+
 int op_flash_varlen(g950_module* m, const g950_view* views, uint32_t nviews, const g950_scalar* sc,
                     uint32_t nsc, void* stream) {
   if (nviews != 12 || nsc != kVarlenNsc)
@@ -1410,6 +1476,15 @@ int op_flash_varlen(g950_module* m, const g950_view* views, uint32_t nviews, con
                     aligned16(v.addr()) && (o.addr() & 7) == 0 && m8(a.q_ss) && m8(a.q_sh) && m8(a.k_ss) &&
                     m8(a.k_sh) && m8(a.v_ss) && m8(a.v_sh) && a.o_ss % 4 == 0 && a.o_sh % 4 == 0 &&
                     m8(vl.q_bs) && m8(vl.k_bs) && m8(vl.v_bs) && vl.o_bs % 4 == 0 && (!paged || m8(vl.page_stride));
+  // few queries per sequence: all heads of a KV head in one tile.  A lane's
+  // key rows are reached by 32-bit offsets within a tile; a page must hold
+  // whole 16-key tiles.
+  const long long off16 = 1ll << 25;
+  if (mfma && SQ * (H / HK) <= 32 && a.k_ss < off16 && a.v_ss < off16 && (!paged || bs % 16 == 0)) {
+    AttnDecArgs da{};
+    da.a = a; da.v = vl; da.rows = (int)(SQ * (H / HK));
+    return launch_attn_decode(m, da, dt, D, paged, stream);
+  }
   if (mfma) {
     // paging is compiled into the kernel: contiguous rows, pages of whole
     // 64-key tiles, or a page-table read per DMA lane
@@ -1520,7 +1595,9 @@ int dispatch(g950_module* m, uint32_t op, const g950_view* views, uint32_t nview
 int g950_launch(g950_module* m, uint32_t op, const g950_view* views, uint32_t nviews,
                 const g950_scalar* scalars, uint32_t nscalars, void* stream) {
   if (!m) return fail(G950_USAGE, "g950_launch: null module");
-  return dispatch(m, op, views, nviews, scalars, nscalars, stream);
+  const int rc = dispatch(m, op, views, nviews, scalars, nscalars, stream);
+  t_ws_use = {};
+  return rc;
 }
 
 int g950_launch_noalloc(g950_module* m, uint32_t op, const g950_view* views, uint32_t nviews,

@@ -235,7 +235,8 @@ int g950_launch_noalloc(g950_module *module, uint32_t op, const g950_view *views
 
 /* Bytes of device workspace the module holds for launches on `stream` (0 if
  * it holds none): what g950_launch allocated there for split rows, copies of
- * B and int8 sums, grown on demand and freed by g950_close.  The runtime-side
+ * B, int8 sums and the key ranges of few-query attention, grown on demand and
+ * freed by g950_close.  The runtime-side
  * counterpart of the reference's workspace queries
  * (operator_workspace_private/_shared, a100c/runtime/a100rt.h:180-181); it
  * lets a caller see that g950_launch_noalloc left it untouched. */

@@ -1,0 +1,104 @@
+"""GPU parity of the few-query attention kernels (g950_attn_dec_*): calls of
+flash_varlen_fwd_kernel whose query rows of one KV head (seqlen_q x heads per
+KV head) are at most 32, against the CPU oracle at the varlen bars (bf16 1e-2,
+fp16 3e-2 on O and LSE: the probabilities and O round to 16 bits)."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from compiler_amd import operators as ops  # noqa: E402
+from compiler_amd import runtime as rt  # noqa: E402
+from oracle import inputs  # noqa: E402
+from oracle import reference as ref  # noqa: E402
+
+import test_gpu_varlen as tv  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+# key counts at the edges of a tile (16), a round of the four waves (64), a
+# key range (256) and beyond several ranges; 1, 2 and 32 rows per KV head
+CASES = {
+    "one_key": dict(batches=1, max_q=1, max_k=1, h=4, hk=4, d=128),
+    "tile_edges": dict(batches=3, max_q=1, max_k=18, h=8, hk=2, d=128, var_q=False),
+    "round_edges": dict(batches=3, max_q=1, max_k=66, h=8, hk=1, d=64, var_q=False),
+    "ranges": dict(batches=2, max_q=1, max_k=1500, h=32, hk=8, d=128, var_q=False, causal=True, window_right=0),
+    "ranges_d64": dict(batches=2, max_q=2, max_k=2051, h=16, hk=4, d=64, var_q=False, causal=True, window_right=0),
+    "rows32": dict(batches=2, max_q=4, max_k=700, h=8, hk=1, d=128, causal=True, window_right=0),
+    "rows17": dict(batches=1, max_q=17, max_k=513, h=2, hk=2, d=64, causal=True, window_right=0),
+    "group3": dict(batches=2, max_q=5, max_k=300, h=6, hk=2, d=128, causal=True, window_right=0),
+    "local": dict(batches=2, max_q=4, max_k=900, h=4, hk=2, d=128, local=True, window_left=100, window_right=0),
+    "local_empty": dict(batches=2, max_q=4, max_k=300, h=4, hk=2, d=64, local=True, window_left=-40,
+                        window_right=80),
+    "paged16": dict(batches=3, max_q=1, max_k=777, h=8, hk=2, d=128, var_q=False, paged=True, block_size=16,
+                    causal=True, window_right=0),
+    "paged64": dict(batches=2, max_q=4, max_k=4500, h=8, hk=1, d=64, paged=True, block_size=64, causal=True,
+                    window_right=0),
+    "paged48": dict(batches=2, max_q=1, max_k=400, h=4, hk=4, d=128, var_q=False, paged=True, block_size=48),
+    "fewer_keys_than_queries": dict(batches=1, max_q=8, max_k=5, h=2, hk=1, d=64, causal=True, window_right=0),
+    "seqused": dict(batches=3, max_q=1, max_k=520, h=8, hk=8, d=128, var_q=False, seqused_trim=37),
+}
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_decode_attention(case, dt):
+    a, meta = inputs.varlen_case(**CASES[case])
+    tv.check(a, meta, dt, f"g950_attn_dec_{'bf16' if dt == 'bfloat16' else 'f16'}_d{CASES[case]['d']}_")
+
+
+def test_decode_attention_sequences_without_keys_or_queries():
+    """A sequence with no keys (O = 0, LSE = +inf), one with no queries, and
+    rows past cu_seqlens_q[-1] (untouched), with and without key ranges."""
+    for max_k in (200, 3000):
+        a, meta = inputs.varlen_case(batches=3, max_q=6, max_k=max_k, h=4, hk=2, d=128, seqused_trim=5)
+        used, cu = a["seqused_k_ptr"].copy(), a["cu_seqlens_q_ptr"].copy()
+        used[0] = 0
+        cu[2] = cu[1]
+        cu[3] = cu[2] + 2
+        a = dict(a, seqused_k_ptr=used, cu_seqlens_q_ptr=cu)
+        tv.check(a, meta, "bfloat16", "g950_attn_dec_")
+
+
+def test_decode_attention_scores_climb():
+    """Scores that grow with the key index by about 16 log2 units per 64 keys:
+    every tile moves the reference maximum, and the key ranges' maxima lie far
+    apart when they are joined."""
+    a, meta = inputs.varlen_case(batches=2, max_q=1, max_k=2000, h=8, hk=2, d=128, var_q=False, var_k=False)
+    q = a["q_ptr"].reshape(-1, 128)
+    q[:, 0] = 4.0
+    k = a["k_ptr"].reshape(2, 2000, 2, 128)
+    k[..., 0] = np.arange(2000)[None, :, None] / 64 * 16 / 1.4427 / (meta["scale_softmax"] * 4.0)
+    tv.check(dict(a, q_ptr=q.reshape(-1), k_ptr=k.reshape(-1)), meta, "bfloat16", "g950_attn_dec_")
+
+
+def test_decode_attention_without_workspace():
+    """No-alloc calls and captured graphs keep to one key range per pair (no
+    workspace) and give the same results within the bar; a graph replayed
+    between other work gives its own result again."""
+    a, meta = inputs.varlen_case(batches=2, max_q=1, max_k=3000, h=8, hk=2, d=128, var_q=False, var_k=False)
+    t = {n: torch.from_numpy(np.ascontiguousarray(a[n]).view(np.int64) if a[n].dtype == np.uint64
+                             else np.ascontiguousarray(a[n])).to("cuda") for n in ops._VARLEN_VIEWS}
+    for n in ("q_ptr", "k_ptr", "v_ptr", "o_ptr"):
+        t[n] = t[n].to(torch.bfloat16)
+    scal = {n: {**a, **meta}[n] for n in ops._VARLEN_SCALARS}
+    ops.flash_varlen_fwd_kernel(**t, **scal, sync=True)
+    assert rt.module().last_kernel.endswith("_merge")
+    split = t["o_ptr"].clone()
+    with rt.no_alloc():
+        ops.flash_varlen_fwd_kernel(**t, **scal, sync=True)
+    assert rt.module().last_kernel == "g950_attn_dec_bf16_d128_r16"
+    one = t["o_ptr"].clone()
+    ok, err = ref.isclose_verdict(one.float().cpu().numpy(), split.float().cpu().numpy(), 1e-2, 1e-2)
+    assert ok, err
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        ops.flash_varlen_fwd_kernel(**t, **scal)
+    for _ in range(3):
+        t["o_ptr"].zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(t["o_ptr"], one)
+        ops.flash_varlen_fwd_kernel(**t, **scal, sync=True)
+        assert torch.equal(t["o_ptr"], split)
