@@ -24,6 +24,9 @@ struct RowArgs {
   int splits;         // split rows: chunks per row
 };
 
+// workgroup tile of the whole-slab MFMA GEMM kernels (M x N outputs)
+enum GemmTile : int { GEMM_TILE_256x256 = 0, GEMM_TILE_128x128 = 1, GEMM_TILE_64x128 = 2, GEMM_TILE_64x64 = 3 };
+
 struct GemmArgs {
   const void* a;      // fast: [M,K] K-contiguous; general: element strides below
   const void* b;      // fast: Bt[N,K] K-contiguous
@@ -48,6 +51,7 @@ struct GemmArgs {
   // where rsum / csum are the int32 sums over k of A's rows / B's columns
   const int* rsum;
   const int* csum;
+  int tile;           // enum GemmTile; tiles_m / tiles_n count tiles of it
 };
 
 // Sums over k of int8 / uint8 rows (A[m, :] and Bt[n, :], K-contiguous):

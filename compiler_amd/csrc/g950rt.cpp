@@ -610,12 +610,46 @@ int op_layernorm_row(g950_module* m, const g950_view* views, uint32_t nviews, co
 }
 
 // --------------------------------------------------------------------- GEMM
-int gemm_tiles(GemmArgs& g) {
-  const long long tm = (g.M + 255) / 256, tn = (g.N + 255) / 256;
+int gemm_tiles(GemmArgs& g, int bm = 256, int bn = 256) {
+  const long long tm = (g.M + (long long)bm - 1) / bm, tn = (g.N + (long long)bn - 1) / bn;
   if (tm * tn > 0x7FFFFFFF) return -1;
   g.tiles_m = (int)tm;
   g.tiles_n = (int)tn;
   return (int)(tm * tn);
+}
+
+// Workgroup tile of a whole-slab MFMA GEMM (GemmArgs::tile) and its tile
+// count: the least of rounds x (slabs x slab time + fixed time), a round
+// being one workgroup per CU.  Smaller tiles cost more per output (a CU's
+// load path moves 70 bytes per ns whatever the tile, and a 64 x 64 tile needs
+// four times the bytes of a 256 x 256 one per output) but fill the chip where
+// the larger would leave CUs idle.  Slab times in us, measured on MI355X with
+// operands from HBM: bf16 M x 4096 x 4096 (64 slabs, each CU at most one
+// tile) 256x256 92-95 us, 128x128 40-43, 64x128 31, 64x64 22; 4096 x 11008 x
+// 512 to 8192 x 8192 x 1536 follow within 10%.  Both sides of a line, bf16:
+// 512x4096x4096 68 (256x256) / 35 (128x128) / 26 (64x128) / 31 (64x64);
+// 2048x4096x4096 93 / 81 / 115 / 149; 2304x4096x4096 94 / 104 / 118 / 138;
+// int8 512x8192x8192 99 / 47 / 64 / 81.  fp32 is bound by its MFMAs, so its
+// slab times are nearly the tiles' areas: 512x4096x4096 896 / 252 / 140 / 148.
+int gemm_pick_tile(const g950_module* m, GemmArgs& g, int slabs, bool f32) {
+  const long long cus = m ? m->cus : 256;
+  static const struct { int tile, bm, bn; double slab, f32_slab, fixed; } kTiles[] = {
+      {GEMM_TILE_256x256, 256, 256, 1.42, 7.0, 4.0},
+      {GEMM_TILE_128x128, 128, 128, 0.59, 1.95, 3.0},
+      {GEMM_TILE_64x128, 64, 128, 0.44, 1.06, 3.0},
+      {GEMM_TILE_64x64, 64, 64, 0.31, 0.58, 2.5}};
+  const auto* pick = &kTiles[0];
+  double best = HUGE_VAL;
+  for (const auto& t : kTiles) {
+    const long long tiles = ((g.M + t.bm - 1ll) / t.bm) * ((g.N + t.bn - 1ll) / t.bn);
+    const double us = (double)((tiles + cus - 1) / cus) * (slabs * (f32 ? t.f32_slab : t.slab) + t.fixed);
+    if (us < best) {
+      best = us;
+      pick = &t;
+    }
+  }
+  g.tile = pick->tile;
+  return gemm_tiles(g, pick->bm, pick->bn);
 }
 
 // A[M,K] and B[K,N] both K-contiguous with 16-byte rows (K a whole number of
@@ -696,9 +730,9 @@ int op_matmul(g950_module* m, const g950_view* views, uint32_t nviews, const g95
   if (same16 && gemm_fast_ok(a, b, (int)K, esz) && out16) {
     g.a_s0 = a.stride[0];
     g.b_s0 = b.stride[1];  // Bt row (n) stride
-    const int tiles = gemm_tiles(g);
-    if (tiles < 0) return fail(G950_USAGE, "matmul: too many tiles");
     const char* name = mfma_kernel();
+    const int tiles = strstr(name, "_kt") ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K * esz / 128), esz == 4);
+    if (tiles < 0) return fail(G950_USAGE, "matmul: too many tiles");
     return launch(m, name, (unsigned)tiles, (unsigned)kernel_threads(m, name, 512), g, stream);
   }
   const bool rowb_ok = same16 && out16 && gemm_rowb_ok(a, b, (int)K, (int)N, esz);
@@ -741,9 +775,9 @@ int op_matmul(g950_module* m, const g950_view* views, uint32_t nviews, const g95
     g.b = bt;
     g.a_s0 = a.stride[0];
     g.b_s0 = K;
-    const int tiles = gemm_tiles(g);
-    if (tiles < 0) return fail(G950_USAGE, "matmul: too many tiles");
     const char* name = mfma_kernel();
+    const int tiles = strstr(name, "_kt") ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K * esz / 128), esz == 4);
+    if (tiles < 0) return fail(G950_USAGE, "matmul: too many tiles");
     return launch(m, name, (unsigned)tiles, (unsigned)kernel_threads(m, name, 512), g, stream);
   }
   g.a_s0 = a.stride[0]; g.a_s1 = a.stride[1];
@@ -806,7 +840,7 @@ int op_matmul_i8(g950_module* m, const g950_view* views, uint32_t nviews, const 
   g.b_s0 = b.stride[1];
   const bool ktail = gemm_ktail((int)K, 1) || !gemm_off32(g, 1);
   if (gemm_fast_ok(a, b, (int)K, 1) && out_ok && (umask == 0 || !ktail)) {
-    const int tiles = gemm_tiles(g);
+    const int tiles = ktail || umask ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K / 128), false);
     if (tiles < 0) return fail(G950_USAGE, "matmul_i8: too many tiles");
     static const char* const names[4] = {"g950_gemm_i8_256x256", "g950_gemm_u8s8_256x256",
                                          "g950_gemm_s8u8_256x256", "g950_gemm_u8u8_256x256"};

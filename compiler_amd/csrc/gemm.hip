@@ -16,7 +16,9 @@
 //     64 x 128: 4 x 8 fragments of v_mfma_f32_16x16x32_{bf16,f16} /
 //     v_mfma_i32_16x16x64_i8 for whole-slab 16-bit / int8 shapes with
 //     M, N >= 256 (gemm_mfma16_body), else 2 x 4 fragments of the 32x32
-//     forms; the B tile feeds the MFMA A port so each lane ends with four
+//     forms; shapes whose 256 x 256 tiles leave CUs idle run 128x128, 64x128
+//     or 64x64 tiles in the same kernels (gemm_tile_body; the host picks by
+//     measured tile times); the B tile feeds the MFMA A port so each lane ends with four
 //     consecutive output columns of one output row
 //   * K in slabs of 128 bytes per row (64 bf16 / 128 int8); two LDS stages
 //     of 64 KiB (A rows then B rows, 128-byte rows), filled by direct
@@ -687,6 +689,179 @@ __device__ __forceinline__ void gemm_mfma16_body(const GemmArgs& p, char* lds) {
                                               n_own);
 }
 
+// Smaller workgroup tiles of the whole-slab kernels (GemmArgs::tile), for
+// shapes whose 256 x 256 tiles would leave most CUs idle: TM x TN outputs,
+// 8 waves as 2 x 2 wave tiles x 2 halves of each K slab (a wave multiplies
+// one 64-byte k-step of every slab, so its fragments are read once for a
+// (TM/2) x (TN/2) tile: half the LDS reads per MFMA of eight smaller wave
+// tiles).  The slabs run through a ring of NST stages filled by direct DMA,
+// every wave issuing its share: NST - 1 slabs are in flight, since with few
+// MFMAs per slab the latency of a load, not its issue, is what a two-stage
+// ring would show.  What bounds it is the CU's load path (16, 24 or 32 KB per
+// slab at about 70 bytes per ns): bf16 512 x 4096 x 4096 68 -> 26 us (64 x 128
+// tiles, one per CU), 256 x 4096 x 4096 68 -> 16, 1000 x 4096 x 4096 68 -> 39,
+// int8 512 x 8192 x 8192 70 -> 40, fp32 512 x 2048 x 2048 452 -> 40 (operands
+// in the MALL).  fp32 sums in two chains: error against 64 bits at 512 x 2048
+// x 4096 1.14e-6 -> 8.1e-7.  Iteration kt multiplies slab kt from registers while slab
+// kt + 1's fragments are read; one barrier per slab, after this wave's loads
+// of slab kt + 1 have landed.  After it nobody reads slab kt's stage again,
+// so slab kt + NST goes there.  The two k-halves of a wave tile are added
+// through LDS, each wave finishing half of the rows.
+template <int MODE, int TM, int TN, int UMASK, int NST>
+__device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
+  constexpr int STAGE = (TM + TN) * SLAB;
+  constexpr int DPW = (TM + TN) / 64;              // DMA instructions (8 rows x 128 bytes) per wave per slab
+  constexpr int FM = TM / 32, FN = TN / 32;        // 16x16 fragments of a wave tile
+  static_assert(NST * STAGE <= 4 * BM * SLAB && NST >= 3, "the ring fits the kernel's LDS");
+  static_assert(FM % 2 == 0 && 8 * (FM / 2) * FN * 1024 <= NST * STAGE, "the k-halves' exchange fits the ring");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+  int tm, tn;
+  tile_of(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+  const int m0 = tm * TM, n0 = tn * TN;
+  constexpr int ES = (MODE == GEMM_I8) ? 1 : (MODE == GEMM_F32) ? 4 : 2;
+  const long long lda = p.a_s0 * ES, ldb = p.b_s0 * ES;
+  const char* abase = (const char*)p.a + (long long)m0 * lda;
+  const char* bbase = (const char*)p.b + (long long)n0 * ldb;
+  const int kslabs = p.K * ES / SLAB;
+  // group t of this wave: 8 rows of A or B (rows past the edge repeat the
+  // last one; their outputs are not stored), the 16-byte chunks XOR-swizzled
+  // by (row >> 1) & 7 as in the 256 x 256 kernels
+  uint32_t doff[DPW];
+  const uint32_t lds32 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)lds;
+#pragma unroll
+  for (int t = 0; t < DPW; ++t) {
+    const int grp = wave * DPW + t;
+    const bool is_a = grp < TM / 8;
+    const int row = (is_a ? grp : grp - TM / 8) * 8 + (lane >> 3);
+    const int src = min(row, (is_a ? p.M - m0 : p.N - n0) - 1);
+    doff[t] = (uint32_t)((long long)src * (is_a ? lda : ldb) + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
+  }
+  auto issue = [&](int slab) {
+    const uint32_t dst = lds32 + (uint32_t)(slab % NST) * STAGE;
+#pragma unroll
+    for (int t = 0; t < DPW; ++t) {
+      const int grp = wave * DPW + t;
+      dma16_asm((grp < TM / 8 ? abase : bbase) + (long long)slab * SLAB, doff[t], dst + grp * 1024);
+    }
+  };
+  const int l16 = lane & 15, g4 = lane >> 4;
+  const int sw = l16 * SLAB + (((kg * 4 + g4) ^ ((l16 >> 1) & 7)) << 4);
+  const int aoff = wm * (TM / 2) * SLAB + sw, boff = (TM + wn * (TN / 2)) * SLAB + sw;
+  u32x4 af[2][FM], bf[2][FN];
+  auto frags = [&](int slab, auto bc) {
+    constexpr int B = decltype(bc)::value;
+    const char* st = lds + (slab % NST) * STAGE;
+#pragma unroll
+    for (int i = 0; i < FM; ++i) af[B][i] = *(const u32x4*)(st + aoff + i * 16 * SLAB);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) bf[B][j] = *(const u32x4*)(st + boff + j * 16 * SLAB);
+  };
+  f32x4 acf[FM][FN];
+  i32x4 aci[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      if constexpr (MODE == GEMM_I8) aci[i][j] = (i32x4){};
+      else acf[i][j] = (f32x4){};
+    }
+  auto mmas = [&](auto bc) {
+    constexpr int B = decltype(bc)::value;
+    if constexpr (UMASK & 1) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) af[B][i] ^= 0x80808080u;
+    }
+    if constexpr (UMASK & 2) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) bf[B][j] ^= 0x80808080u;
+    }
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        if constexpr (MODE == GEMM_BF16)
+          acf[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, bf[B][j]),
+                                                              __builtin_bit_cast(bf16x8, af[B][i]), acf[i][j], 0, 0, 0);
+        else if constexpr (MODE == GEMM_F16)
+          acf[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, bf[B][j]),
+                                                             __builtin_bit_cast(f16x8, af[B][i]), acf[i][j], 0, 0, 0);
+        else if constexpr (MODE == GEMM_I8)
+          aci[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, bf[B][j]),
+                                                            __builtin_bit_cast(i32x4, af[B][i]), aci[i][j], 0, 0, 0);
+        else {  // a chunk's four k in four MFMAs, the same k order on both sides
+          const f32x4 bv = __builtin_bit_cast(f32x4, bf[B][j]), av = __builtin_bit_cast(f32x4, af[B][i]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acf[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[e], av[e], acf[i][j], 0, 0, 0);
+        }
+      }
+  };
+  using B0 = std::integral_constant<int, 0>;
+  using B1 = std::integral_constant<int, 1>;
+  // this wave's loads of slab s have landed, at most the NST - 2 later ones
+  // still in flight (all of them waited for where fewer were issued)
+  auto landed = [&](int s) {
+    if (s + NST - 2 < kslabs) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * DPW) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+  // first NST - 1 slabs; slab kt + NST - 1 is issued before iteration kt's
+  // wait, so that wait leaves NST - 2 slabs in flight
+  for (int s = 0; s < NST - 1 && s < kslabs; ++s) issue(s);
+  landed(0);
+  asm volatile("s_barrier" ::: "memory");
+  frags(0, B0{});
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if (NST - 1 < kslabs) issue(NST - 1);
+  auto iter = [&](int kt, auto bc) {
+    constexpr int B = decltype(bc)::value;
+    if (kt + 1 < kslabs) {
+      landed(kt + 1);
+      asm volatile("s_barrier" ::: "memory");
+      if (kt + NST < kslabs) issue(kt + NST);
+      frags(kt + 1, std::integral_constant<int, B ^ 1>{});
+    }
+    mmas(bc);
+    // the fragments read above are in registers before the next barrier
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+  int kt = 0;
+  for (; kt + 1 < kslabs; kt += 2) {
+    iter(kt, B0{});
+    iter(kt + 1, B1{});
+  }
+  if (kt < kslabs) iter(kt, B0{});
+
+  // ---- add the two k-halves: each wave keeps half of its rows' fragments
+  // and hands the other half to its partner (wave ^ 4)
+  constexpr int HM = FM / 2;
+  __syncthreads();
+  char* mine = lds + wave * HM * FN * 1024 + lane * 16;
+#pragma unroll
+  for (int i = 0; i < HM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      u32x4 v;
+      if constexpr (MODE == GEMM_I8) v = __builtin_bit_cast(u32x4, kg ? aci[i][j] : aci[i + HM][j]);
+      else v = __builtin_bit_cast(u32x4, kg ? acf[i][j] : acf[i + HM][j]);
+      *(u32x4*)(mine + (i * FN + j) * 1024) = v;
+    }
+  __syncthreads();
+  const char* theirs = lds + (wave ^ 4) * HM * FN * 1024 + lane * 16;
+  f32x4 hf[HM][FN];
+  i32x4 hi[HM][FN];
+#pragma unroll
+  for (int i = 0; i < HM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const u32x4 v = *(const u32x4*)(theirs + (i * FN + j) * 1024);
+      // k-half 0 first on both waves
+      if constexpr (MODE == GEMM_I8) hi[i][j] = (kg ? aci[i + HM][j] : aci[i][j]) + __builtin_bit_cast(i32x4, v);
+      else hf[i][j] = (kg ? acf[i + HM][j] : acf[i][j]) + __builtin_bit_cast(f32x4, v);
+    }
+  gemm_epilogue<MODE, HM, FN, UMASK, 16>(p, hf, hi, m0 + wm * (TM / 2) + kg * HM * 16, n0 + wn * (TN / 2), lane);
+}
+
 // WM x WN waves; wave tile (BM/WM) x (BN/WN) = FM x FN fragments of 32x32.
 // UMASK (int8): bit 0 A unsigned, bit 1 B unsigned.  An unsigned operand's
 // bytes are flipped (XOR 0x80: u - 128, a signed int8) as its fragments enter
@@ -702,6 +877,22 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmArgs& p) {
   constexpr int H = GROUPS / 2;
   static_assert(GROUPS * 8 * DW == BM + BN && GROUPS % 2 == 0, "DMA split over waves and halves");
   __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE];
+  if constexpr (!KTAIL && UMASK == 0) {
+    // smaller tiles where 256 x 256 ones would leave CUs idle (uniform per
+    // launch; the host's gemm_pick_tile)
+    if (p.tile == GEMM_TILE_128x128) {
+      gemm_tile_body<MODE, 128, 128, UMASK, 4>(p, lds);
+      return;
+    }
+    if (p.tile == GEMM_TILE_64x128) {
+      gemm_tile_body<MODE, 64, 128, UMASK, 5>(p, lds);
+      return;
+    }
+    if (p.tile == GEMM_TILE_64x64) {
+      gemm_tile_body<MODE, 64, 64, UMASK, 8>(p, lds);
+      return;
+    }
+  }
   if constexpr (G950_GEMM16 && MODE != GEMM_F32 && !KTAIL) {
     // whole-slab 16-bit / int8 GEMMs of at least one tile each way take the
     // 16x16-fragment form (uniform per launch)
