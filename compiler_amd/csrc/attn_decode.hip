@@ -185,13 +185,14 @@ __device__ __forceinline__ void attn_decode_body(const AttnDecArgs& g) {
       const char* st = ring + (i % ST) * 2 * KT;
       const int kv0 = lo + DEC_TK * (wave + DEC_WAVES * i);
       f32x4 s[RT];
+      i32x4 unused;
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) s[rt] = (f32x4){};
 #pragma unroll
       for (int ks = 0; ks < DS; ++ks) {
         const u32x4 kf = *(const u32x4*)(st + koff[ks]);
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) s[rt] = mfma16x16x32<F16>(kf, qf[rt][ks], s[rt]);
+        for (int rt = 0; rt < RT; ++rt) mfma16_step<F16 ? GEMM_F16 : GEMM_BF16>(kf, qf[rt][ks], s[rt], unused);
       }
       // keys kv0 + 4 g4 .. + 3 of query row l16
       const bool mask = kv0 + DEC_TK > Sk || (has_hi && kv0 + DEC_TK - 1 > q0 + hi_off) ||

@@ -652,6 +652,44 @@ int gemm_pick_tile(const g950_module* m, GemmArgs& g, int slabs, bool f32) {
   return gemm_tiles(g, pick->bm, pick->bn);
 }
 
+// Few rows of A (M <= 64, gemm.hip gemm_few_rows): whether the kernels take
+// the call -- a lane reaches an operand's rows by 32-bit byte offsets -- and
+// the column groups T per workgroup (GemmArgs::tile) with that form's waves.
+// Each CU gets at most one workgroup (their rings fill its LDS), so T is the
+// smallest whose grid is one round: every workgroup reads all of A, so more
+// columns cost each CU more but a second round costs all of the first again.
+// Measured on MI355X with operands from HBM (us for T = 1 / 2 / 3 / 4): bf16
+// 16x4096x4096 10.0 / 12.7 / 13.3 / 15.4, 16x11008x4096 24.4 / 27.3 / 18.7 /
+// 19.4; with int8 weights 16x4096x4096 9.1 / 8.8 / 9.9 / 11.7, 16x6144x4096
+// 14.0 / 9.4 / 10.6, 16x8192x8192 23.9 / 20.4 / 18.8 / 20.9 (T = 2 at exactly
+// one workgroup per CU loses to T = 3 on two thirds of them, so it ends at
+// three quarters).
+struct FewRowsForm { int t, waves, quarters; };  // taken up to quarters / 4 workgroups per CU
+constexpr FewRowsForm kFewRows[2][3][4] = {
+    // 16-bit, int8 and fp32 operands: up to 16, 32, 64 rows
+    {{{1, 8, 4}, {3, 8, 4}, {4, 8, 4}, {}}, {{1, 8, 4}, {2, 8, 4}, {4, 4, 4}, {}}, {{1, 8, 4}, {2, 4, 4}, {4, 4, 4}, {}}},
+    // int8 weights
+    {{{1, 8, 4}, {2, 8, 3}, {3, 8, 4}, {4, 4, 4}}, {{1, 4, 4}, {2, 4, 4}, {3, 4, 4}, {}}, {{1, 4, 4}, {2, 4, 4}, {}, {}}}};
+
+bool few_rows_ok(const GemmArgs& g, int a_esz, int b_esz) {
+  auto reach = [](long long rows, long long s0, int esz) { return (__int128)(rows - 1) * s0 * esz + 256 <= (__int128)0xFFFFFFFFll; };
+  return g.M <= 64 && reach(64, g.a_s0, a_esz) && reach(64, g.b_s0, b_esz);
+}
+
+int launch_few_rows(g950_module* m, const char* name, GemmArgs& g, bool w8, void* stream) {
+  const long long cus = m ? m->cus : 256;
+  const FewRowsForm* form = kFewRows[w8][g.M <= 16 ? 0 : g.M <= 32 ? 1 : 2];
+  long long blocks = 0;
+  for (int i = 0; i < 4 && form[i].t; ++i) {
+    blocks = (g.N + 16ll * form[i].t - 1) / (16 * form[i].t);
+    g.tile = i;
+    if (4 * blocks <= form[i].quarters * cus) break;
+  }
+  form += g.tile;
+  g.tile = form->t;
+  return launch(m, name, (unsigned)blocks, (unsigned)(64 * form->waves), g, stream);
+}
+
 // A[M,K] and B[K,N] both K-contiguous with 16-byte rows (K a whole number of
 // 16-byte chunks): the MFMA kernels apply -- the plain ones when K is a whole
 // number of 128-byte slabs, else the _kt ones (gemm_ktail).
@@ -720,20 +758,25 @@ int op_matmul(g950_module* m, const g950_view* views, uint32_t nviews, const g95
   const bool same16 = a.v->dtype == b.v->dtype && is_float(a.v->dtype);
   const int esz = a.isz;
   const bool out16 = y.stride[1] == 1 && aligned16(y.addr());
-  char mfma_name[48];
-  // (call once g.a_s0 / g.b_s0 hold the operand row strides)
-  auto mfma_kernel = [&]() -> const char* {
-    snprintf(mfma_name, sizeof mfma_name, "g950_gemm_%s_256x256%s", rr_dtype(a.v->dtype),
-             gemm_ktail((int)K, esz) || !gemm_off32(g, esz) ? "_kt" : "");
-    return mfma_name;
+  // K-contiguous operands, once g.a_s0 / g.b_s0 hold their row strides: few
+  // rows of A over a K that gives each of the eight waves a 128-byte unit,
+  // else tiles
+  auto mfma = [&]() -> int {
+    char name[48];
+    if (K * esz >= 1024 && few_rows_ok(g, esz, esz)) {
+      snprintf(name, sizeof name, "g950_gemm_skinny%d_%s", M <= 16 ? 16 : M <= 32 ? 32 : 64, rr_dtype(a.v->dtype));
+      return launch_few_rows(m, name, g, false, stream);
+    }
+    const bool kt = gemm_ktail((int)K, esz) || !gemm_off32(g, esz);
+    const int tiles = kt ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K * esz / 128), esz == 4);
+    if (tiles < 0) return fail(G950_USAGE, "matmul: too many tiles");
+    snprintf(name, sizeof name, "g950_gemm_%s_256x256%s", rr_dtype(a.v->dtype), kt ? "_kt" : "");
+    return launch(m, name, (unsigned)tiles, (unsigned)kernel_threads(m, name, 512), g, stream);
   };
   if (same16 && gemm_fast_ok(a, b, (int)K, esz) && out16) {
     g.a_s0 = a.stride[0];
     g.b_s0 = b.stride[1];  // Bt row (n) stride
-    const char* name = mfma_kernel();
-    const int tiles = strstr(name, "_kt") ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K * esz / 128), esz == 4);
-    if (tiles < 0) return fail(G950_USAGE, "matmul: too many tiles");
-    return launch(m, name, (unsigned)tiles, (unsigned)kernel_threads(m, name, 512), g, stream);
+    return mfma();
   }
   const bool rowb_ok = same16 && out16 && gemm_rowb_ok(a, b, (int)K, (int)N, esz);
   // Row-major B read directly by the 16x16 MFMA kernel (transposing LDS
@@ -775,10 +818,7 @@ int op_matmul(g950_module* m, const g950_view* views, uint32_t nviews, const g95
     g.b = bt;
     g.a_s0 = a.stride[0];
     g.b_s0 = K;
-    const char* name = mfma_kernel();
-    const int tiles = strstr(name, "_kt") ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K * esz / 128), esz == 4);
-    if (tiles < 0) return fail(G950_USAGE, "matmul: too many tiles");
-    return launch(m, name, (unsigned)tiles, (unsigned)kernel_threads(m, name, 512), g, stream);
+    return mfma();
   }
   g.a_s0 = a.stride[0]; g.a_s1 = a.stride[1];
   g.b_s0 = b.stride[0]; g.b_s1 = b.stride[1];
@@ -839,6 +879,10 @@ int op_matmul_i8(g950_module* m, const g950_view* views, uint32_t nviews, const 
   g.a_s0 = a.stride[0];
   g.b_s0 = b.stride[1];
   const bool ktail = gemm_ktail((int)K, 1) || !gemm_off32(g, 1);
+  if (gemm_fast_ok(a, b, (int)K, 1) && out_ok && umask == 0 && K >= 1024 && few_rows_ok(g, 1, 1)) {
+    const char* name = M <= 16 ? "g950_gemm_skinny16_i8" : M <= 32 ? "g950_gemm_skinny32_i8" : "g950_gemm_skinny64_i8";
+    return launch_few_rows(m, name, g, false, stream);
+  }
   if (gemm_fast_ok(a, b, (int)K, 1) && out_ok && (umask == 0 || !ktail)) {
     const int tiles = ktail || umask ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K / 128), false);
     if (tiles < 0) return fail(G950_USAGE, "matmul_i8: too many tiles");
@@ -1029,24 +1073,23 @@ int op_dequant_matmul(g950_module* m, const g950_view* views, uint32_t nviews, c
     transposed = true;  // the workspace now holds the copy: no second copy below
   }
   if (fast && M <= 64) {
-    // decode shapes: the few-row kernels stream B, 32 columns and all of K
-    // per workgroup (8 waves, one K range each, summed in LDS), for up to 16,
-    // 32 or 64 rows of A.  With at most 16 rows, 16 columns per workgroup
-    // (twice the workgroups, each reading all of A) where the 32-column grid
-    // leaves CUs idle or exceeds them by more than a quarter, and for one row
-    // of A.  Measured on MI355X (rotating inputs): 16x4096x4096 12.3 -> 9.1 us,
-    // 16x4096x11008 27.1 -> 19.8, 16x11008x4096 22.2 -> 21.1, 1x8192x8192
-    // 20.9 -> 15.1; 16x8192x8192 ties and 16x8192x8000 loses (21.7 -> 24.8).
+    // decode shapes: the few-row kernels stream B.  The 16-row kernel has two
+    // names, by the class of its 32-column grid: short of the CUs or more than
+    // a quarter past them, or one row of A (_c16), else the plain one.
     g.a_s0 = a.stride[0];
     g.b_s0 = bts;
-    const long long blocks32 = (N + 31) / 32;
-    const bool c16 = M <= 16 && (M == 1 || blocks32 < cus || 4 * blocks32 > 5 * cus);
-    const long long blocks = c16 ? (N + 15) / 16 : blocks32;
-    if (blocks > 0x7FFFFFFF) return fail(G950_USAGE, "dequant_matmul: too many tiles");
-    char name[48];
-    snprintf(name, sizeof name, "g950_gemm_w8a16_skinny%s_%s", c16 ? "_c16" : M <= 16 ? "" : M <= 32 ? "32" : "64",
-             bf16 ? "bf16" : "f16");
-    return launch(m, name, (unsigned)blocks, 512u, g, stream);
+    g.bscale = nullptr;
+    g.cscale = s.v->data; g.cscale_dtype = (int)s.v->dtype;
+    if (few_rows_ok(g, 2, 1)) {
+      const long long blocks32 = (N + 31) / 32;
+      const bool c16 = M <= 16 && (M == 1 || blocks32 < cus || 4 * blocks32 > 5 * cus);
+      char name[48];
+      snprintf(name, sizeof name, "g950_gemm_w8a16_skinny%s_%s", c16 ? "_c16" : M <= 16 ? "" : M <= 32 ? "32" : "64",
+               bf16 ? "bf16" : "f16");
+      return launch_few_rows(m, name, g, true, stream);
+    }
+    g.cscale = nullptr;
+    g.bscale = s.v->data;
   }
   // Many output tiles: widen B once into an exact bf16 / f16 copy in the
   // workspace and run the 256x256 GEMM with the column scale in its epilogue.

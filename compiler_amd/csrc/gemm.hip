@@ -303,6 +303,26 @@ __device__ __forceinline__ void mfma_step(const u32x4& bfrag, const u32x4& afrag
   }
 }
 
+// The same for 16x16 fragments: lane (g4, l16) holds 16-byte chunk g4 of row
+// l16 of both operands; fp32 takes the chunk's four k in four MFMAs.
+template <int MODE>
+__device__ __forceinline__ void mfma16_step(const u32x4& bfrag, const u32x4& afrag, f32x4& accf, i32x4& acci) {
+  if constexpr (MODE == GEMM_F32) {
+    const f32x4 bv = __builtin_bit_cast(f32x4, bfrag), av = __builtin_bit_cast(f32x4, afrag);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) accf = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[e], av[e], accf, 0, 0, 0);
+  } else if constexpr (MODE == GEMM_BF16) {
+    accf = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, bfrag),
+                                                   __builtin_bit_cast(bf16x8, afrag), accf, 0, 0, 0);
+  } else if constexpr (MODE == GEMM_F16) {
+    accf = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, bfrag), __builtin_bit_cast(f16x8, afrag),
+                                                  accf, 0, 0, 0);
+  } else {
+    acci = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, bfrag), __builtin_bit_cast(i32x4, afrag),
+                                                 acci, 0, 0, 0);
+  }
+}
+
 // Epilogue of the 16x16 form for a 16-bit output whose tile owns all of its
 // window's columns: the wave's 64 x 128 output tile passes through its own
 // 16 KiB of LDS and leaves as whole 256-byte row pieces, 16 bytes per lane,
@@ -781,20 +801,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
-        if constexpr (MODE == GEMM_BF16)
-          acf[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, bf[B][j]),
-                                                              __builtin_bit_cast(bf16x8, af[B][i]), acf[i][j], 0, 0, 0);
-        else if constexpr (MODE == GEMM_F16)
-          acf[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, bf[B][j]),
-                                                             __builtin_bit_cast(f16x8, af[B][i]), acf[i][j], 0, 0, 0);
-        else if constexpr (MODE == GEMM_I8)
-          aci[i][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, bf[B][j]),
-                                                            __builtin_bit_cast(i32x4, af[B][i]), aci[i][j], 0, 0, 0);
-        else {  // a chunk's four k in four MFMAs, the same k order on both sides
-          const f32x4 bv = __builtin_bit_cast(f32x4, bf[B][j]), av = __builtin_bit_cast(f32x4, af[B][i]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) acf[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bv[e], av[e], acf[i][j], 0, 0, 0);
-        }
+        mfma16_step<MODE>(bf[B][j], af[B][i], acf[i][j], aci[i][j]);
       }
   };
   using B0 = std::integral_constant<int, 0>;
@@ -1354,36 +1361,6 @@ __device__ __forceinline__ void gemm_w8a16_body(const GemmArgs& p) {
   gemm_epilogue<F16 ? GEMM_F16 : GEMM_BF16, 2, 2>(p, acc, unused, wm0, wn0, lane);
 }
 
-// -------------------------------------- W8A16 for few rows of A (decode)
-// M <= 64: the 128-row tile would multiply mostly padding and stage 128 A
-// rows per K tile, so a decode-shaped product streams B instead.  A
-// workgroup of 8 waves owns 32 columns (two 16-column tiles) and the whole
-// K: wave w sums K range w of 8, and the waves' partial tiles are added in
-// wave order through LDS (no workspace, no second launch, no workgroup
-// waits on another, the same result every run).  A holds R groups of 16 rows
-// (R = 1, 2, 4: M <= 16, 32, 64); each widened B operand feeds all R groups.
-// Each wave multiplies with v_mfma_f32_16x16x32 (the A rows on the A port,
-// B columns widened from int8 on the B port).  Per 64-element K step, lane
-// (g = lane/16, i = lane%16) loads 16 contiguous int8 of column n0 + 16t + i
-// at k + 16g (64-byte runs per column) and the 32 bytes of A row 16r + i at
-// the same k: its first 8 k feed one MFMA, the next 8 a second one (the two
-// MFMAs' k sets interleave, which leaves each dot product unchanged).
-// SKINNY_STEPS / R steps are in flight per wave, each reloaded with the next
-// batch's step once its MFMAs have issued.
-constexpr int SKINNY_STEPS = 8;   // 64-element K steps loaded together (R = 1)
-constexpr int SKINNY_WAVES = 8;   // K ranges (waves) per workgroup
-constexpr int SKINNY_TILES = 2;   // 16-column tiles per workgroup
-
-template <bool F16>
-__device__ __forceinline__ f32x4 mfma16x16x32(const u32x4& a, const u32x4& b, const f32x4& c) {
-  if constexpr (F16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c,
-                                                  0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
-                                                   c, 0, 0, 0);
-}
-
 // 16 int8 -> 16 exact 16-bit floats, as two 8-element operands (k 0..7, 8..15)
 template <bool F16>
 __device__ __forceinline__ void widen_i8x16(const u32x4& w, u32x4& lo, u32x4& hi) {
@@ -1423,125 +1400,197 @@ __device__ __forceinline__ void widen_i8_body(const GemmArgs& p) {
   dst[1] = hi;
 }
 
-// T: 16-column tiles per workgroup (SKINNY_TILES, or 1 for the 16-column form)
-template <bool F16, int R, int T = SKINNY_TILES>
-__device__ __forceinline__ void gemm_w8a16_skinny_body(const GemmArgs& p) {
-  constexpr int STEPS = SKINNY_STEPS / R;
-  __shared__ f32x4 part[SKINNY_WAVES][R][T][64];
-  if (blockDim.x != SKINNY_WAVES * 64) return;  // launch shape must match the kernel
+// ------------------------------------------------ few rows of A (decode)
+// Y = A . B for M <= 64 rows and K-contiguous operands, in every GEMM mode,
+// and with int8 weights (W8: A bf16 / f16, B int8 widened exactly, the column
+// scale in the epilogue).  Such a product is bound by reading B once, and a
+// tiled kernel would leave it to few CUs.  A workgroup owns 16 T columns and
+// all of K; its W waves take 128-byte units of K in turn, each through its own
+// LDS ring of NS units filled by direct DMA -- instructions of 8 whole
+// 128-byte lines -- and waits for its own loads only, so the loop holds no
+// barrier.  B rows feed the MFMA A port and the 16 R rows of A (from L2) the
+// B port, in the tiled kernels' LDS layout.  The waves' partial tiles are
+// added in wave order through LDS: no workspace, no second launch, the same
+// bits every run.  Measured on MI355X with operands from HBM: bf16 16 x 4096
+// x 4096 17.3 (64 x 64 tiles) -> 10.0 us, 16 x 11008 x 4096 21.5 -> 18.7, 64
+// x 4096 x 4096 22.3 -> 14.8; int8 weights 16 x 8192 x 8192 23.1 (each lane
+// loading its own operand chunks, 64-byte pieces of 16 rows) -> 18.8, 16 x
+// 11008 x 4096 21.0 -> 12.8, 64 x 8192 x 8192 48.7 -> 29.9.  About 5 us of
+// these are the launch and the first loads; the rest is HBM.
+// FEW: M <= 8 (W8: 4), one DMA instruction brings all of A's unit; the other
+// rows of the operand hold whatever LDS holds and feed outputs that are not
+// stored (an output row depends on its own row of A alone).
+constexpr int FEW_LDS = 160 * 1024;
+
+template <int MODE, bool W8, int R, int T, int W, int NS, bool FEW = false>
+__device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
+  constexpr int ES = W8 ? 1 : (MODE == GEMM_I8) ? 1 : (MODE == GEMM_F32) ? 4 : 2;  // bytes of a B element
+  constexpr int AROW = W8 ? 256 : 128;       // bytes of an A row's unit
+  constexpr int AU = 16 * R * AROW, BU = 16 * T * 128, UNIT = AU + BU;
+  constexpr int DA = FEW ? 1 : AU / 1024, DB = BU / 1024, DPU = DA + DB;
+  static_assert(W * NS * UNIT <= FEW_LDS && NS >= 2 && R * T * 1024 <= NS * UNIT, "the rings fit LDS");
+  if (blockDim.x != W * 64) return;  // launch shape must match the kernel
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int g = lane >> 4;
-  const int i = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g4 = lane >> 4, l16 = lane & 15;
   const int n0 = blockIdx.x * 16 * T;
-  const int kw = (p.K + SKINNY_WAVES * 64 - 1) / (SKINNY_WAVES * 64) * 64;  // K range of one wave
-  const int kb = wave * kw;
-  const int ke = min(p.K, kb + kw);
-  // rows past M repeat row M-1 and columns past N repeat column N-1: their
-  // outputs are never stored
-  const char* arow[R];
+  const long long lda = p.a_s0 * (W8 ? 2 : ES), ldb = p.b_s0 * ES;
+  const char* abase = (const char*)p.a;
+  const char* bbase = (const char*)p.b + (long long)n0 * ldb;
+  const int kb = p.K * ES;                   // bytes of a B row
+  const int units = (kb + 127) / 128;
+  const int tb = kb - (units - 1) * 128;     // bytes of the last unit (a multiple of 16)
+  const int nloc = units > wave ? (units - wave + W - 1) / W : 0;
+  char* ring = lds + wave * NS * UNIT;
+  const uint32_t ring32 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)ring;
+  // DMA instruction u: 8 rows x 128 bytes (W8's A: 4 rows x 256 bytes), the
+  // 16-byte chunks XOR-swizzled by the row.  Rows past M repeat row M - 1 and
+  // columns past N column N - 1: their outputs are never stored.
+  uint32_t aoff[DA], boff[DB];
+  auto achunk = [&](int u) {
+    const int row = W8 ? u * 4 + (lane >> 4) : u * 8 + (lane >> 3);
+    return W8 ? (lane & 15) ^ (row & 15) : (lane & 7) ^ ((row >> 1) & 7);
+  };
+  auto bchunk = [&](int u) { return (lane & 7) ^ (((u * 8 + (lane >> 3)) >> 1) & 7); };
 #pragma unroll
-  for (int r = 0; r < R; ++r) arow[r] = (const char*)p.a + (long long)min(16 * r + i, p.M - 1) * p.a_s0 * 2;
-  const char* bcol[T];
+  for (int u = 0; u < DA; ++u) {
+    const int row = W8 ? u * 4 + (lane >> 4) : u * 8 + (lane >> 3);
+    aoff[u] = (uint32_t)((long long)min(row, p.M - 1) * lda) + (achunk(u) << 4);
+  }
 #pragma unroll
-  for (int t = 0; t < T; ++t) bcol[t] = (const char*)p.b + (long long)min(n0 + 16 * t + i, p.N - 1) * p.b_s0;
-  f32x4 acc[R][T];
+  for (int u = 0; u < DB; ++u) boff[u] = (uint32_t)((long long)min(u * 8 + (lane >> 3), p.N - 1 - n0) * ldb) + (bchunk(u) << 4);
+  auto issue = [&](int j) {
+    const int unit = wave + W * j;
+    const char* as = abase + (long long)unit * AROW;
+    const char* bs = bbase + (long long)unit * 128;
+    const uint32_t dst = ring32 + (uint32_t)(j % NS) * UNIT;
+    if (unit == units - 1 && tb != 128) {
+      // chunks past K repeat the row's last one (zeroed as they are used)
+#pragma unroll
+      for (int u = 0; u < DB; ++u) dma16_asm(bs, boff[u] - max(0, (bchunk(u) << 4) + 16 - tb), dst + AU + u * 1024);
+#pragma unroll
+      for (int u = 0; u < DA; ++u)
+        dma16_asm(as, aoff[u] - max(0, (achunk(u) << 4) + 16 - tb * (W8 ? 2 : 1)), dst + u * 1024);
+    } else {
+#pragma unroll
+      for (int u = 0; u < DB; ++u) dma16_asm(bs, boff[u], dst + AU + u * 1024);
+#pragma unroll
+      for (int u = 0; u < DA; ++u) dma16_asm(as, aoff[u], dst + u * 1024);
+    }
+  };
+  f32x4 acf[R][T];
+  i32x4 aci[R][T];
 #pragma unroll
   for (int r = 0; r < R; ++r)
-#pragma unroll
-    for (int t = 0; t < T; ++t) acc[r][t] = (f32x4){};
-  // Weights use plain (cacheable) loads: an instruction reads 64 bytes of
-  // each of its 16 columns, so every 128-byte line is requested in two halves
-  // by consecutive steps, and with nontemporal loads the line was fetched
-  // again for its second half (rocprofv3 FETCH_SIZE 1.20x the algorithmic
-  // bytes at 16 x 8192 x 8192; 16 x 8192 x 8192 25.4 -> 23.0 us and
-  // 32 x 8192 x 8192 32.8 -> 30.0 us with six rotating input sets).
-  // STEPS 64-element K steps in flight per wave.  Over whole batches, step st
-  // of the next batch is loaded into step st's registers as soon as their
-  // MFMAs have issued, so the loads stream without a gap between batches (no
-  // per-lane branch around them, so each MFMA waits only for its own
-  // step's loads).  A last partial batch loads per lane: a lane whose 16 k
-  // lie past the range contributes zeros (K % 16 == 0).
-  u32x4 a0[STEPS][R], a1[STEPS][R], bw[STEPS][T];
-  auto load = [&](int st, int k0) {
-    const int kk = k0 + st * 64 + 16 * g;
-#pragma unroll
-    for (int t = 0; t < T; ++t) bw[st][t] = *(const u32x4*)(bcol[t] + kk);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      a0[st][r] = *(const u32x4*)(arow[r] + 2 * (long long)kk);
-      a1[st][r] = *(const u32x4*)(arow[r] + 2 * (long long)kk + 16);
-    }
-    __builtin_amdgcn_sched_barrier(0);  // keep the steps' loads in step order
-  };
-  auto mma = [&](int st) {
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      u32x4 lo, hi;
-      widen_i8x16<F16>(bw[st][t], lo, hi);
+      if constexpr (MODE == GEMM_I8) aci[r][t] = (i32x4){};
+      else acf[r][t] = (f32x4){};
+    }
+  for (int j = 0; j < NS && j < nloc; ++j) issue(j);
+  for (int j = 0; j < nloc; ++j) {
+    // unit j has landed once at most the later units' loads are in flight
+    if (j + NS <= nloc) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * DPU) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const char* st = ring + (j % NS) * UNIT;
+    const bool tail = wave + W * j == units - 1 && tb != 128;
+    u32x4 av[2][R][W8 ? 2 : 1], bv[2][T];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int c = 4 * h + g4;
+#pragma unroll
+      for (int t = 0; t < T; ++t) bv[h][t] = *(const u32x4*)(st + AU + (16 * t + l16) * 128 + ((c ^ ((l16 >> 1) & 7)) << 4));
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        acc[r][t] = mfma16x16x32<F16>(a0[st][r], lo, acc[r][t]);
-        acc[r][t] = mfma16x16x32<F16>(a1[st][r], hi, acc[r][t]);
+        if constexpr (W8) {
+          av[h][r][0] = *(const u32x4*)(st + (16 * r + l16) * 256 + (((2 * c) ^ l16) << 4));
+          av[h][r][1] = *(const u32x4*)(st + (16 * r + l16) * 256 + (((2 * c + 1) ^ l16) << 4));
+        } else {
+          av[h][r][0] = *(const u32x4*)(st + (16 * r + l16) * 128 + ((c ^ ((l16 >> 1) & 7)) << 4));
+        }
+      }
+      if (tail && c * 16 >= tb) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) bv[h][t] = (u32x4){0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int q = 0; q < (W8 ? 2 : 1); ++q) av[h][r][q] = (u32x4){0u, 0u, 0u, 0u};
       }
     }
-  };
-  constexpr int BK = STEPS * 64;
-  int k0 = kb;
-  const int kwhole = kb + (ke > kb ? (ke - kb) / BK * BK : 0);  // end of the whole batches
-  if (k0 < kwhole) {
+    // the unit's reads have returned before its slot is refilled
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (j + NS < nloc) issue(j + NS);
 #pragma unroll
-    for (int st = 0; st < STEPS; ++st) load(st, k0);
-    for (; k0 + BK < kwhole; k0 += BK) {
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int st = 0; st < STEPS; ++st) {
-        mma(st);
-        load(st, k0 + BK);
+      for (int t = 0; t < T; ++t) {
+        if constexpr (W8) {
+          u32x4 lo, hi;
+          widen_i8x16<MODE == GEMM_F16>(bv[h][t], lo, hi);
+#pragma unroll
+          for (int r = 0; r < R; ++r) {
+            mfma16_step<MODE>(lo, av[h][r][0], acf[r][t], aci[r][t]);
+            mfma16_step<MODE>(hi, av[h][r][1], acf[r][t], aci[r][t]);
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < R; ++r) mfma16_step<MODE>(bv[h][t], av[h][r][0], acf[r][t], aci[r][t]);
+        }
       }
-    }
-#pragma unroll
-    for (int st = 0; st < STEPS; ++st) mma(st);
-    k0 += BK;
   }
-  if (k0 < ke) {
-#pragma unroll
-    for (int st = 0; st < STEPS; ++st) {
-      if (k0 + st * 64 + 16 * g < ke) {
-        load(st, k0);
-      } else {
-#pragma unroll
-        for (int t = 0; t < T; ++t) bw[st][t] = (u32x4){};
-#pragma unroll
-        for (int r = 0; r < R; ++r) a0[st][r] = a1[st][r] = (u32x4){};
-      }
-    }
-#pragma unroll
-    for (int st = 0; st < STEPS; ++st) mma(st);
-  }
-  // lane (g, i) holds rows 16r + 4g .. +3 of column n0 + 16t + i; wave 0
-  // adds the waves' tiles in wave order, scales and stores
+  __syncthreads();  // every wave is done with its ring
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int t = 0; t < T; ++t) part[wave][r][t][lane] = acc[r][t];
-  __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int t = 0; t < T; ++t) {
-    const int n = n0 + 16 * t + i;
-    if (n >= p.N) continue;
-    const float sc = load_as_f32(p.bscale, n, p.bscale_dtype);
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      f32x4 sum = part[0][r][t][lane];
-#pragma unroll
-      for (int w = 1; w < SKINNY_WAVES; ++w) sum += part[w][r][t][lane];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int m = 16 * r + 4 * g + j;
-        if (m < p.M) store_from_f32(p.c, (long long)m * p.c_s0 + n, p.c_dtype, sum[j] * sc);
-      }
+    for (int t = 0; t < T; ++t) {
+      f32x4 v;
+      if constexpr (MODE == GEMM_I8) v = __builtin_bit_cast(f32x4, aci[r][t]);
+      else v = acf[r][t];
+      *(f32x4*)(lds + ((wave * R * T + r * T + t) * 64 + lane) * 16) = v;
     }
+  __syncthreads();
+  // fragment f (rows 16 (f / T), columns 16 (f % T)) is wave f % W's: lane
+  // (g4, l16) holds row l16, columns 4 g4 .. + 3
+  for (int f = wave; f < R * T; f += W) {
+    f32x4 sf[1][1];
+    i32x4 si[1][1];
+    sf[0][0] = *(const f32x4*)(lds + (f * 64 + lane) * 16);
+    si[0][0] = __builtin_bit_cast(i32x4, sf[0][0]);
+#pragma unroll
+    for (int w = 1; w < W; ++w) {
+      const f32x4 v = *(const f32x4*)(lds + ((w * R * T + f) * 64 + lane) * 16);
+      if constexpr (MODE == GEMM_I8) si[0][0] += __builtin_bit_cast(i32x4, v);
+      else sf[0][0] += v;
+    }
+    gemm_epilogue<MODE, 1, 1, 0, 16>(p, sf, si, 16 * (f / T), n0 + 16 * (f % T), lane);
+  }
+}
+
+// The forms of one row class (R groups of 16 rows of A): GemmArgs::tile is
+// the column groups T per workgroup, picked by the host with the workgroup
+// size that form has (g950rt.cpp, kFewRows).
+template <int MODE, bool W8, int R>
+__device__ __forceinline__ void gemm_few_rows(const GemmArgs& p, char* lds) {
+  if constexpr (R == 1) {
+    auto forms = [&](auto few) {
+      constexpr bool F = decltype(few)::value;
+      if (p.tile == 1) gemm_stream_body<MODE, W8, 1, 1, 8, W8 ? 3 : 4, F>(p, lds);
+      else if (p.tile == 3) gemm_stream_body<MODE, W8, 1, 3, 8, 2, F>(p, lds);
+      else if (p.tile == 4) gemm_stream_body<MODE, W8, 1, 4, W8 ? 4 : 8, W8 ? 3 : 2, F>(p, lds);
+      else if constexpr (W8) gemm_stream_body<MODE, W8, 1, 2, 8, 2, F>(p, lds);
+    };
+    if (p.M <= (W8 ? 4 : 8)) forms(std::true_type{});
+    else forms(std::false_type{});
+  } else if constexpr (R == 2) {
+    if (p.tile == 1) gemm_stream_body<MODE, W8, 2, 1, W8 ? 4 : 8, W8 ? 4 : 3>(p, lds);
+    else if (p.tile == 2) gemm_stream_body<MODE, W8, 2, 2, W8 ? 4 : 8, W8 ? 3 : 2>(p, lds);
+    else if constexpr (W8) gemm_stream_body<MODE, W8, 2, 3, 4, 2>(p, lds);
+    else gemm_stream_body<MODE, W8, 2, 4, 4, 3>(p, lds);
+  } else {
+    if (p.tile == 1) gemm_stream_body<MODE, W8, 4, 1, W8 ? 4 : 8, 2>(p, lds);
+    else if (W8 || p.tile == 2) gemm_stream_body<MODE, W8, 4, 2, 4, W8 ? 2 : 3>(p, lds);
+    else if constexpr (!W8) gemm_stream_body<MODE, W8, 4, 4, 4, 2>(p, lds);
   }
 }
 
@@ -1634,6 +1683,29 @@ G950_GEMM_MFMA(g950_gemm_i8_256x256, g950::GEMM_I8, 4, 2, 0, false)
 G950_GEMM_MFMA(g950_gemm_bf16_256x256_kt, g950::GEMM_BF16, 4, 2, 0, true)
 G950_GEMM_MFMA(g950_gemm_f16_256x256_kt, g950::GEMM_F16, 4, 2, 0, true)
 G950_GEMM_MFMA(g950_gemm_i8_256x256_kt, g950::GEMM_I8, 4, 2, 0, true)
+// few rows of A: up to 16, 32 and 64
+#define G950_FEW_ROWS(NAME, MODE, W8, R)                                                   \
+  extern "C" __global__ __launch_bounds__(512) void NAME(const g950::GemmArgs p) {         \
+    __shared__ __attribute__((aligned(1024))) char lds[g950::FEW_LDS];                     \
+    g950::gemm_few_rows<MODE, W8, R>(p, lds);                                              \
+  }
+#define G950_GEMM_SKINNY(TY, MODE)                          \
+  G950_FEW_ROWS(g950_gemm_skinny16_##TY, MODE, false, 1)    \
+  G950_FEW_ROWS(g950_gemm_skinny32_##TY, MODE, false, 2)    \
+  G950_FEW_ROWS(g950_gemm_skinny64_##TY, MODE, false, 4)
+G950_GEMM_SKINNY(bf16, g950::GEMM_BF16)
+G950_GEMM_SKINNY(f16, g950::GEMM_F16)
+G950_GEMM_SKINNY(f32, g950::GEMM_F32)
+G950_GEMM_SKINNY(i8, g950::GEMM_I8)
+// int8 weights; _c16 and the plain name are one kernel: the names tell the
+// two classes of grids that callers and tests know
+#define G950_W8A16_SKINNY(TY, MODE)                                \
+  G950_FEW_ROWS(g950_gemm_w8a16_skinny_##TY, MODE, true, 1)        \
+  G950_FEW_ROWS(g950_gemm_w8a16_skinny_c16_##TY, MODE, true, 1)    \
+  G950_FEW_ROWS(g950_gemm_w8a16_skinny32_##TY, MODE, true, 2)      \
+  G950_FEW_ROWS(g950_gemm_w8a16_skinny64_##TY, MODE, true, 4)
+G950_W8A16_SKINNY(bf16, g950::GEMM_BF16)
+G950_W8A16_SKINNY(f16, g950::GEMM_F16)
 extern "C" __global__ __launch_bounds__(256) void g950_transpose_b16(const g950::GemmArgs p) {
   g950::transpose16_body(p);
 }
@@ -1657,21 +1729,6 @@ extern "C" __global__ __launch_bounds__(256) void g950_i8_sums(const g950::I8Sum
 extern "C" __global__ __launch_bounds__(256) void g950_gemm_w8a16_bf16_128x128(const g950::GemmArgs p) {
   g950::gemm_w8a16_body<false>(p);
 }
-// W8A16 decode: up to 16, 32 and 64 rows of A
-#define G950_W8A16_SKINNY(NAME, F16, R, T)                                                 \
-  extern "C" __global__ __launch_bounds__(512) void NAME(const g950::GemmArgs p) {        \
-    g950::gemm_w8a16_skinny_body<F16, R, T>(p);                                            \
-  }
-G950_W8A16_SKINNY(g950_gemm_w8a16_skinny_bf16, false, 1, 2)
-G950_W8A16_SKINNY(g950_gemm_w8a16_skinny_f16, true, 1, 2)
-G950_W8A16_SKINNY(g950_gemm_w8a16_skinny32_bf16, false, 2, 2)
-G950_W8A16_SKINNY(g950_gemm_w8a16_skinny32_f16, true, 2, 2)
-G950_W8A16_SKINNY(g950_gemm_w8a16_skinny64_bf16, false, 4, 2)
-G950_W8A16_SKINNY(g950_gemm_w8a16_skinny64_f16, true, 4, 2)
-// 16 columns per workgroup: twice the workgroups, for grids the 32-column
-// form leaves short of the CUs and for a one-row A (whose loads cost little)
-G950_W8A16_SKINNY(g950_gemm_w8a16_skinny_c16_bf16, false, 1, 1)
-G950_W8A16_SKINNY(g950_gemm_w8a16_skinny_c16_f16, true, 1, 1)
 extern "C" __global__ __launch_bounds__(256) void g950_gemm_w8a16_f16_128x128(const g950::GemmArgs p) {
   g950::gemm_w8a16_body<true>(p);
 }
