@@ -22,6 +22,7 @@ struct RowArgs {
   int stat_dtype;     // dtype code of stat0/stat1
   void* part;         // split rows: [rows * splits] partial records of 4 floats
   int splits;         // split rows: chunks per row
+  int masked;         // split rows, v1: masked 16-byte vectors (x and y rows share their phase)
 };
 
 // workgroup tile of the whole-slab MFMA GEMM kernels (M x N outputs)

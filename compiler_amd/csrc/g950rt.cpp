@@ -322,7 +322,10 @@ int launch(g950_module* m, const std::string& name, unsigned grid, unsigned bloc
 constexpr long long kRsChunkVecs = 1024;
 
 int launch_split_rows(g950_module* m, const char* op, RowArgs& a, uint32_t dt, int v, void* stream) {
-  const long long nvec = a.cols / v;
+  // masked rows: vectors from the 16-byte boundary at or below the row start,
+  // whatever the row's phase
+  const int vmax = 16 / itemsize(dt);
+  const long long nvec = a.masked ? ((long long)a.cols + 2 * (vmax - 1)) / vmax : a.cols / v;
   const long long splits = (nvec + kRsChunkVecs - 1) / kRsChunkVecs;
   const long long blocks = (long long)a.rows * splits;
   if (blocks > 0x7FFFFFFF) return fail(G950_USAGE, "%s: too many row chunks", op);
@@ -353,8 +356,10 @@ int launch_rows(g950_module* m, const char* op, RowArgs& a, uint32_t dt, const V
   // rows that are not whole aligned 16-byte vectors: masked aligned vectors
   // when one wave holds a row at any phase and y's rows share x's phase
   // (empty rows never: their start address need not lie in any allocation)
-  if (!vec && a.cols > 0 && (isz == 2 || isz == 4) && ((x.addr() - y.addr()) % 16) == 0 &&
-      (((a.x_row - a.y_row) * isz) % 16) == 0 && (x.addr() % isz) == 0) {
+  const bool phase = a.cols > 0 && (isz == 2 || isz == 4) && ((x.addr() - y.addr()) % 16) == 0 &&
+                     (((a.x_row - a.y_row) * isz) % 16) == 0 && (x.addr() % isz) == 0 &&
+                     (!p0 || p0->addr() % isz == 0) && (!p1 || p1->addr() % isz == 0);
+  if (!vec && phase) {
     static const int kItems[] = {1, 2, 4, 6, 8};
     for (int items : kItems) {
       if ((long long)items * 64 * vmax >= (long long)a.cols + vmax - 1) {
@@ -371,7 +376,26 @@ int launch_rows(g950_module* m, const char* op, RowArgs& a, uint32_t dt, const V
   // one workgroup per row leaves most of the chip idle when rows are few and
   // long: split them (two or more chunks each) instead
   const long long cus = m ? m->cus : 256;
-  const bool few = (long long)a.rows * 2 < cus && nvec > kRsChunkVecs;
+  // 16-byte vectors of a row, at any phase if rows are not aligned
+  const long long mvec = vec ? nvec : ((long long)a.cols + 2 * (vmax - 1)) / vmax;
+  const bool few = (long long)a.rows * 2 < cus && (phase ? mvec : nvec) > kRsChunkVecs;
+  // rows that are not whole aligned vectors or that no register form holds:
+  // one workgroup per row of masked vectors.  Softmax holds 16384 vectors
+  // (packed), the norms 8192 (their parameters come with the row); logsumexp,
+  // which reads x once either way, splits rows past 2048.  Measured on MI355X
+  // against the split pair (us): softmax bf16 [256, 50001] 41.9 -> 14.1,
+  // aligned [512, 65536] 33.5 -> 30.2, LayerNorm bf16 [4555, 5001] 79.3 ->
+  // 27.3; logsumexp bf16 [512, 100000] 21.1 split, 30.0 as one workgroup.
+  if (phase && !few && (!vec || !pick)) {
+    static const struct { int items, block; } kRl[] = {{4, 256}, {8, 256}, {8, 1024}, {16, 1024}};
+    const int forms = !strcmp(op, "softmax") ? 4 : !strcmp(op, "logsumexp") ? 2 : 3;
+    for (int f = 0; f < forms; ++f) {
+      const auto& c = kRl[f];
+      if (mvec > (long long)c.items * c.block) continue;
+      snprintf(name, sizeof name, "g950_rl_%s_%s_v1_i%d_b%d", op, rr_dtype(dt), c.items, c.block);
+      return launch(m, name, (unsigned)a.rows, (unsigned)c.block, a, stream);
+    }
+  }
   // LayerNorm over many rows of at most 512 vectors: parameters staged in LDS
   // once per 4-wave workgroup of 8 rows (g950_rw_*) instead of once per
   // one-row wave
@@ -386,6 +410,7 @@ int launch_rows(g950_module* m, const char* op, RowArgs& a, uint32_t dt, const V
     return launch(m, name, row_grid(m, a.rows, pick->block, pick->waves), (unsigned)pick->block, a,
                   stream);
   }
+  a.masked = !vec && phase;
   return launch_split_rows(m, op, a, dt, v, stream);
 }
 

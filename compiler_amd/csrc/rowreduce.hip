@@ -16,7 +16,8 @@
 //             round the product and the sum, as the reference's typed ops do)
 // All arithmetic is fp32; 16-bit inputs widen exactly and outputs round once.
 //
-// Two kernel shapes:
+// Three kernel shapes (and rw / rm, one-wave rows with parameters in LDS and
+// masked edges):
 //   rr_regs  -- the row lives in registers.  Each thread owns ITEMS vectors of
 //               VEC elements (VEC*sizeof(T) = 16 B => one 128-bit nontemporal
 //               load each) of a row handled by one BLOCK-thread workgroup.
@@ -26,6 +27,9 @@
 //               next row's loads are in flight while the current row is
 //               reduced.  The tail of a non-power-of-two row is a per-vector
 //               predicate; x is read from HBM once and y written once.
+//   rl       -- one workgroup per row of masked 16-byte vectors: rows that are
+//               long or not whole aligned vectors, enough of them to fill the
+//               chip.
 //   rs       -- rows longer than the register budget, or too few rows to
 //               fill the chip: each row is cut into register-resident chunks,
 //               one workgroup per chunk, partial statistics go through a small
@@ -152,6 +156,14 @@ __device__ __forceinline__ void load_param(const void* base, long long idx, floa
       out[0] = Elem<T>::to_f32(((const uint16_t*)base)[idx]);
     }
   }
+}
+
+// element idx widened
+template <typename T>
+__device__ __forceinline__ float load_first(const void* base, long long idx) {
+  float v;
+  load_vec<T, 1>(base, idx, &v);
+  return v;
 }
 
 // Raw (undecoded) row vectors: what one 16-byte (or scalar) load returns.
@@ -741,6 +753,157 @@ __device__ __forceinline__ void rm_body(const RowArgs& a) {
   }
 }
 
+// ------------------------------------------------------- long masked rows
+// How a masked kernel's vectors meet a row of `cols` elements whose start
+// lies ph elements past a 16-byte boundary: vector j holds columns j*VEC - ph
+// .. + VEC - 1.  (The rules of rm_body, for vectors spread over a workgroup.)
+template <typename T, int VEC>
+struct MaskedRow {
+  using IO = RawIO<T, VEC>;
+  using R = typename IO::type;
+  char* lo;  // the 16-byte boundary at or below the row start
+  int ph, cols;
+  __device__ __forceinline__ MaskedRow(const void* p, long long row, long long stride, int n) {
+    const uintptr_t at = (uintptr_t)p + (uintptr_t)(row * stride * (long long)sizeof(T));
+    ph = (int)((at & 15) / sizeof(T));
+    lo = (char*)(at & ~(uintptr_t)15);
+    cols = n;
+  }
+  __device__ __forceinline__ int col(int j) const { return j * VEC - ph; }
+  __device__ __forceinline__ bool live(int j) const { return col(j) < cols; }
+  __device__ __forceinline__ bool whole(int j) const { return col(j) >= 0 && col(j) + VEC <= cols; }
+  __device__ __forceinline__ bool ok(int j, int e) const { return col(j) + e >= 0 && col(j) + e < cols; }
+  // elements of a live vector, those outside the row as `ident`
+  __device__ __forceinline__ void unpack(const R& r, int j, float ident, float* v) const {
+    IO::unpack(r, v);
+    if (!whole(j)) {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[e] = ok(j, e) ? v[e] : ident;
+    }
+  }
+  __device__ __forceinline__ void store(int j, const float* o) const {
+    if (whole(j)) {
+      store_vec<T, VEC>(lo, (long long)j * VEC, o);
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e)
+        if (ok(j, e)) store_vec<T, 1>(lo, (long long)j * VEC + e, &o[e]);
+    }
+  }
+  // per-column parameters of vector j: one load of any alignment where all of
+  // its columns lie in the row, else element by element
+  __device__ __forceinline__ void params(const void* base, int j, float* w) const {
+    typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+    if (whole(j)) {
+      const u32x4_any t = *(const u32x4_any*)((const char*)base + (long long)col(j) * (long long)sizeof(T));
+      IO::unpack(__builtin_bit_cast(R, (u32x4){t[0], t[1], t[2], t[3]}), w);
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) w[e] = ok(j, e) ? load_first<T>(base, col(j) + e) : 0.0f;
+    }
+  }
+};
+
+// One workgroup per row, the row in registers: rows no one-wave or aligned
+// kernel holds (too long, or not whole aligned 16-byte vectors), where there
+// are rows enough to fill the chip.  x is read once and y written once, in
+// one launch; the split pair reads x twice, and its element-wise form (which
+// odd rows took before) loads 2 or 4 bytes a lane.  Bound by HBM and, at 256
+// rows, by the single round of one workgroup per CU: bf16 [256, 50001]
+// softmax 41.9 -> 14.1 us on MI355X (51 MB, 3.6 TB/s), [4555, 5001] 70 -> 20
+// (4.6 TB/s), [512, 130001] 185 -> 68.
+// PACKED (softmax and logsumexp): the row stays in its storage type and is
+// widened in each of the passes, so 16-bit rows of up to 131072 elements fit
+// the 128 registers that 1024 threads leave each; the exponentials are
+// computed twice.
+template <int OP, typename T, int VEC, int ITEMS, int BLOCK, bool PACKED>
+__device__ __forceinline__ void rl_body(const RowArgs& a) {
+  using M = MaskedRow<T, VEC>;
+  using R = typename M::R;
+  __shared__ float scratch[BLOCK / 64];
+  if (a.cols <= 0) return;  // no row element: no vector may be read
+  const int tid = threadIdx.x, row = blockIdx.x;
+  const M x(a.x, row, a.x_row, a.cols), y(a.y, row, a.y_row, a.cols);
+  constexpr float ident = (OP == ROW_SOFTMAX || OP == ROW_LOGSUMEXP) ? -__builtin_huge_valf() : 0.0f;
+  R raw[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const int j = tid + i * BLOCK;
+    if (x.live(j)) raw[i] = M::IO::load(x.lo, (long long)j * VEC);
+  }
+  if constexpr (!PACKED) {
+    float v[ITEMS][VEC];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+      const int j = tid + i * BLOCK;
+      if (x.live(j)) {
+        x.unpack(raw[i], j, ident, v[i]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[i][e] = ident;
+      }
+    }
+    row_finish<OP, T, VEC, ITEMS, BLOCK>(
+        a, row, v, tid, scratch,
+        row_edge([&](int i) { return x.live(tid + i * BLOCK); }, [&](int i, int e) { return x.ok(tid + i * BLOCK, e); },
+                 [&](int i, float* w, float* bb) {
+                   if constexpr (row_has_w(OP)) x.params(a.w, tid + i * BLOCK, w);
+                   if constexpr (row_has_b(OP)) x.params(a.b, tid + i * BLOCK, bb);
+                 },
+                 [&](int i, const float* o) { y.store(tid + i * BLOCK, o); }));
+  } else {
+    // each(f): f(vector index, its elements) for this lane's live vectors
+    auto each = [&](auto f) {
+#pragma unroll
+      for (int i = 0; i < ITEMS; ++i) {
+        const int j = tid + i * BLOCK;
+        if (x.live(j)) {
+          float v[VEC];
+          x.unpack(raw[i], j, ident, v);
+          f(j, v);
+        }
+      }
+    };
+    float m4[4] = {ident, ident, ident, ident}, nan = 0.0f;
+    each([&](int, const float* v) {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        m4[e & 3] = fmaxf(m4[e & 3], v[e]);
+        if constexpr (OP == ROW_LOGSUMEXP) nan = (v[e] != v[e]) ? 1.0f : nan;
+      }
+    });
+    const float m = block_reduce<OpMax, BLOCK>(fmaxf(fmaxf(m4[0], m4[1]), fmaxf(m4[2], m4[3])), scratch);
+    if constexpr (OP == ROW_LOGSUMEXP) nan = block_reduce<OpMax, BLOCK>(nan, scratch);
+    const float mL = m * kLog2e;
+    float s4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (OP == ROW_SOFTMAX || __builtin_fabsf(m) != __builtin_huge_valf()) {
+      with_exp_form(m, [&](auto fc) {
+        constexpr bool F = decltype(fc)::value;
+        each([&](int, const float* v) {
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) s4[e & 3] += row_exp<F>(v[e], m, mL);  // masked: exp(-inf) = 0
+        });
+      });
+    }
+    const float s = block_reduce<OpSum, BLOCK>((s4[0] + s4[1]) + (s4[2] + s4[3]), scratch);
+    if constexpr (OP == ROW_LOGSUMEXP) {
+      if (tid == 0)
+        store_from_f32(a.stat0, (long long)row * a.stat0_stride, a.stat_dtype, lse_finish(m, s, nan != 0.0f));
+    } else {
+      const float inv = 1.0f / s;
+      with_exp_form(m, [&](auto fc) {
+        constexpr bool F = decltype(fc)::value;
+        each([&](int j, const float* v) {
+          float o[VEC];
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) o[e] = row_exp<F>(v[e], m, mL) * inv;
+          y.store(j, o);
+        });
+      });
+    }
+  }
+}
+
 // ------------------------------------------------------------- split rows
 // Rows longer than one workgroup's registers hold, or too few rows to fill
 // the chip, are cut into chunks of RS_CHUNK_VECS vectors; one RS_BLOCK-thread
@@ -791,13 +954,42 @@ __device__ __forceinline__ void rs_load(const RowArgs& a, int row, int split, fl
   }
 }
 
+// The same chunk of a row that is not whole aligned vectors (MaskedRow): ok
+// marks the live vectors, elements outside the row read as the identity.
+// Against element loads: softmax bf16 [64, 50001] 12.4 -> 9.0 us, fp32 [400,
+// 100001] 115 -> 77, logsumexp bf16 [100, 100001] 15.5 -> 9.3.
 template <int OP, typename T, int VEC>
-__device__ __forceinline__ void rs_part_body(const RowArgs& a) {
-  __shared__ float scratch[RS_BLOCK / 64];
+__device__ __forceinline__ void rs_load_masked(const MaskedRow<T, VEC>& x, int split, float (&v)[RS_ITEMS][VEC],
+                                               bool (&ok)[RS_ITEMS], bool cached) {
+  using IO = RawIO<T, VEC>;
+  constexpr float ident = (OP == ROW_SOFTMAX || OP == ROW_LOGSUMEXP) ? -__builtin_huge_valf() : 0.0f;
+  const int base = split * (RS_BLOCK * RS_ITEMS);
+  typename IO::type raw[RS_ITEMS];
+#pragma unroll
+  for (int i = 0; i < RS_ITEMS; ++i) {
+    const int j = base + threadIdx.x + i * RS_BLOCK;
+    ok[i] = x.live(j);
+    if (ok[i]) raw[i] = cached ? IO::load_cached(x.lo, (long long)j * VEC) : IO::load(x.lo, (long long)j * VEC);
+  }
+#pragma unroll
+  for (int i = 0; i < RS_ITEMS; ++i) {
+    if (ok[i]) {
+      x.unpack(raw[i], base + threadIdx.x + i * RS_BLOCK, ident, v[i]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) v[i][e] = ident;
+    }
+  }
+}
+
+template <int OP, typename T, int VEC, bool MASKED = false>
+__device__ __forceinline__ void rs_part_body(const RowArgs& a, float* scratch) {
   const int row = blockIdx.x / a.splits, split = blockIdx.x % a.splits;
   float v[RS_ITEMS][VEC];
   bool ok[RS_ITEMS];
-  rs_load<OP, T, VEC>(a, row, split, v, ok, true);
+  const MaskedRow<T, VEC> x(a.x, row, a.x_row, a.cols);
+  if constexpr (MASKED) rs_load_masked<OP, T, VEC>(x, split, v, ok, true);
+  else rs_load<OP, T, VEC>(a, row, split, v, ok, true);
   f32x4 p = {0.0f, 0.0f, 0.0f, 0.0f};
   if constexpr (OP == ROW_SOFTMAX || OP == ROW_LOGSUMEXP) {
     float m = -__builtin_huge_valf(), nan = 0.0f;
@@ -840,8 +1032,8 @@ __device__ __forceinline__ void rs_part_body(const RowArgs& a) {
     p[0] = block_reduce<OpSum, RS_BLOCK>(s, scratch);
     p[1] = block_reduce<OpSum, RS_BLOCK>(q, scratch);
   } else {
-    const int first = split * (RS_BLOCK * RS_ITEMS * VEC);
-    const float n = (float)min(RS_BLOCK * RS_ITEMS * VEC, a.cols - first);
+    const int first = split * (RS_BLOCK * RS_ITEMS * VEC) - (MASKED ? x.ph : 0);
+    const float n = (float)(min(first + RS_BLOCK * RS_ITEMS * VEC, a.cols) - max(first, 0));
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < RS_ITEMS; ++i)
@@ -854,6 +1046,7 @@ __device__ __forceinline__ void rs_part_body(const RowArgs& a) {
       if (ok[i]) {
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
+          if (MASKED && !x.ok(split * (RS_BLOCK * RS_ITEMS) + threadIdx.x + i * RS_BLOCK, e)) continue;
           const float c = v[i][e] - mean;
           q = fmaf(c, c, q);
         }
@@ -917,9 +1110,8 @@ __device__ __forceinline__ f32x4 rs_merge(const RowArgs& a, int row, float* scra
   return r;
 }
 
-template <int OP, typename T, int VEC>
-__device__ __forceinline__ void rs_final_body(const RowArgs& a) {
-  __shared__ float scratch[RS_BLOCK / 64];
+template <int OP, typename T, int VEC, bool MASKED = false>
+__device__ __forceinline__ void rs_final_body(const RowArgs& a, float* scratch) {
   if constexpr (OP == ROW_LOGSUMEXP) {
     const int row = blockIdx.x;
     const f32x4 r = rs_merge<OP>(a, row, scratch);
@@ -929,7 +1121,14 @@ __device__ __forceinline__ void rs_final_body(const RowArgs& a) {
     const int row = blockIdx.x / a.splits, split = blockIdx.x % a.splits;
     float v[RS_ITEMS][VEC];
     bool ok[RS_ITEMS];
-    rs_load<OP, T, VEC>(a, row, split, v, ok, false);  // in flight during the merge
+    const MaskedRow<T, VEC> x(a.x, row, a.x_row, a.cols), y(a.y, row, a.y_row, a.cols);
+    // in flight during the merge
+    if constexpr (MASKED) rs_load_masked<OP, T, VEC>(x, split, v, ok, false);
+    else rs_load<OP, T, VEC>(a, row, split, v, ok, false);
+    auto param = [&](const void* base, int j, float* w) {
+      if constexpr (MASKED) x.params(base, j, w);
+      else load_param<T, VEC>(base, (long long)j * VEC, w);
+    };
     const f32x4 r = rs_merge<OP>(a, row, scratch);
     void* yrow = (char*)a.y + (long long)row * a.y_row * (long long)sizeof(T);
     const int base = split * (RS_BLOCK * RS_ITEMS);
@@ -966,25 +1165,43 @@ __device__ __forceinline__ void rs_final_body(const RowArgs& a) {
         for (int e = 0; e < VEC; ++e) o[e] = row_exp<false>(v[i][e], sub, 0.0f) * mul;
       } else if constexpr (OP == ROW_RMSNORM) {
         float w[VEC];
-        load_param<T, VEC>(a.w, (long long)j * VEC, w);
+        param(a.w, j, w);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) o[e] = (v[i][e] * mul) * w[e];
       } else if constexpr (OP == ROW_LNROW) {
         float w[VEC], bb[VEC];
-        load_param<T, VEC>(a.w, (long long)j * VEC, w);
-        load_param<T, VEC>(a.b, (long long)j * VEC, bb);
+        param(a.w, j, w);
+        param(a.b, j, bb);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) o[e] = lnrow_affine<T>(v[i][e], sub, mul, w[e], bb[e]);
       } else {
         float w[VEC], bb[VEC];
-        load_param<T, VEC>(a.w, (long long)j * VEC, w);
-        load_param<T, VEC>(a.b, (long long)j * VEC, bb);
+        param(a.w, j, w);
+        param(a.b, j, bb);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) o[e] = (v[i][e] - sub) * mul * w[e] + bb[e];
       }
-      store_vec<T, VEC>(yrow, (long long)j * VEC, o);
+      if constexpr (MASKED) y.store(j, o);
+      else store_vec<T, VEC>(yrow, (long long)j * VEC, o);
     }
   }
+}
+
+// The v1 split kernels: any rows.  Where x and y rows share their 16-byte
+// phase (RowArgs::masked, the host's check) chunks of masked 16-byte vectors,
+// else of elements.
+template <int OP, typename T, int VEC, bool FINAL>
+__device__ __forceinline__ void rs_body(const RowArgs& a) {
+  __shared__ float scratch[RS_BLOCK / 64];
+  if constexpr (VEC == 1) {
+    if (a.masked) {
+      if constexpr (FINAL) rs_final_body<OP, T, Elem<T>::VEC, true>(a, scratch);
+      else rs_part_body<OP, T, Elem<T>::VEC, true>(a, scratch);
+      return;
+    }
+  }
+  if constexpr (FINAL) rs_final_body<OP, T, VEC>(a, scratch);
+  else rs_part_body<OP, T, VEC>(a, scratch);
 }
 
 }  // namespace g950
@@ -1003,11 +1220,11 @@ __device__ __forceinline__ void rs_final_body(const RowArgs& a) {
 #define G950_RS(OPNAME, OP, TNAME, T, VEC)                                                       \
   extern "C" __global__ __launch_bounds__(g950::RS_BLOCK) void                                      \
       g950_rs_part_##OPNAME##_##TNAME##_v##VEC(const g950::RowArgs a) {                             \
-    g950::rs_part_body<OP, T, VEC>(a);                                                              \
+    g950::rs_body<OP, T, VEC, false>(a);                                                              \
   }                                                                                                 \
   extern "C" __global__ __launch_bounds__(g950::RS_BLOCK) void                                      \
       g950_rs_final_##OPNAME##_##TNAME##_v##VEC(const g950::RowArgs a) {                            \
-    g950::rs_final_body<OP, T, VEC>(a);                                                             \
+    g950::rs_body<OP, T, VEC, true>(a);                                                             \
   }
 
 // register configurations: (VEC, ITEMS, BLOCK).  Vector forms need
@@ -1084,6 +1301,31 @@ G950_RM_ALL(logsumexp, g950::ROW_LOGSUMEXP)
 G950_RM_ALL(rmsnorm, g950::ROW_RMSNORM)
 G950_RM_ALL(layernorm, g950::ROW_LAYERNORM)
 G950_RM_ALL(lnrow, g950::ROW_LNROW)
+
+// One workgroup per long or odd row (rl_body): g950_rl_<op>_<dtype>_v1_
+// i<ITEMS>_b<BLOCK> (v1: rows of any length and phase).
+#define G950_RL(OPNAME, OP, TNAME, T, VEC, ITEMS, BLOCK, PACKED)                             \
+  extern "C" __global__ __launch_bounds__(BLOCK) void                                        \
+      g950_rl_##OPNAME##_##TNAME##_v1_i##ITEMS##_b##BLOCK(const g950::RowArgs a) {           \
+    g950::rl_body<OP, T, VEC, ITEMS, BLOCK, PACKED>(a);                                      \
+  }
+#define G950_RL_ALL(OPNAME, OP, ITEMS, BLOCK, PACKED)                   \
+  G950_RL(OPNAME, OP, f32, float, 4, ITEMS, BLOCK, PACKED)              \
+  G950_RL(OPNAME, OP, bf16, g950::bf16_t, 8, ITEMS, BLOCK, PACKED)      \
+  G950_RL(OPNAME, OP, f16, g950::f16_t, 8, ITEMS, BLOCK, PACKED)
+#define G950_RL_SHORT(OPNAME, OP, PACKED)  \
+  G950_RL_ALL(OPNAME, OP, 4, 256, PACKED)  \
+  G950_RL_ALL(OPNAME, OP, 8, 256, PACKED)
+G950_RL_SHORT(softmax, g950::ROW_SOFTMAX, true)
+G950_RL_SHORT(logsumexp, g950::ROW_LOGSUMEXP, true)
+G950_RL_SHORT(rmsnorm, g950::ROW_RMSNORM, false)
+G950_RL_SHORT(layernorm, g950::ROW_LAYERNORM, false)
+G950_RL_SHORT(lnrow, g950::ROW_LNROW, false)
+G950_RL_ALL(softmax, g950::ROW_SOFTMAX, 8, 1024, true)
+G950_RL_ALL(rmsnorm, g950::ROW_RMSNORM, 8, 1024, false)
+G950_RL_ALL(layernorm, g950::ROW_LAYERNORM, 8, 1024, false)
+G950_RL_ALL(lnrow, g950::ROW_LNROW, 8, 1024, false)
+G950_RL_ALL(softmax, g950::ROW_SOFTMAX, 16, 1024, true)
 
 // ------------------------------------------------------------- stream copy
 // y = x for n 16-byte vectors, grid-stride, nontemporal loads and stores --

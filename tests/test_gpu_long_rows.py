@@ -1,0 +1,110 @@
+"""GPU parity of the one-workgroup-per-row masked kernels (g950_rl_*) and of
+the masked chunks of the split kernels, for every row operator: row lengths
+one element around each form's capacity, every 16-byte phase of the row
+starts (odd row strides), gaps between rows untouched, special values in the
+edge vectors' neighbours; against the CPU oracle (fp32 1e-5, 16-bit 1e-2)."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+from compiler_amd import operators as ops  # noqa: E402
+from compiler_amd import runtime as rt  # noqa: E402
+from oracle import reference as ref  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+TD = {"float32": torch.float32, "bfloat16": torch.bfloat16, "float16": torch.float16}
+
+
+def case(rows, cols, stride, dt, seed):
+    """x as the cols first elements of rows `stride` apart, the gaps holding
+    the largest finite values (they must never reach a reduction)."""
+    rng = np.random.default_rng(seed)
+    big = {"float32": 3e38, "bfloat16": 3e38, "float16": 6e4}[dt]
+    full = torch.full((rows * stride + 16,), big, dtype=TD[dt], device=DEV)
+    x = torch.as_strided(full, (rows, cols), (stride, 1), 3)
+    x.copy_(torch.from_numpy((rng.standard_normal((rows, cols)) * 3).astype(np.float32)).to(DEV))
+    w = torch.from_numpy(rng.uniform(0.5, 1.5, cols + 1).astype(np.float32)).to(DEV).to(TD[dt])[1:]
+    b = torch.from_numpy((rng.standard_normal(cols + 1) * 0.1).astype(np.float32)).to(DEV).to(TD[dt])[1:]
+    return x, w, b
+
+
+def guarded(rows, cols, stride, dt):
+    full = torch.full((rows * stride + 16,), -7.0, dtype=TD[dt], device=DEV)
+    return full, torch.as_strided(full, (rows, cols), (stride, 1), 3)
+
+
+def host(t):
+    return t.float().cpu().numpy()
+
+
+SHAPES = {  # rows, cols, extra stride, kernel prefix
+    "float32": [(130, 2049, 1, "rl"), (140, 4089, 0, "rl"), (129, 4097, 3, "rl"), (128, 8191, 0, "rl"),
+                (131, 32761, 2, "rl"), (3, 20001, 1, "rs"), (2, 70001, 0, "rs")],
+    "bfloat16": [(5, 4097, 0, "rl"), (130, 8185, 1, "rl"), (128, 8193, 6, "rl"), (129, 16379, 0, "rl"),
+                 (128, 50001, 0, "rl"), (128, 65521, 3, "rl"), (3, 40001, 1, "rs"), (2, 140001, 0, "rs")],
+}
+SHAPES["float16"] = SHAPES["bfloat16"][1::2]
+
+
+@pytest.mark.parametrize("dt,shape", [(d, s) for d in SHAPES for s in SHAPES[d]])
+def test_long_odd_rows(dt, shape):
+    rows, cols, extra, kind = shape
+    stride = cols + extra
+    x, w, b = case(rows, cols, stride, dt, rows + cols)
+    xr, wr, br = host(x), host(w), host(b)
+    bar = (1e-5, 1e-6) if dt == "float32" else (1e-2, 1e-2)
+
+    def check(got, want, rtol, atol, kind=kind):
+        ok, err = ref.isclose_verdict(got, want, rtol, atol)
+        assert ok, (rt.module().last_kernel, err)
+        name = rt.module().last_kernel
+        assert name.startswith(f"g950_{kind}_") and "_v1" in name, name
+
+    full, y = guarded(rows, cols, stride, dt)
+    ops.softmax_kernel(x, y, cols, sync=True)
+    check(host(y), ref.softmax(xr), *bar)
+    lse = torch.empty(rows, device=DEV)
+    ops.logsumexp_kernel(x, lse, cols, sync=True)
+    # logsumexp splits rows that reach past 2048 vectors at some phase
+    v = 16 // x.element_size()
+    check(lse.cpu().numpy(), ref.logsumexp(xr), 3e-5, 3e-6, "rs" if (cols + 2 * (v - 1)) // v > 2048 else kind)
+    r = torch.empty(rows, device=DEV)
+    ops.rms_layernorm_forward_kernel(y, stride, x, stride, w, 1, r, 1, cols, 1e-6, sync=True)
+    ey, er = ref.rms_layernorm(xr, wr, 1e-6)
+    check(host(y), ey, *bar)
+    check(r.cpu().numpy(), er, 1e-5, 1e-6)
+    mean, rstd = torch.empty(rows, device=DEV), torch.empty(rows, device=DEV)
+    ops.layernorm_kernel(x, y, w, b, mean, rstd, stride, cols, 1e-5, sync=True)
+    ey, em, es = ref.layernorm(xr, wr, br, 1e-5)
+    check(host(y), ey, *(bar if dt != "float32" else (1e-5, 1e-5)))
+    check(mean.cpu().numpy(), em, 1e-5, 1e-6)
+    check(rstd.cpu().numpy(), es, 1e-5, 1e-6)
+    y.fill_(-7.0)
+    assert bool((full == -7.0).all())
+
+
+@pytest.mark.parametrize("rows,cols", [(130, 131065), (129, 65537), (128, 131072)])
+def test_long_rows_packed(rows, cols):
+    """softmax and logsumexp rows past the widened forms: bf16 up to 131072
+    elements in one workgroup, aligned ones too, and the special rows."""
+    x = (torch.randn(rows, cols, device=DEV) * 3).to(torch.bfloat16)
+    x[1, 5], x[2, cols - 1], x[3, :], x[4, 0] = float("inf"), float("nan"), float("-inf"), float("-inf")
+    xr = host(x)
+    y = ops.softmax(x, sync=True)
+    assert rt.module().last_kernel == "g950_rl_softmax_bf16_v1_i16_b1024"
+    got = host(y)
+    with np.errstate(invalid="ignore"):
+        want = ref.softmax(xr)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    keep = ~np.isnan(want)
+    ok, err = ref.isclose_verdict(got[keep], want[keep], 1e-2, 1e-2)
+    assert ok, err
+    assert abs(got[5].astype(np.float64).sum() - 1) < 1e-2
+    lse = ops.logsumexp(x, sync=True).cpu().numpy()
+    want = ref.logsumexp(xr)
+    assert np.array_equal(np.isnan(lse), np.isnan(want)) and np.isposinf(lse[1]) and np.isneginf(lse[3])
+    ok, err = ref.isclose_verdict(lse[5:], want[5:], 3e-5, 3e-6)
+    assert ok, err
