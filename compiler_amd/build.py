@@ -2,10 +2,11 @@
 
   compiler_amd/lib/g950.hsaco     every hot-path kernel (hipcc --genco, gfx950)
   compiler_amd/lib/libg950rt.so   the C-ABI module loader/launcher (include/g950rt.h)
+  compiler_amd/lib/g950_py.so     packing of a call's arguments for the Python side
   compiler_amd/lib/g950_exec      the bundle-driven command-line runner
 
 They are written next to the package so they travel with the source tree; the
-Python runtime loads exactly the first two.
+Python runtime loads exactly the first three.
 """
 from __future__ import annotations
 
@@ -20,6 +21,7 @@ CSRC = PKG / "csrc"
 LIB = PKG / "lib"
 HSACO = LIB / "g950.hsaco"
 RTLIB = LIB / "libg950rt.so"
+PYLIB = LIB / "g950_py.so"
 EXEC = LIB / "g950_exec"
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -58,6 +60,22 @@ def build_runtime() -> Path:
     return RTLIB
 
 
+def build_python() -> Path:
+    """g950_py.so: a CPython extension over torch's tensors (no HIP code)."""
+    import sysconfig
+
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    tmp = PYLIB.with_name(PYLIB.name + ".tmp")
+    _run(["g++", "-O2", "-std=c++17", "-Wall", "-fPIC", "-shared",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{ROOT / 'include'}",
+          f"-I{sysconfig.get_paths()['include']}", f"-I{root / 'include'}",
+          f"-I{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}", "-o", str(tmp), str(CSRC / "g950_py.cpp"),
+          f"-L{root / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10"])
+    os.replace(tmp, PYLIB)
+    return PYLIB
+
+
 def build_exec() -> Path:
     """g950_exec: the bundle-driven command-line runner (links libg950rt.so)."""
     tmp = EXEC.with_name(EXEC.name + ".tmp")
@@ -70,6 +88,7 @@ def build_exec() -> Path:
 def build_all() -> None:
     build_code_object()
     build_runtime()
+    build_python()
     build_exec()
 
 

@@ -20,13 +20,20 @@ import numpy as np
 from . import runtime as rt
 
 
+# sorted argument names of each call form: (op, views, scalars) names one form
+_ORDER: dict = {}
+
+
 def _launch(op, named_tensors: dict, outputs: set, named_scalars: dict, stream=None, sync=False,
             prepare=False):
-    names = sorted(named_tensors)
+    form = (op, len(named_tensors), len(named_scalars))
+    order = _ORDER.get(form)
+    if order is None:
+        names = sorted(named_tensors)
+        order = _ORDER[form] = (names, [n in outputs for n in names], sorted(named_scalars))
+    names, outs, scalar_names = order
     tensors = [named_tensors[n] for n in names]
-    outs = [n in outputs for n in names]
-    scalars = [named_scalars[n] if isinstance(named_scalars[n], rt.Scalar) else rt.scalar(named_scalars[n])
-               for n in sorted(named_scalars)]
+    scalars = [named_scalars[n] for n in scalar_names]
     if prepare:
         return rt.module().prepare(op, tensors, outs, scalars, stream=stream)
     return rt.module().launch(op, tensors, outs, scalars, stream=stream, sync=sync)
@@ -127,6 +134,7 @@ _VARLEN_SCALARS = ("q_row_stride", "k_row_stride", "v_row_stride", "q_head_strid
                    "block_size", "k_page_stride")
 # tile-shape constexprs of the reference kernel: accepted, no semantics here
 _VARLEN_TILE = ("BLOCK_M", "BLOCK_N", "BLOCK_K", "KERNEL_NUM_WARPS", "PIPELINE_STAGES", "d_rounded")
+_VARLEN_NAMES = frozenset(_VARLEN_VIEWS + _VARLEN_SCALARS + _VARLEN_TILE)
 
 
 def flash_varlen_fwd_kernel(*, stream=None, sync=False, prepare=False, **args):
@@ -135,7 +143,7 @@ def flash_varlen_fwd_kernel(*, stream=None, sync=False, prepare=False, **args):
     batches, seqused_k, GQA, causal and local windows, paged K/V.  Pointer
     arguments are device tensors (flattened to 1-D views); softcap, dropout,
     alibi, return_softmax and seqlenq_ngroups_swapped must be off."""
-    unknown = set(args) - set(_VARLEN_VIEWS) - set(_VARLEN_SCALARS) - set(_VARLEN_TILE)
+    unknown = args.keys() - _VARLEN_NAMES
     if unknown:
         raise TypeError(f"flash_varlen_fwd_kernel: unexpected arguments {sorted(unknown)}")
     missing = [n for n in _VARLEN_VIEWS + _VARLEN_SCALARS if n not in args]

@@ -16,6 +16,7 @@ import numpy as np
 PKG = Path(__file__).resolve().parent
 LIB_PATH = PKG / "lib" / "libg950rt.so"
 HSACO_PATH = PKG / "lib" / "g950.hsaco"
+PYLIB_PATH = PKG / "lib" / "g950_py.so"
 
 OK, USAGE, REJECTED, RESOURCE, REPEAT_MISMATCH, SYNC = 0, 2, 3, 4, 5, 6
 
@@ -183,6 +184,30 @@ def scalar(value, dtype: str | None = None) -> Scalar:
     return Scalar(codes[arr.dtype.name], arr.itemsize, bits)
 
 
+_packer = None
+
+
+def _load_packer():
+    """g950_py.so (native packing of a call's arguments); torch must be
+    importable.  No fallback: a missing library is an error."""
+    global _packer
+    with _lib_lock:
+        if _packer is None:
+            if not PYLIB_PATH.exists():
+                raise G950Error(RESOURCE, f"{PYLIB_PATH} is not built (run __graft_entry__.build())")
+            import importlib.machinery
+            import importlib.util
+
+            import torch  # noqa: F401  (the extension resolves against torch's libraries)
+            loader = importlib.machinery.ExtensionFileLoader("g950_py", str(PYLIB_PATH))
+            spec = importlib.util.spec_from_file_location("g950_py", str(PYLIB_PATH), loader=loader)
+            mod = importlib.util.module_from_spec(spec)
+            loader.exec_module(mod)
+            mod.init(Scalar, np.float32)
+            _packer = mod
+        return _packer
+
+
 class _ViewArray:
     """Keeps the ctypes shape/stride arrays alive for the duration of a call."""
 
@@ -227,24 +252,35 @@ class Module:
             raise G950Error(rc, lib.g950_last_error().decode())
         self._lib = lib
         self._handle = handle
+        self._pack_launch = _load_packer().launch
+        self._entries = tuple(ctypes.cast(f, ctypes.c_void_p).value
+                              for f in (lib.g950_launch, lib.g950_launch_noalloc))
         self.last_kernel = ""
 
     def launch(self, op: int, tensors, outputs, scalars, stream=None, sync=False):
         """Launch operator ``op``.  ``tensors``/``scalars`` are in sorted
-        argument-name order; ``outputs`` flags the output views."""
-        import torch
-        views = _ViewArray(tensors, outputs)
-        sc = (Scalar * max(len(scalars), 1))(*scalars)
+        argument-name order; ``outputs`` flags the output views; a scalar is a
+        packed ``Scalar`` or a value ``scalar()`` takes."""
         if stream is None:
-            stream = torch.cuda.current_stream(self.device)
-        handle = ctypes.c_void_p(stream.cuda_stream if hasattr(stream, "cuda_stream") else stream)
-        entry = self._lib.g950_launch_noalloc if noalloc_active() else self._lib.g950_launch
-        rc = entry(self._handle, op, views.views, len(tensors), sc, len(scalars), handle)
+            handle = _raw_stream(self.device)
+        else:
+            handle = stream.cuda_stream if hasattr(stream, "cuda_stream") else stream
+        noalloc = noalloc_active()
+        # native packing (g950_py.cpp); None: arguments it leaves to ctypes
+        rc = None
+        if type(handle) is int and self._handle:
+            rc = self._pack_launch(self._entries[noalloc], self._handle.value, op, tensors, outputs, scalars, handle)
+        if rc is None:
+            views = _ViewArray(tensors, outputs)
+            packed = [s if isinstance(s, Scalar) else scalar(s) for s in scalars]
+            sc = (Scalar * max(len(packed), 1))(*packed)
+            entry = self._lib.g950_launch_noalloc if noalloc else self._lib.g950_launch
+            rc = entry(self._handle, op, views.views, len(tensors), sc, len(packed), ctypes.c_void_p(handle))
         if rc != OK:
             raise G950Error(rc, self._lib.g950_last_error().decode())
         self.last_kernel = self._lib.g950_last_kernel().decode()
         if sync:
-            rc = self._lib.g950_sync(handle)
+            rc = self._lib.g950_sync(ctypes.c_void_p(handle))
             if rc != OK:
                 raise G950Error(rc, self._lib.g950_last_error().decode())
         return self.last_kernel
@@ -270,11 +306,24 @@ class Module:
 
 
 _modules: dict = {}
+_current_device = None  # torch.cuda.current_device once a module is loaded
+
+
+def _raw_stream(device: int) -> int:
+    """The handle of torch's current stream on ``device``."""
+    import torch
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def module() -> Module:
     """The process-wide module for the current device (loaded once)."""
+    global _current_device
+    if _current_device is not None:
+        mod = _modules.get(_current_device())
+        if mod is not None:
+            return mod
     import torch
+    _current_device = torch.cuda.current_device if torch.cuda.is_available() else None
     dev = torch.cuda.current_device() if torch.cuda.is_available() else -1
     mod = _modules.get(dev)
     if mod is None:
@@ -292,7 +341,8 @@ class Prepared:
         self._tensors = list(tensors)  # keep the storages alive
         self._views = _ViewArray(self._tensors, outputs)
         self._n = len(self._tensors)
-        self._scalars = (Scalar * max(len(scalars), 1))(*scalars)
+        self._scalars = (Scalar * max(len(scalars), 1))(
+            *[s if isinstance(s, Scalar) else scalar(s) for s in scalars])
         self._ns = len(scalars)
         self._op = op
         if stream is None:
