@@ -656,18 +656,23 @@ int gemm_tiles(GemmArgs& g, int bm = 256, int bn = 256) {
 // 2048x4096x4096 93 / 81 / 115 / 149; 2304x4096x4096 94 / 104 / 118 / 138;
 // int8 512x8192x8192 99 / 47 / 64 / 81.  fp32 is bound by its MFMAs, so its
 // slab times are nearly the tiles' areas: 512x4096x4096 896 / 252 / 140 / 148.
-int gemm_pick_tile(const g950_module* m, GemmArgs& g, int slabs, bool f32) {
+// int8 weights (slabs of 128 k): 256x4096x4096 - / 40 / 30 / 22, 512x4096x4096
+// - / 43 / 32 / 41, 1000x4096x4096 - / 44 / 59 / 78.
+enum TileClass { TILES_16 = 0, TILES_F32 = 1, TILES_W8 = 2 };
+
+int gemm_pick_tile(const g950_module* m, GemmArgs& g, int slabs, TileClass cls) {
   const long long cus = m ? m->cus : 256;
-  static const struct { int tile, bm, bn; double slab, f32_slab, fixed; } kTiles[] = {
-      {GEMM_TILE_256x256, 256, 256, 1.42, 7.0, 4.0},
-      {GEMM_TILE_128x128, 128, 128, 0.59, 1.95, 3.0},
-      {GEMM_TILE_64x128, 64, 128, 0.44, 1.06, 3.0},
-      {GEMM_TILE_64x64, 64, 64, 0.31, 0.58, 2.5}};
-  const auto* pick = &kTiles[0];
+  static const struct { int tile, bm, bn; double slab[3], fixed; } kTiles[] = {
+      {GEMM_TILE_256x256, 256, 256, {1.42, 7.0, 0.0}, 4.0},  // (no such tile for int8 weights)
+      {GEMM_TILE_128x128, 128, 128, {0.59, 1.95, 1.25}, 3.0},
+      {GEMM_TILE_64x128, 64, 128, {0.44, 1.06, 0.86}, 3.0},
+      {GEMM_TILE_64x64, 64, 64, {0.31, 0.58, 0.60}, 2.5}};
+  const auto* pick = &kTiles[1];
   double best = HUGE_VAL;
   for (const auto& t : kTiles) {
+    if (t.slab[cls] == 0.0) continue;
     const long long tiles = ((g.M + t.bm - 1ll) / t.bm) * ((g.N + t.bn - 1ll) / t.bn);
-    const double us = (double)((tiles + cus - 1) / cus) * (slabs * (f32 ? t.f32_slab : t.slab) + t.fixed);
+    const double us = (double)((tiles + cus - 1) / cus) * (slabs * t.slab[cls] + t.fixed);
     if (us < best) {
       best = us;
       pick = &t;
@@ -696,9 +701,13 @@ constexpr FewRowsForm kFewRows[2][3][4] = {
     // int8 weights
     {{{1, 8, 4}, {2, 8, 3}, {3, 8, 4}, {4, 4, 4}}, {{1, 4, 4}, {2, 4, 4}, {3, 4, 4}, {}}, {{1, 4, 4}, {2, 4, 4}, {}, {}}}};
 
+// `rows` rows at stride s0 (plus a row's part of a slab) within 32-bit offsets
+bool rows_off32(long long rows, long long s0, int esz) {
+  return (__int128)(rows - 1) * s0 * esz + 256 <= (__int128)0xFFFFFFFFll;
+}
+
 bool few_rows_ok(const GemmArgs& g, int a_esz, int b_esz) {
-  auto reach = [](long long rows, long long s0, int esz) { return (__int128)(rows - 1) * s0 * esz + 256 <= (__int128)0xFFFFFFFFll; };
-  return g.M <= 64 && reach(64, g.a_s0, a_esz) && reach(64, g.b_s0, b_esz);
+  return g.M <= 64 && rows_off32(64, g.a_s0, a_esz) && rows_off32(64, g.b_s0, b_esz);
 }
 
 int launch_few_rows(g950_module* m, const char* name, GemmArgs& g, bool w8, void* stream) {
@@ -793,7 +802,7 @@ int op_matmul(g950_module* m, const g950_view* views, uint32_t nviews, const g95
       return launch_few_rows(m, name, g, false, stream);
     }
     const bool kt = gemm_ktail((int)K, esz) || !gemm_off32(g, esz);
-    const int tiles = kt ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K * esz / 128), esz == 4);
+    const int tiles = kt ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K * esz / 128), esz == 4 ? TILES_F32 : TILES_16);
     if (tiles < 0) return fail(G950_USAGE, "matmul: too many tiles");
     snprintf(name, sizeof name, "g950_gemm_%s_256x256%s", rr_dtype(a.v->dtype), kt ? "_kt" : "");
     return launch(m, name, (unsigned)tiles, (unsigned)kernel_threads(m, name, 512), g, stream);
@@ -909,7 +918,7 @@ int op_matmul_i8(g950_module* m, const g950_view* views, uint32_t nviews, const 
     return launch_few_rows(m, name, g, false, stream);
   }
   if (gemm_fast_ok(a, b, (int)K, 1) && out_ok && (umask == 0 || !ktail)) {
-    const int tiles = ktail || umask ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K / 128), false);
+    const int tiles = ktail || umask ? gemm_tiles(g) : gemm_pick_tile(m, g, (int)(K / 128), TILES_16);
     if (tiles < 0) return fail(G950_USAGE, "matmul_i8: too many tiles");
     static const char* const names[4] = {"g950_gemm_i8_256x256", "g950_gemm_u8s8_256x256",
                                          "g950_gemm_s8u8_256x256", "g950_gemm_u8u8_256x256"};
@@ -1118,10 +1127,11 @@ int op_dequant_matmul(g950_module* m, const g950_view* views, uint32_t nviews, c
   }
   // Many output tiles: widen B once into an exact bf16 / f16 copy in the
   // workspace and run the 256x256 GEMM with the column scale in its epilogue.
-  // The fused kernel converts every B element once per 128-row output tile,
-  // which costs more than one copy (3 bytes per weight through HBM) once the
-  // 256x256 tiles outnumber half the CUs.  Measured on MI355X at N = K = 8192:
-  // M = 1024 (128 tiles) 186 us fused vs 148 + 36 us; M = 1536 334 vs 172 + 36.
+  // The fused kernel's tiles end at 128 x 128 and widen every weight once per
+  // row of tiles, so past half the CUs in 256x256 tiles one copy (3 bytes per
+  // weight through HBM) and the 256x256 kernel are ahead.  Measured on MI355X
+  // at N = K = 8192: M = 1024 (128 tiles) 153 us fused against 189 + 36 us;
+  // M = 1536 about 230 against 196 + 36.
   void* wide = nullptr;
   bool widened = fast && !transposed && K > 0 && K % 64 == 0 && 2 * ((M + 255) / 256) * ((N + 255) / 256) > cus &&
                  (unsigned long long)N * K * 2 <= (1ull << 31);
@@ -1153,14 +1163,14 @@ int op_dequant_matmul(g950_module* m, const g950_view* views, uint32_t nviews, c
       return launch(m, name, (unsigned)tiles, (unsigned)kernel_threads(m, name, 512), g, stream);
     }
   }
-  if (fast) {
+  if (fast && rows_off32(128, a.stride[0], 2) && rows_off32(128, bts, 1)) {
     g.a_s0 = a.stride[0];
     g.b_s0 = bts;  // Bt row (n) stride
-    g.tiles_m = (int)((M + 127) / 128);
-    g.tiles_n = (int)((N + 127) / 128);
-    const long long tiles = (long long)g.tiles_m * g.tiles_n;
-    if (tiles > 0x7FFFFFFF) return fail(G950_USAGE, "dequant_matmul: too many tiles");
-    return launch(m, bf16 ? "g950_gemm_w8a16_bf16_128x128" : "g950_gemm_w8a16_f16_128x128", (unsigned)tiles, 256u, g,
+    g.bscale = nullptr;
+    g.cscale = s.v->data; g.cscale_dtype = (int)s.v->dtype;
+    const int tiles = gemm_pick_tile(m, g, (int)((K + 127) / 128), TILES_W8);
+    if (tiles < 0) return fail(G950_USAGE, "dequant_matmul: too many tiles");
+    return launch(m, bf16 ? "g950_gemm_w8a16_bf16_128x128" : "g950_gemm_w8a16_f16_128x128", (unsigned)tiles, 512u, g,
                   stream);
   }
   g.a_s0 = a.stride[0]; g.a_s1 = a.stride[1];

@@ -709,6 +709,29 @@ __device__ __forceinline__ void gemm_mfma16_body(const GemmArgs& p, char* lds) {
                                               n_own);
 }
 
+// 16 int8 -> 16 exact 16-bit floats, as two 8-element operands (k 0..7, 8..15)
+template <bool F16>
+__device__ __forceinline__ void widen_i8x16(const u32x4& w, u32x4& lo, u32x4& hi) {
+  uint32_t o[8];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int x = (int)w[d];
+    const float f0 = (float)((x << 24) >> 24), f1 = (float)((x << 16) >> 24);
+    const float f2 = (float)((x << 8) >> 24), f3 = (float)(x >> 24);
+    if constexpr (F16) {
+      o[2 * d] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){f0, f1}, f16x2));
+      o[2 * d + 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){f2, f3}, f16x2));
+    } else {
+      o[2 * d] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){f0, f1}, bf16x2));
+      o[2 * d + 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){f2, f3}, bf16x2));
+    }
+  }
+  lo = (u32x4){o[0], o[1], o[2], o[3]};
+  hi = (u32x4){o[4], o[5], o[6], o[7]};
+}
+
+constexpr int W8_LDS = 144 * 1024;  // of the tiled int8-weight kernels
+
 // Smaller workgroup tiles of the whole-slab kernels (GemmArgs::tile), for
 // shapes whose 256 x 256 tiles would leave most CUs idle: TM x TN outputs,
 // 8 waves as 2 x 2 wave tiles x 2 halves of each K slab (a wave multiplies
@@ -727,12 +750,24 @@ __device__ __forceinline__ void gemm_mfma16_body(const GemmArgs& p, char* lds) {
 // of slab kt + 1 have landed.  After it nobody reads slab kt's stage again,
 // so slab kt + NST goes there.  The two k-halves of a wave tile are added
 // through LDS, each wave finishing half of the rows.
-template <int MODE, int TM, int TN, int UMASK, int NST>
+//
+// W8 (int8 weights under 16-bit A): a slab is 128 k -- 256 bytes of an A row,
+// 128 of a B row -- and a lane's 16 weights are widened as they leave LDS,
+// for two MFMAs; B then costs half the load path's bytes.  K need only be a
+// multiple of 16: the last slab's chunks past K repeat the row's last one and
+// are zeroed in registers.  The column scale is the epilogue's.  It is bound
+// by the load path like the others: 512 x 4096 x 4096 30 us, 256 x 4096 x
+// 4096 22 and 1024 x 8192 x 8192 153, against 102, 102 and 186 for the 128 x
+// 128 kernel it replaced (operands staged through registers, one slab ahead).
+template <int MODE, int TM, int TN, int UMASK, int NST, bool W8 = false>
 __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
-  constexpr int STAGE = (TM + TN) * SLAB;
-  constexpr int DPW = (TM + TN) / 64;              // DMA instructions (8 rows x 128 bytes) per wave per slab
+  constexpr int AROW = W8 ? 256 : SLAB;            // bytes of an A row per slab
+  constexpr int STAGE = TM * AROW + TN * SLAB;
+  constexpr int AG = TM * AROW / 1024;             // DMA instructions (1 KiB) of A per slab
+  constexpr int DPW = STAGE / 8192;                // DMA instructions per wave per slab
+  constexpr int AV = W8 ? 2 : 1;                   // A chunks of a lane per fragment
   constexpr int FM = TM / 32, FN = TN / 32;        // 16x16 fragments of a wave tile
-  static_assert(NST * STAGE <= 4 * BM * SLAB && NST >= 3, "the ring fits the kernel's LDS");
+  static_assert(NST * STAGE <= (W8 ? W8_LDS : 4 * BM * SLAB) && NST >= 3 && DPW * 8192 == STAGE, "LDS");
   static_assert(FM % 2 == 0 && 8 * (FM / 2) * FN * 1024 <= NST * STAGE, "the k-halves' exchange fits the ring");
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -740,43 +775,72 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
   int tm, tn;
   tile_of(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
   const int m0 = tm * TM, n0 = tn * TN;
-  constexpr int ES = (MODE == GEMM_I8) ? 1 : (MODE == GEMM_F32) ? 4 : 2;
-  const long long lda = p.a_s0 * ES, ldb = p.b_s0 * ES;
+  constexpr int ES = W8 ? 1 : (MODE == GEMM_I8) ? 1 : (MODE == GEMM_F32) ? 4 : 2;  // bytes of a B element
+  const long long lda = p.a_s0 * (W8 ? 2 : ES), ldb = p.b_s0 * ES;
   const char* abase = (const char*)p.a + (long long)m0 * lda;
   const char* bbase = (const char*)p.b + (long long)n0 * ldb;
-  const int kslabs = p.K * ES / SLAB;
+  const int kslabs = (p.K * ES + SLAB - 1) / SLAB;
+  const int tb = p.K * ES - (kslabs - 1) * SLAB;   // bytes of the last slab
   // group t of this wave: 8 rows of A or B (rows past the edge repeat the
   // last one; their outputs are not stored), the 16-byte chunks XOR-swizzled
   // by (row >> 1) & 7 as in the 256 x 256 kernels
   uint32_t doff[DPW];
   const uint32_t lds32 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)lds;
+  // this lane's 16-byte chunk of DMA instruction grp
+  auto chunk = [&](int grp) {
+    if (W8 && grp < AG) return (lane & 15) ^ ((grp * 4 + (lane >> 4)) & 15);
+    const int row = (grp < AG ? grp : grp - AG) * 8 + (lane >> 3);
+    return (lane & 7) ^ ((row >> 1) & 7);
+  };
 #pragma unroll
   for (int t = 0; t < DPW; ++t) {
     const int grp = wave * DPW + t;
-    const bool is_a = grp < TM / 8;
-    const int row = (is_a ? grp : grp - TM / 8) * 8 + (lane >> 3);
+    const bool is_a = grp < AG;
+    const int row = W8 && is_a ? grp * 4 + (lane >> 4) : (is_a ? grp : grp - AG) * 8 + (lane >> 3);
     const int src = min(row, (is_a ? p.M - m0 : p.N - n0) - 1);
-    doff[t] = (uint32_t)((long long)src * (is_a ? lda : ldb) + (((lane & 7) ^ ((row >> 1) & 7)) << 4));
+    doff[t] = (uint32_t)((long long)src * (is_a ? lda : ldb) + (chunk(grp) << 4));
   }
   auto issue = [&](int slab) {
     const uint32_t dst = lds32 + (uint32_t)(slab % NST) * STAGE;
+    const bool tail = W8 && slab == kslabs - 1 && tb != SLAB;
 #pragma unroll
     for (int t = 0; t < DPW; ++t) {
       const int grp = wave * DPW + t;
-      dma16_asm((grp < TM / 8 ? abase : bbase) + (long long)slab * SLAB, doff[t], dst + grp * 1024);
+      const bool is_a = grp < AG;
+      uint32_t off = doff[t];
+      if (tail) off -= max(0, (chunk(grp) << 4) + 16 - (is_a ? 2 * tb : tb));
+      dma16_asm((is_a ? abase : bbase) + (long long)slab * (is_a ? AROW : SLAB), off, dst + grp * 1024);
     }
   };
   const int l16 = lane & 15, g4 = lane >> 4;
-  const int sw = l16 * SLAB + (((kg * 4 + g4) ^ ((l16 >> 1) & 7)) << 4);
-  const int aoff = wm * (TM / 2) * SLAB + sw, boff = (TM + wn * (TN / 2)) * SLAB + sw;
-  u32x4 af[2][FM], bf[2][FN];
+  const int kc = kg * 4 + g4;  // this lane's 16-byte chunk of a B row's slab
+  const int sw = l16 * SLAB + ((kc ^ ((l16 >> 1) & 7)) << 4);
+  const int boff = TM * AROW + wn * (TN / 2) * SLAB + sw;
+  int aoff[AV];
+  if constexpr (W8) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) aoff[q] = (wm * (TM / 2) + l16) * AROW + (((2 * kc + q) ^ l16) << 4);
+  } else {
+    aoff[0] = wm * (TM / 2) * SLAB + sw;
+  }
+  u32x4 af[2][FM][AV], bf[2][FN];
   auto frags = [&](int slab, auto bc) {
     constexpr int B = decltype(bc)::value;
     const char* st = lds + (slab % NST) * STAGE;
 #pragma unroll
-    for (int i = 0; i < FM; ++i) af[B][i] = *(const u32x4*)(st + aoff + i * 16 * SLAB);
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int q = 0; q < AV; ++q) af[B][i][q] = *(const u32x4*)(st + aoff[q] + i * 16 * AROW);
 #pragma unroll
     for (int j = 0; j < FN; ++j) bf[B][j] = *(const u32x4*)(st + boff + j * 16 * SLAB);
+    if (W8 && slab == kslabs - 1 && kc * 16 >= tb) {  // chunks past K
+#pragma unroll
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int q = 0; q < AV; ++q) af[B][i][q] = (u32x4){0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int j = 0; j < FN; ++j) bf[B][j] = (u32x4){0u, 0u, 0u, 0u};
+    }
   };
   f32x4 acf[FM][FN];
   i32x4 aci[FM][FN];
@@ -791,18 +855,26 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
     constexpr int B = decltype(bc)::value;
     if constexpr (UMASK & 1) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i) af[B][i] ^= 0x80808080u;
+      for (int i = 0; i < FM; ++i) af[B][i][0] ^= 0x80808080u;
     }
     if constexpr (UMASK & 2) {
 #pragma unroll
       for (int j = 0; j < FN; ++j) bf[B][j] ^= 0x80808080u;
     }
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+    for (int j = 0; j < FN; ++j) {
+      if constexpr (W8) {
+        u32x4 lo, hi;
+        widen_i8x16<MODE == GEMM_F16>(bf[B][j], lo, hi);
 #pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        mfma16_step<MODE>(bf[B][j], af[B][i], acf[i][j], aci[i][j]);
+        for (int i = 0; i < FM; ++i) mfma16_step<MODE>(lo, af[B][i][0], acf[i][j], aci[i][j]);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) mfma16_step<MODE>(hi, af[B][i][1], acf[i][j], aci[i][j]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < FM; ++i) mfma16_step<MODE>(bf[B][j], af[B][i][0], acf[i][j], aci[i][j]);
       }
+    }
   };
   using B0 = std::integral_constant<int, 0>;
   using B1 = std::integral_constant<int, 1>;
@@ -1227,159 +1299,13 @@ __device__ __forceinline__ void i8_sums_body(const I8SumArgs& p) {
 // matmul.py:21-37).  int8 values are exact in bf16/fp16, so A.B accumulates
 // exactly as the unfused pair would from exact weights; the scale multiplies
 // the fp32 accumulator and the result rounds once at the store.
-//   * workgroup tile 128 x 128, 4 waves (2 x 2), wave tile 64 x 64 = 2 x 2
-//     fragments of v_mfma_f32_32x32x16; K in tiles of 64
-//   * register-staged: each thread loads its 4 A and 2 B 16-byte vectors of
-//     the next K tile while the current one is multiplied, widens the 32 int8
-//     weights to 16-bit once (per workgroup, not per wave), and writes both
-//     to the other LDS stage (128-byte rows, the main kernel's XOR swizzle, so
-//     fragment reads are the main kernel's); one barrier per K tile
-//   * B moves as int8: half the weight bytes of the unfused path, which
-//     matters where the product is bandwidth-bound (few rows of A)
-//   * K must be a multiple of 16 (whole 16-byte B vectors); a K tile past K
-//     is zero-filled; M/N edges clamp loads and mask stores
-template <bool F16>
-__device__ __forceinline__ void gemm_w8a16_body(const GemmArgs& p) {
-  constexpr int TM = 128, TN = 128, TK = 64;
-  constexpr int ROW = TK * 2;              // LDS row bytes (16-bit elements)
-  constexpr int STAGE = (TM + TN) * ROW;   // 32 KiB
-  __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
-  int tm, tn;
-  tile_of(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
-  const int m0 = tm * TM, n0 = tn * TN;
-  const long long lda = p.a_s0 * 2, ldb = p.b_s0;  // bytes
-  const int kend = p.K;
-  const int nk = (p.K + TK - 1) / TK;
-
-  // register staging: A vector i (of 4): row (tid + 256 i) >> 3, chunk & 7;
-  // B vector i (of 2): row (tid + 256 i) >> 2, 16-int8 part & 3
-  u32x4 ra[4], rb[2];
-  auto load = [&](int kt) {
-    const int k0 = kt * TK;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int v = tid + 256 * i, row = v >> 3, ch = v & 7;
-      const int k = k0 + ch * 8;
-      const char* src = (const char*)p.a + (long long)min(m0 + row, p.M - 1) * lda + (long long)k * 2;
-      ra[i] = k < kend ? *(const u32x4*)src : (u32x4){0u, 0u, 0u, 0u};
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int v = tid + 256 * i, row = v >> 2, part = v & 3;
-      const int k = k0 + part * 16;
-      const char* src = (const char*)p.b + (long long)min(n0 + row, p.N - 1) * ldb + k;
-      rb[i] = k < kend ? *(const u32x4*)src : (u32x4){0u, 0u, 0u, 0u};
-    }
-  };
-  auto store = [&](int stage) {
-    char* st = lds + stage * STAGE;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int v = tid + 256 * i, row = v >> 3, ch = v & 7;
-      *(u32x4*)(st + row * ROW + ((ch ^ ((row >> 1) & 7)) << 4)) = ra[i];
-    }
-    char* sb = st + TM * ROW;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int v = tid + 256 * i, row = v >> 2, part = v & 3;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {  // 8 int8 -> 8 16-bit values = one 16-byte chunk
-        u32x4 o;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t w = rb[i][2 * h + j / 2];
-          const int sh = (j & 1) * 16;
-          const float lo = (float)(int8_t)((w >> sh) & 0xFFu);
-          const float hi = (float)(int8_t)((w >> (sh + 8)) & 0xFFu);
-          o[j] = F16 ? (uint32_t)f32_to_f16(lo) | ((uint32_t)f32_to_f16(hi) << 16)
-                     : (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
-        }
-        const int ch = part * 2 + h;
-        *(u32x4*)(sb + row * ROW + ((ch ^ ((row >> 1) & 7)) << 4)) = o;
-      }
-    }
-  };
-
-  const int g = lane >> 5, r = lane & 31;
-  f32x16 acc[2][2];
-  i32x16 unused[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = (f32x16){};
-  if (nk > 0) {
-    load(0);
-    store(0);
-  }
-  __syncthreads();
-  int cur = 0;
-  for (int kt = 0; kt < nk; ++kt) {
-    if (kt + 1 < nk) load(kt + 1);
-    const char* st = lds + cur * STAGE;
-    const char* sb = st + TM * ROW;
-#pragma unroll
-    for (int ks = 0; ks < TK / 16; ++ks) {
-      const int chunk = ks * 2 + g;
-      u32x4 af[2], bf[2];
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi) {
-        const int row = wm * 64 + mi * 32 + r;
-        af[mi] = *(const u32x4*)(st + row * ROW + ((chunk ^ ((row >> 1) & 7)) << 4));
-      }
-#pragma unroll
-      for (int ni = 0; ni < 2; ++ni) {
-        const int row = wn * 64 + ni * 32 + r;
-        bf[ni] = *(const u32x4*)(sb + row * ROW + ((chunk ^ ((row >> 1) & 7)) << 4));
-      }
-#pragma unroll
-      for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
-          mfma_step<F16 ? GEMM_F16 : GEMM_BF16>(bf[ni], af[mi], acc[mi][ni], unused[mi][ni]);
-    }
-    if (kt + 1 < nk) store(cur ^ 1);
-    __syncthreads();
-    cur ^= 1;
-  }
-  const int wm0 = m0 + wm * 64, wn0 = n0 + wn * 64;
-  // scale the accumulator by its column's scale (lane layout of gemm_epilogue)
-#pragma unroll
-  for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int n = wn0 + ni * 32 + q * 8 + g * 4 + e;
-        const float sc = n < p.N ? load_as_f32(p.bscale, n, p.bscale_dtype) : 0.0f;
-#pragma unroll
-        for (int mi = 0; mi < 2; ++mi) acc[mi][ni][q * 4 + e] *= sc;
-      }
-  gemm_epilogue<F16 ? GEMM_F16 : GEMM_BF16, 2, 2>(p, acc, unused, wm0, wn0, lane);
-}
-
-// 16 int8 -> 16 exact 16-bit floats, as two 8-element operands (k 0..7, 8..15)
-template <bool F16>
-__device__ __forceinline__ void widen_i8x16(const u32x4& w, u32x4& lo, u32x4& hi) {
-  uint32_t o[8];
-#pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    const int x = (int)w[d];
-    const float f0 = (float)((x << 24) >> 24), f1 = (float)((x << 16) >> 24);
-    const float f2 = (float)((x << 8) >> 24), f3 = (float)(x >> 24);
-    if constexpr (F16) {
-      o[2 * d] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){f0, f1}, f16x2));
-      o[2 * d + 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){f2, f3}, f16x2));
-    } else {
-      o[2 * d] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){f0, f1}, bf16x2));
-      o[2 * d + 1] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){f2, f3}, bf16x2));
-    }
-  }
-  lo = (u32x4){o[0], o[1], o[2], o[3]};
-  hi = (u32x4){o[4], o[5], o[6], o[7]};
+template <int MODE>
+__device__ __forceinline__ void gemm_w8a16_tiles(const GemmArgs& p) {
+  __shared__ __attribute__((aligned(1024))) char lds[W8_LDS];
+  if (blockDim.x != 512) return;  // launch shape must match the kernel
+  if (p.tile == GEMM_TILE_128x128) gemm_tile_body<MODE, 128, 128, 0, 3, true>(p, lds);
+  else if (p.tile == GEMM_TILE_64x128) gemm_tile_body<MODE, 64, 128, 0, 4, true>(p, lds);
+  else gemm_tile_body<MODE, 64, 64, 0, 6, true>(p, lds);
 }
 
 // Exact copy of an int8 weight matrix Bt[N, K] (row stride b_s0 bytes, K a
@@ -1726,11 +1652,12 @@ G950_GEMM_MFMA(g950_gemm_u8u8_256x256, g950::GEMM_I8, 4, 2, 3, false)
 extern "C" __global__ __launch_bounds__(256) void g950_i8_sums(const g950::I8SumArgs p) {
   g950::i8_sums_body(p);
 }
-extern "C" __global__ __launch_bounds__(256) void g950_gemm_w8a16_bf16_128x128(const g950::GemmArgs p) {
-  g950::gemm_w8a16_body<false>(p);
+// (128x128: the largest of its tiles)
+extern "C" __global__ __launch_bounds__(512) void g950_gemm_w8a16_bf16_128x128(const g950::GemmArgs p) {
+  g950::gemm_w8a16_tiles<g950::GEMM_BF16>(p);
 }
-extern "C" __global__ __launch_bounds__(256) void g950_gemm_w8a16_f16_128x128(const g950::GemmArgs p) {
-  g950::gemm_w8a16_body<true>(p);
+extern "C" __global__ __launch_bounds__(512) void g950_gemm_w8a16_f16_128x128(const g950::GemmArgs p) {
+  g950::gemm_w8a16_tiles<g950::GEMM_F16>(p);
 }
 extern "C" __global__ __launch_bounds__(256) void g950_gemm_general(const g950::GemmArgs p) {
   g950::gemm_general_body<false>(p);

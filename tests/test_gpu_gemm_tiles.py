@@ -47,3 +47,23 @@ def test_gemm_tiles(m, n, k, dt):
     assert ok, err
     y.fill_(7.0)
     assert bool((full == 7.0).all())
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("m,n,k", [(65, 3, 128), (65, 129, 16), (100, 1000, 2064), (500, 2100, 112), (513, 1900, 704),
+                                   (1000, 2500, 144), (1023, 2401, 1280)])
+def test_w8a16_tiles(m, n, k, dt):
+    """int8 weights on the same tiles, slabs of 128 k with tails of every
+    multiple of 16, against float64 a . (b * scale) on the rounded inputs."""
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    a = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32) * 0.5).to(DEV).to(TD[dt])
+    bt = rng.integers(-127, 128, (n, k)).astype(np.int8)
+    s = torch.from_numpy((rng.random(n) / 64).astype(np.float32)).to(DEV).to(TD[dt])
+    full = torch.full((m + 2, n + 5), 7.0, dtype=TD[dt], device=DEV)
+    y = torch.as_strided(full, (m, n), (n + 5, 1), (n + 5) // 8 * 8)
+    ops.dequant_matmul_kernel(a, torch.from_numpy(bt).to(DEV).t(), s, y, m, n, k, sync=True)
+    expect = ref.matmul(a.float().cpu().numpy(), ref.dequantize(bt.T, s.float().cpu().numpy()))
+    ok, err = ref.isclose_verdict(y.float().cpu().numpy(), expect, 2e-2, 2e-2)
+    assert ok, err
+    y.fill_(7.0)
+    assert bool((full == 7.0).all())
