@@ -1431,14 +1431,15 @@ void* optional_workspace(g950_module* m, void* stream, size_t bytes) {
 // sequences of 2048 keys 93 / 99 / 107 / 112, 64 of 8000..400 226 / 205 /
 // 221 / 220, 32 of 4096..300 70 / 71 / 69 / 77; ranges from 128 keys up cost
 // one sequence of 8192 keys 29.5 us against 21.8 (256) and 19.8 (512), one
-// of 1024 keys runs 11.7 against 13.6 with 512.
-constexpr long long kDecTarget = 4, kDecMinKeys = 256;
+// of 1024 keys runs 11.7 against 13.6 with 512.  Up to 512 keys one range and
+// one launch: 40 sequences of 400 keys 21.3 -> 14.5, 2 of 500 11.4 -> 7.4.
+constexpr long long kDecTarget = 4, kDecMinKeys = 256, kDecOneRange = 512;
 
 int launch_attn_decode(g950_module* m, AttnDecArgs& a, uint32_t dt, long long D, bool paged, void* stream) {
   const long long pairs = (long long)a.a.Z * a.a.Hkv;
   const long long cus = m ? m->cus : 256;
   long long splits = std::min({(kDecTarget * cus + pairs - 1) / pairs, (long long)(a.a.Sk + kDecMinKeys - 1) / kDecMinKeys, 64ll});
-  splits = std::max(splits, 1ll);
+  splits = a.a.Sk <= kDecOneRange ? 1 : std::max(splits, 1ll);
   if (splits > 1 && m) {
     const long long recs = pairs * a.rows * splits;
     a.part = (float*)optional_workspace(m, stream, (size_t)recs * (size_t)(D + 2) * 4);
