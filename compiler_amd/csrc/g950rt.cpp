@@ -821,7 +821,8 @@ int op_matmul(g950_module* m, const g950_view* views, uint32_t nviews, const g95
       (__int128)(M - 1) * a.stride[0] * 2 + 128 <= (__int128)0xFFFFFFFFll) {
     g.a_s0 = a.stride[0];
     g.b_s0 = b.stride[0];  // k-row stride of B
-    const int tiles = gemm_tiles(g);
+    // (the smaller tiles' lanes span a slab's 64 k-rows of B by 32-bit offsets)
+    const int tiles = rows_off32(64, b.stride[0], 2) ? gemm_pick_tile(m, g, (int)(K / 64), TILES_16) : gemm_tiles(g);
     if (tiles < 0) return fail(G950_USAGE, "matmul: too many tiles");
     const char* name = a.v->dtype == G950_DTYPE_BFLOAT16 ? "g950_gemm_bf16_256x256_rb" : "g950_gemm_f16_256x256_rb";
     return launch(m, name, (unsigned)tiles, 512u, g, stream);
@@ -1086,7 +1087,7 @@ int op_dequant_matmul(g950_module* m, const g950_view* views, uint32_t nviews, c
     g.b_s0 = N;  // k-row stride of the copy
     g.bscale = nullptr;
     g.cscale = s.v->data; g.cscale_dtype = (int)s.v->dtype;
-    const int tiles = gemm_tiles(g);
+    const int tiles = rows_off32(64, N, 2) ? gemm_pick_tile(m, g, (int)(K / 64), TILES_16) : gemm_tiles(g);
     if (tiles < 0) return fail(G950_USAGE, "dequant_matmul: too many tiles");
     const char* name = bf16 ? "g950_gemm_bf16_256x256_rb" : "g950_gemm_f16_256x256_rb";
     return launch(m, name, (unsigned)tiles, 512u, g, stream);

@@ -759,7 +759,14 @@ constexpr int W8_LDS = 144 * 1024;  // of the tiled int8-weight kernels
 // by the load path like the others: 512 x 4096 x 4096 30 us, 256 x 4096 x
 // 4096 22 and 1024 x 8192 x 8192 153, against 102, 102 and 186 for the 128 x
 // 128 kernel it replaced (operands staged through registers, one slab ahead).
-template <int MODE, int TM, int TN, int UMASK, int NST, bool W8 = false>
+//
+// BROW (16-bit): row-major B read as it lies (gemm_mfma16_body's notes): a
+// slab is 64 k-rows of TN columns, in blocks of 64 columns x 128 bytes, and a
+// fragment comes out of two transposing reads; a tile at the right edge
+// computes the TN columns ending there and stores its own.  bf16 512 x 4096 x
+// 4096 97.6 -> 34 us, 300 x 2048 x 2048 41.8 -> 11.7, 1024 x 8192 x 8192 183 ->
+// 152, against the 256 x 256 form; 8192^3 as before.
+template <int MODE, int TM, int TN, int UMASK, int NST, bool W8 = false, bool BROW = false>
 __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
   constexpr int AROW = W8 ? 256 : SLAB;            // bytes of an A row per slab
   constexpr int STAGE = TM * AROW + TN * SLAB;
@@ -774,11 +781,12 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
   const int kg = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
   int tm, tn;
   tile_of(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
-  const int m0 = tm * TM, n0 = tn * TN;
+  const int m0 = tm * TM, n0 = BROW ? min(tn * TN, p.N - TN) : tn * TN;
   constexpr int ES = W8 ? 1 : (MODE == GEMM_I8) ? 1 : (MODE == GEMM_F32) ? 4 : 2;  // bytes of a B element
   const long long lda = p.a_s0 * (W8 ? 2 : ES), ldb = p.b_s0 * ES;
   const char* abase = (const char*)p.a + (long long)m0 * lda;
-  const char* bbase = (const char*)p.b + (long long)n0 * ldb;
+  const char* bbase = (const char*)p.b + (BROW ? (long long)n0 * ES : (long long)n0 * ldb);
+  const long long bstep = BROW ? 64 * ldb : SLAB;  // from slab to slab of B
   const int kslabs = (p.K * ES + SLAB - 1) / SLAB;
   const int tb = p.K * ES - (kslabs - 1) * SLAB;   // bytes of the last slab
   // group t of this wave: 8 rows of A or B (rows past the edge repeat the
@@ -789,6 +797,10 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
   // this lane's 16-byte chunk of DMA instruction grp
   auto chunk = [&](int grp) {
     if (W8 && grp < AG) return (lane & 15) ^ ((grp * 4 + (lane >> 4)) & 15);
+    if (BROW && grp >= AG) {  // k-row 8 (grp % 8) + lane / 8 of column block (grp - AG) / 8
+      const int k = ((grp - AG) & 7) * 8 + (lane >> 3);
+      return (lane & 7) ^ (2 * (((k >> 1) & 1) | (((k >> 3) & 1) << 1)));
+    }
     const int row = (grp < AG ? grp : grp - AG) * 8 + (lane >> 3);
     return (lane & 7) ^ ((row >> 1) & 7);
   };
@@ -797,6 +809,11 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
     const int grp = wave * DPW + t;
     const bool is_a = grp < AG;
     const int row = W8 && is_a ? grp * 4 + (lane >> 4) : (is_a ? grp : grp - AG) * 8 + (lane >> 3);
+    if (BROW && !is_a) {
+      doff[t] = (uint32_t)((long long)(((grp - AG) & 7) * 8 + (lane >> 3)) * ldb) + ((grp - AG) >> 3) * 128 +
+                (chunk(grp) << 4);
+      continue;
+    }
     const int src = min(row, (is_a ? p.M - m0 : p.N - n0) - 1);
     doff[t] = (uint32_t)((long long)src * (is_a ? lda : ldb) + (chunk(grp) << 4));
   }
@@ -809,7 +826,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
       const bool is_a = grp < AG;
       uint32_t off = doff[t];
       if (tail) off -= max(0, (chunk(grp) << 4) + 16 - (is_a ? 2 * tb : tb));
-      dma16_asm((is_a ? abase : bbase) + (long long)slab * (is_a ? AROW : SLAB), off, dst + grp * 1024);
+      dma16_asm((is_a ? abase : bbase) + (long long)slab * (is_a ? AROW : bstep), off, dst + grp * 1024);
     }
   };
   const int l16 = lane & 15, g4 = lane >> 4;
@@ -823,6 +840,18 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
   } else {
     aoff[0] = wm * (TM / 2) * SLAB + sw;
   }
+  // BROW: fragment j is column group cg = wn FN + j of the tile; lane (g4,
+  // 4 r + i) reads k-rows 32 kg + 8 g4 + r (and + 4), columns 4 i .. + 3
+  int btr[FN];
+  if constexpr (BROW) {
+    const int r = l16 >> 2;
+    const int bsw = ((r >> 1) & 1) | ((g4 & 1) << 1);
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int cg = wn * FN + j;
+      btr[j] = TM * AROW + (cg >> 2) * 64 * SLAB + (32 * kg + 8 * g4 + r) * SLAB + 32 * ((cg & 3) ^ bsw) + 8 * (l16 & 3);
+    }
+  }
   u32x4 af[2][FM][AV], bf[2][FN];
   auto frags = [&](int slab, auto bc) {
     constexpr int B = decltype(bc)::value;
@@ -832,7 +861,19 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
 #pragma unroll
       for (int q = 0; q < AV; ++q) af[B][i][q] = *(const u32x4*)(st + aoff[q] + i * 16 * AROW);
 #pragma unroll
-    for (int j = 0; j < FN; ++j) bf[B][j] = *(const u32x4*)(st + boff + j * 16 * SLAB);
+    for (int j = 0; j < FN; ++j) {
+      if constexpr (BROW) {
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(st + btr[j]));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(st + btr[j] + 4 * SLAB));
+        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+        bf[B][j] = (u32x4){l2[0], l2[1], h2[0], h2[1]};
+      } else {
+        bf[B][j] = *(const u32x4*)(st + boff + j * 16 * SLAB);
+      }
+    }
     if (W8 && slab == kslabs - 1 && kc * 16 >= tb) {  // chunks past K
 #pragma unroll
       for (int i = 0; i < FM; ++i)
@@ -938,7 +979,8 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
       if constexpr (MODE == GEMM_I8) hi[i][j] = (kg ? aci[i + HM][j] : aci[i][j]) + __builtin_bit_cast(i32x4, v);
       else hf[i][j] = (kg ? acf[i + HM][j] : acf[i][j]) + __builtin_bit_cast(f32x4, v);
     }
-  gemm_epilogue<MODE, HM, FN, UMASK, 16>(p, hf, hi, m0 + wm * (TM / 2) + kg * HM * 16, n0 + wn * (TN / 2), lane);
+  gemm_epilogue<MODE, HM, FN, UMASK, 16>(p, hf, hi, m0 + wm * (TM / 2) + kg * HM * 16, n0 + wn * (TN / 2), lane, 0,
+                                         tn * TN);
 }
 
 // WM x WN waves; wave tile (BM/WM) x (BN/WN) = FM x FN fragments of 32x32.
@@ -1598,7 +1640,14 @@ __device__ __forceinline__ void gemm_general_body(const GemmArgs& p) {
 #define G950_GEMM_MFMA_RB(NAME, MODE)                                                       \
   extern "C" __global__ __launch_bounds__(512) void NAME(const g950::GemmArgs p) {         \
     __shared__ __attribute__((aligned(1024))) char lds[4 * g950::BM * g950::SLAB];        \
-    g950::gemm_mfma16_body<MODE, 4, 2, 0, true>(p, lds);                                   \
+    if (p.tile == g950::GEMM_TILE_128x128)                                                 \
+      g950::gemm_tile_body<MODE, 128, 128, 0, 4, false, true>(p, lds);                     \
+    else if (p.tile == g950::GEMM_TILE_64x128)                                             \
+      g950::gemm_tile_body<MODE, 64, 128, 0, 5, false, true>(p, lds);                      \
+    else if (p.tile == g950::GEMM_TILE_64x64)                                              \
+      g950::gemm_tile_body<MODE, 64, 64, 0, 8, false, true>(p, lds);                       \
+    else                                                                                   \
+      g950::gemm_mfma16_body<MODE, 4, 2, 0, true>(p, lds);                                 \
   }
 G950_GEMM_MFMA_RB(g950_gemm_bf16_256x256_rb, g950::GEMM_BF16)
 G950_GEMM_MFMA_RB(g950_gemm_f16_256x256_rb, g950::GEMM_F16)

@@ -67,3 +67,30 @@ def test_w8a16_tiles(m, n, k, dt):
     assert ok, err
     y.fill_(7.0)
     assert bool((full == 7.0).all())
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("m,n,k", [(256, 256, 64), (257, 264, 576), (300, 1000, 448), (500, 2104, 128), (513, 1912, 704),
+                                   (1000, 2504, 128), (1023, 2408, 640)])
+def test_row_major_b_tiles(m, n, k, dt):
+    """Row-major B on the smaller tiles: right-edge windows, every fragment of
+    the transposing reads, and the column scale of row-major int8 weights."""
+    rng = np.random.default_rng(m + 3 * n + 7 * k)
+    a = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32) / np.float32(np.sqrt(k))).to(DEV).to(TD[dt])
+    b = torch.from_numpy(rng.standard_normal((k, n + 8)).astype(np.float32)).to(DEV).to(TD[dt])[:, :n]
+    full = torch.full((m + 2, n + 5), 7.0, dtype=TD[dt], device=DEV)
+    y = torch.as_strided(full, (m, n), (n + 5, 1), (n + 5) // 8 * 8)
+    ops.matmul_kernel(a, b, y, m, n, k, sync=True)
+    bar = {"bfloat16": (2e-2, 2e-2), "float16": (1e-2, 1e-2)}[dt]
+    ok, err = ref.isclose_verdict(y.float().cpu().numpy(), ref.matmul(a.float().cpu().numpy(), b.float().cpu().numpy()),
+                                  *bar)
+    assert ok, err
+    y.fill_(7.0)
+    assert bool((full == 7.0).all())
+    n -= n % 16
+    w = rng.integers(-127, 128, (k, n)).astype(np.int8)
+    s = torch.from_numpy((rng.random(n) / 64).astype(np.float32)).to(DEV).to(TD[dt])
+    got = ops.dequant_matmul(a, torch.from_numpy(w).to(DEV), s, sync=True)
+    expect = ref.matmul(a.float().cpu().numpy(), ref.dequantize(w, s.float().cpu().numpy()))
+    ok, err = ref.isclose_verdict(got.float().cpu().numpy(), expect, 2e-2, 2e-2)
+    assert ok, err
