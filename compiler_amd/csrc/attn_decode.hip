@@ -31,7 +31,6 @@ namespace g950 {
 constexpr int DEC_WAVES = 4;
 constexpr int DEC_TK = 16;          // keys per tile of one wave
 constexpr int DEC_RING = 16384;     // LDS bytes of one wave's ring
-constexpr int DEC_MAXSPLIT = 64;    // key ranges per (sequence, KV head)
 
 __device__ __forceinline__ f32x4 mfma16x16x16(const u32x2& a, const u32x2& b, const f32x4& c, std::true_type) {
   typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));

@@ -1439,7 +1439,8 @@ constexpr long long kDecTarget = 4, kDecMinKeys = 256, kDecOneRange = 512;
 int launch_attn_decode(g950_module* m, AttnDecArgs& a, uint32_t dt, long long D, bool paged, void* stream) {
   const long long pairs = (long long)a.a.Z * a.a.Hkv;
   const long long cus = m ? m->cus : 256;
-  long long splits = std::min({(kDecTarget * cus + pairs - 1) / pairs, (long long)(a.a.Sk + kDecMinKeys - 1) / kDecMinKeys, 64ll});
+  long long splits = std::min({(kDecTarget * cus + pairs - 1) / pairs, (long long)(a.a.Sk + kDecMinKeys - 1) / kDecMinKeys,
+                               64ll});  // the merge holds a pair's ranges in one wave's lanes
   splits = a.a.Sk <= kDecOneRange ? 1 : std::max(splits, 1ll);
   if (splits > 1 && m) {
     const long long recs = pairs * a.rows * splits;
