@@ -1033,13 +1033,15 @@ __device__ __forceinline__ void rs_part_body(const RowArgs& a, float* scratch) {
     p[1] = block_reduce<OpSum, RS_BLOCK>(q, scratch);
   } else {
     const int first = split * (RS_BLOCK * RS_ITEMS * VEC) - (MASKED ? x.ph : 0);
-    const float n = (float)(min(first + RS_BLOCK * RS_ITEMS * VEC, a.cols) - max(first, 0));
+    // (the host counts a masked row's vectors at its worst phase, so the last
+    // chunk may hold no element: weight 0 and, not 0 / 0, mean 0)
+    const float n = (float)max(min(first + RS_BLOCK * RS_ITEMS * VEC, a.cols) - max(first, 0), 0);
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < RS_ITEMS; ++i)
 #pragma unroll
       for (int e = 0; e < VEC; ++e) s += v[i][e];
-    const float mean = block_reduce<OpSum, RS_BLOCK>(s, scratch) / n;
+    const float mean = block_reduce<OpSum, RS_BLOCK>(s, scratch) / fmaxf(n, 1.0f);
     float q = 0.0f;
 #pragma unroll
     for (int i = 0; i < RS_ITEMS; ++i)

@@ -86,6 +86,35 @@ def test_long_odd_rows(dt, shape):
     assert bool((full == -7.0).all())
 
 
+# rows whose vectors fill their chunks exactly at some phases and reach one
+# vector further at others (chunks of 1024 vectors): the last chunk is empty
+# for part of the rows
+@pytest.mark.parametrize("dt,cols", [("bfloat16", 8186), ("bfloat16", 8190), ("bfloat16", 16383), ("float16", 8192),
+                                     ("float32", 4095), ("float32", 4094), ("float32", 12287)])
+def test_split_rows_last_chunk_empty(dt, cols):
+    rows, stride = 9, cols + 1
+    x, w, b = case(rows, cols, stride, dt, cols)
+    _, y = guarded(rows, cols, stride, dt)
+    xr, wr, br = host(x), host(w), host(b)
+    bar = (1e-5, 1e-6) if dt == "float32" else (1e-2, 1e-2)
+    mean, rstd = torch.empty(rows, device=DEV), torch.empty(rows, device=DEV)
+    ops.layernorm_kernel(x, y, w, b, mean, rstd, stride, cols, 1e-5, sync=True)
+    assert rt.module().last_kernel.startswith("g950_rs_final_layernorm") and "_v1" in rt.module().last_kernel
+    want = ref.layernorm(xr, wr, br, 1e-5)
+    ln_bar = bar if dt != "float32" else (1e-5, 1e-5)
+    for got, exp, (rtol, atol) in zip((host(y), mean.cpu().numpy(), rstd.cpu().numpy()), want,
+                                      (ln_bar, (1e-5, 1e-6), (1e-5, 1e-6))):
+        ok, err = ref.isclose_verdict(got, exp, rtol, atol)
+        assert ok, err
+    ops.softmax_kernel(x, y, cols, sync=True)
+    ok, err = ref.isclose_verdict(host(y), ref.softmax(xr), *bar)
+    assert ok, err
+    r = torch.empty(rows, device=DEV)
+    ops.rms_layernorm_forward_kernel(y, stride, x, stride, w, 1, r, 1, cols, 1e-6, sync=True)
+    ok, err = ref.isclose_verdict(host(y), ref.rms_layernorm(xr, wr, 1e-6)[0], *bar)
+    assert ok, err
+
+
 @pytest.mark.parametrize("rows,cols", [(130, 131065), (129, 65537), (128, 131072)])
 def test_long_rows_packed(rows, cols):
     """softmax and logsumexp rows past the widened forms: bf16 up to 131072
