@@ -90,7 +90,9 @@ __device__ __forceinline__ void attn_decode_body(const AttnDecArgs& g) {
   const long long kstride = 2 * p.k_ss, vstride = PG ? kstride : 2 * p.v_ss;
   char* ring = lds + wave * DEC_RING;  // this wave's
   const uint32_t ring32 = lds_addr(ring);
-  const int qpass = ROWS / G;  // queries per pass (the host: seqlen_q * group <= ROWS)
+  // queries per pass: seqlen_q (the host: seqlen_q * group <= ROWS), so a
+  // pass's rows are those a pair's partial records have room for
+  const int qpass = g.rows / G;
 
   // lane's share of a DMA instruction: key u * KPI + dkey, LDS chunk slot dpos
   const int dkey = lane / CH, dpos = lane % CH;

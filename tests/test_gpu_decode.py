@@ -72,6 +72,17 @@ def test_decode_attention_scores_climb():
     tv.check(dict(a, q_ptr=q.reshape(-1), k_ptr=k.reshape(-1)), meta, "bfloat16", "g950_attn_dec_")
 
 
+@pytest.mark.parametrize("seqlen_q,d", [(1, 128), (2, 64), (5, 128)])
+def test_decode_attention_longer_sequences_than_seqlen_q(seqlen_q, d):
+    """cu_seqlens_q lives on the device, so a sequence may hold more queries
+    than the scalar seqlen_q (1 and 2 queries: fewer rows than the kernel's
+    tile holds): every query is computed, and the partial records of the other
+    sequences and KV heads are left alone."""
+    a, meta = inputs.varlen_case(batches=3, max_q=12, max_k=2500, h=8, hk=2, d=d, causal=True, window_right=0)
+    tv.check(dict(a, seqlen_q=seqlen_q), meta, "bfloat16", "g950_attn_dec_")
+    assert rt.module().last_kernel.endswith("_merge")
+
+
 def test_decode_attention_without_workspace():
     """No-alloc calls and captured graphs keep to one key range per pair (no
     workspace) and give the same results within the bar; a graph replayed
