@@ -42,6 +42,9 @@ struct g950_module {
   // ordered, so each stream owns one buffer, grown on demand
   std::mutex ws_mu;
   std::unordered_map<void*, std::pair<void*, size_t>> ws;
+  // the same for optional_workspace(), which no captured graph uses: growing
+  // it leaves alone the address that a graph on this stream may hold of `ws`
+  std::unordered_map<void*, std::pair<void*, size_t>> ws_opt;
   // held by a call from its first use of the workspace until its last launch
   // is queued, so calls of several threads on one stream do not interleave
   // their launches on one buffer
@@ -283,7 +286,7 @@ const char* rr_dtype(uint32_t dt) {
 
 // Device workspace of at least `bytes` for launches on `stream`.  Growing it
 // waits for the stream (the old buffer may still be read by queued work).
-int workspace(g950_module* m, void* stream, size_t bytes, void** out) {
+int workspace(g950_module* m, void* stream, size_t bytes, void** out, bool optional = false) {
   if (t_scratch) {
     if (bytes > kScratchWorkspace)
       return fail(G950_USAGE, "no-alloc launch: the call needs %zu bytes of workspace, the scratch array holds %zu",
@@ -293,7 +296,7 @@ int workspace(g950_module* m, void* stream, size_t bytes, void** out) {
   }
   if (!t_ws_use.owns_lock()) t_ws_use = std::unique_lock<std::mutex>(m->ws_use);
   std::lock_guard<std::mutex> lock(m->ws_mu);
-  auto& w = m->ws[stream];
+  auto& w = (optional ? m->ws_opt : m->ws)[stream];
   if (w.second < bytes) {
     if (w.first) {
       if (hipError_t e = hipStreamSynchronize((hipStream_t)stream))
@@ -1416,7 +1419,7 @@ void* optional_workspace(g950_module* m, void* stream, size_t bytes) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   void* ws = nullptr;
   if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone ||
-      workspace(m, stream, bytes, &ws) != G950_OK) {
+      workspace(m, stream, bytes, &ws, true) != G950_OK) {
     (void)hipGetLastError();
     ws = nullptr;
   }
@@ -1737,8 +1740,10 @@ const char* g950_last_kernel(void) { return t_kernel.c_str(); }
 size_t g950_workspace_bytes(g950_module* m, void* stream) {
   if (!m) return 0;
   std::lock_guard<std::mutex> lock(m->ws_mu);
-  const auto it = m->ws.find(stream);
-  return it == m->ws.end() ? 0 : it->second.second;
+  size_t n = 0;
+  for (const auto* ws : {&m->ws, &m->ws_opt})
+    if (const auto it = ws->find(stream); it != ws->end()) n += it->second.second;
+  return n;
 }
 
 int g950_sync(void* stream) {
@@ -1763,11 +1768,12 @@ const char* g950_last_error(void) { return t_error.c_str(); }
 
 void g950_close(g950_module* m) {
   if (!m) return;
-  for (auto& kv : m->ws)
-    if (kv.second.first) {
-      (void)hipStreamSynchronize((hipStream_t)kv.first);
-      (void)hipFree(kv.second.first);
-    }
+  for (auto* ws : {&m->ws, &m->ws_opt})
+    for (auto& kv : *ws)
+      if (kv.second.first) {
+        (void)hipStreamSynchronize((hipStream_t)kv.first);
+        (void)hipFree(kv.second.first);
+      }
   if (m->mod) (void)hipModuleUnload(m->mod);
   delete m;
 }

@@ -113,3 +113,39 @@ def test_decode_attention_without_workspace():
         assert torch.equal(t["o_ptr"], one)
         ops.flash_varlen_fwd_kernel(**t, **scal, sync=True)
         assert torch.equal(t["o_ptr"], split)
+
+
+def test_decode_attention_leaves_captured_workspace_alone():
+    """A graph may hold the address of its stream's workspace (split softmax
+    rows): a decoding step's key ranges on that stream, which need more, leave
+    it as it is."""
+    stream = torch.cuda.Stream()
+    a, meta = inputs.varlen_case(batches=4, max_q=1, max_k=4000, h=32, hk=8, d=128, var_q=False, var_k=False)
+    t = {n: torch.from_numpy(np.ascontiguousarray(a[n]).view(np.int64) if a[n].dtype == np.uint64
+                             else np.ascontiguousarray(a[n])).to("cuda") for n in ops._VARLEN_VIEWS}
+    for n in ("q_ptr", "k_ptr", "v_ptr", "o_ptr"):
+        t[n] = t[n].to(torch.bfloat16)
+    scal = {n: {**a, **meta}[n] for n in ops._VARLEN_SCALARS}
+    x = torch.randn(2, 60000, device="cuda")
+    y = torch.zeros_like(x)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        ops.softmax_kernel(x, y, 60000, sync=True)
+        assert rt.module().last_kernel.startswith("g950_rs_final_softmax")
+        want = y.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        ops.softmax_kernel(x, y, 60000)
+    held = rt.module().workspace_bytes(stream)
+    with torch.cuda.stream(stream):
+        ops.flash_varlen_fwd_kernel(**t, **scal, sync=True)
+        assert rt.module().last_kernel.endswith("_merge")
+    # the key ranges came on top of what the softmax call holds
+    recs = 4 * 32 * 16
+    assert rt.module().workspace_bytes(stream) >= held + recs * (128 + 2) * 4
+    for _ in range(3):
+        y.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
