@@ -11,7 +11,11 @@
 //     heads sharing the KV head are the columns of one MFMA tile, so K and V
 //     leave HBM once.  The host cuts the keys into `splits` ranges when the
 //     (sequence, KV head) pairs alone would not fill the chip or would leave
-//     it waiting for the longest sequence; attn_decode_merge joins them;
+//     it waiting for the longest sequence; attn_decode_merge joins them.
+//     Without a workspace for their records (captured graphs, no-alloc
+//     calls) one workgroup takes a pair's ranges in turn and joins them in
+//     registers by the same operations in the same order (DecRow), so both
+//     forms of a call give the same bits;
 //   * its 4 waves take 16-key tiles in turn and share nothing until the end:
 //     each has its own LDS ring filled by direct global->LDS DMA and waits
 //     for its own loads only, so there is no barrier in the loop.  64 KiB of
@@ -57,9 +61,30 @@ __device__ __forceinline__ float row4(float v) {
   return Op::apply(v, __shfl_xor(v, 32));
 }
 
+// A query row's key ranges joined one after the other: maximum (log2 units)
+// and sum so far.  join() takes the next range's and gives the weights of
+// what was gathered before (was) and of the range's own O (now); a range in
+// which the row saw no key has weight 0 and is to be left out (its O may hold
+// anything).  Both users apply them as fmaf(now, range, was * gathered).
+struct DecRow {
+  float m = -__builtin_huge_valf(), l = 0.0f;
+  __device__ __forceinline__ bool join(float mr, float lr, float& was, float& now) {
+    if (mr == -__builtin_huge_valf() && lr == 0.0f) return false;
+    const float to = fmaxf(m, mr);
+    // no finite score yet on a side: its sum is 0, or NaN and kept
+    was = m == -__builtin_huge_valf() ? 1.0f : __builtin_amdgcn_exp2f(m - to);
+    now = mr == -__builtin_huge_valf() ? 1.0f : __builtin_amdgcn_exp2f(mr - to);
+    l = fmaf(now, lr, was * l);
+    m = to;
+    return true;
+  }
+};
+
 // RT: 16-row query tiles per workgroup (1 or 2).  PG: 0 contiguous K/V rows,
-// 1 pages of a multiple of 16 keys (a tile lies in one page).
-template <int D, bool F16, int RT, int PG>
+// 1 pages of a multiple of 16 keys (a tile lies in one page).  PART: this
+// workgroup takes one of a pair's ranges and leaves its record, else all of
+// them.
+template <int D, bool F16, int RT, int PG, bool PART>
 __device__ __forceinline__ void attn_decode_body(const AttnDecArgs& g) {
   constexpr int ROW = D * 2, CH = ROW / 16;      // row bytes, 16-byte chunks per row
   constexpr int KT = DEC_TK * ROW;               // K (or V) bytes of one tile
@@ -78,7 +103,7 @@ __device__ __forceinline__ void attn_decode_body(const AttnDecArgs& g) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g4 = lane >> 4, l16 = lane & 15;
   const int pairs = p.Z * p.Hkv;
-  const int split = blockIdx.x / pairs, pair = blockIdx.x % pairs;
+  const int split = PART ? blockIdx.x / pairs : 0, pair = blockIdx.x % pairs;
   const int z = pair / p.Hkv, hk = pair % p.Hkv;
   const int G = p.group;
   const SeqGeom sg = varlen_geom(p, vl, z);
@@ -107,20 +132,15 @@ __device__ __forceinline__ void attn_decode_body(const AttnDecArgs& g) {
   const int voff = KT + vkey * ROW + (vswz(vkey) << 5) + (l16 & 3) * 8;
 
   // A sequence holding more queries than seqlen_q (outside the contract, but
-  // in reach of a device-held length) is finished by its first range alone.
+  // in reach of a device-held length): the further passes run over all keys
+  // in one range, by the workgroup of the first.
   for (int q0 = 0; q0 < Sq && q0 < 256; q0 += qpass) {
-    const bool whole = q0 > 0 || g.splits == 1;
-    if (q0 > 0 && split != 0) break;
+    const bool ranged = q0 == 0 && g.splits > 1;
+    if (PART && !ranged && split != 0) break;
     const int qn = min(qpass, Sq - q0);  // queries of this pass
     int kend = Sk;
     if (has_hi) kend = min(kend, q0 + qn - 1 + hi_off + 1);
-    int lo = has_lo ? max(0, q0 + lo_off) / DEC_TK * DEC_TK : 0, hi = kend;
-    if (!whole) {
-      lo = max(lo, split * g.chunk);
-      if (split + 1 < g.splits) hi = min(hi, (split + 1) * g.chunk);
-    }
-    const int ntiles = hi > lo ? (hi - lo + DEC_TK - 1) / DEC_TK : 0;
-    const int nloc = ntiles > wave ? (ntiles - wave + DEC_WAVES - 1) / DEC_WAVES : 0;
+    const int kbeg = has_lo ? max(0, q0 + lo_off) / DEC_TK * DEC_TK : 0;
 
     // query fragments (B port): row rt*16 + l16 = query qi of head hk*G + hg
     u32x4 qf[RT][DS];
@@ -136,153 +156,182 @@ __device__ __forceinline__ void attn_decode_body(const AttnDecArgs& g) {
       for (int ks = 0; ks < DS; ++ks) qf[rt][ks] = *(const u32x4*)(src + (ks * 32 + g4 * 8) * 2);
     }
 
-    // page numbers of this wave's next 64 tiles, one per lane
-    int pages = 0;
-    auto issue = [&](int j) {
-      const int kv0 = lo + DEC_TK * (wave + DEC_WAVES * j);
-      long long row0 = 0;  // byte offset of the tile's first key row
-      if constexpr (PG == 1) {
-        if ((j & 63) == 0) {
-          const int key = kv0 + DEC_TK * DEC_WAVES * lane;
-          const long long e = (long long)z * vl.pt_stride + key / vl.block_size;
-          int ph = key < hi && e < vl.pt_elems ? vl.page_table[e] : 0;
-          pages = ph < 0 || ph >= vl.pages ? 0 : ph;
-        }
-        const int ph = __builtin_amdgcn_readlane(pages, j & 63);
-        row0 = 2 * (long long)ph * vl.page_stride + (long long)(kv0 % vl.block_size) * kstride;
-      }
-      const char* ks0 = uniform_ptr(kbase + (PG ? row0 : (long long)kv0 * kstride));
-      const char* vs0 = uniform_ptr(vbase + (PG ? row0 : (long long)kv0 * vstride));
-      const uint32_t dst = ring32 + (j % ST) * 2 * KT;
-      const int last = Sk - 1 - kv0;  // keys past the end repeat the last one
-#pragma unroll
-      for (int u = 0; u < DPT / 2; ++u) {
-        const int key = u * KPI + dkey;
-        dma16_asm(ks0, (uint32_t)(min(key, last) * (int)kstride) + ((dpos ^ kswz(key)) << 4), dst + u * 1024);
-      }
-#pragma unroll
-      for (int u = 0; u < DPT / 2; ++u) {
-        const int key = u * KPI + dkey;
-        dma16_asm(vs0, (uint32_t)(min(key, last) * (int)vstride) + ((dpos ^ (vswz(key) << 1)) << 4),
-                  dst + KT + u * 1024);
-      }
-    };
+    // keys lo .. hi - 1 (of the pass's window) into the waves' partial rows
+    auto attend = [&](int lo, int hi) {
+      const int ntiles = hi > lo ? (hi - lo + DEC_TK - 1) / DEC_TK : 0;
+      const int nloc = ntiles > wave ? (ntiles - wave + DEC_WAVES - 1) / DEC_WAVES : 0;
 
-    f32x4 o[RT][DB];
-    float ms[RT], l[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      ms[rt] = -__builtin_huge_valf();
-      l[rt] = 0.0f;
-#pragma unroll
-      for (int b = 0; b < DB; ++b) o[rt][b] = (f32x4){};
-    }
-    const float c2 = p.scale_log2;
-    for (int j = 0; j < ST && j < nloc; ++j) issue(j);
-    for (int i = 0; i < nloc; ++i) {
-      // tile i has landed once at most the later tiles' loads are in flight
-      if (i + ST <= nloc) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((ST - 1) * DPT) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      const char* st = ring + (i % ST) * 2 * KT;
-      const int kv0 = lo + DEC_TK * (wave + DEC_WAVES * i);
-      f32x4 s[RT];
-      i32x4 unused;
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) s[rt] = (f32x4){};
-#pragma unroll
-      for (int ks = 0; ks < DS; ++ks) {
-        const u32x4 kf = *(const u32x4*)(st + koff[ks]);
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) mfma16_step<F16 ? GEMM_F16 : GEMM_BF16>(kf, qf[rt][ks], s[rt], unused);
-      }
-      // keys kv0 + 4 g4 .. + 3 of query row l16
-      const bool mask = kv0 + DEC_TK > Sk || (has_hi && kv0 + DEC_TK - 1 > q0 + hi_off) ||
-                        (has_lo && kv0 < q0 + qn - 1 + lo_off);
-      if (mask) {
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int key = kv0 + 4 * g4 + e;
-            if (key >= Sk || (has_hi && key > qi[rt] + hi_off) || (has_lo && key < qi[rt] + lo_off))
-              s[rt][e] = -__builtin_huge_valf();
+      // page numbers of this wave's next 64 tiles, one per lane
+      int pages = 0;
+      auto issue = [&](int j) {
+        const int kv0 = lo + DEC_TK * (wave + DEC_WAVES * j);
+        long long row0 = 0;  // byte offset of the tile's first key row
+        if constexpr (PG == 1) {
+          if ((j & 63) == 0) {
+            const int key = kv0 + DEC_TK * DEC_WAVES * lane;
+            const long long e = (long long)z * vl.pt_stride + key / vl.block_size;
+            int ph = key < hi && e < vl.pt_elems ? vl.page_table[e] : 0;
+            pages = ph < 0 || ph >= vl.pages ? 0 : ph;
           }
-      }
-      u32x2 pf[RT];
+          const int ph = __builtin_amdgcn_readlane(pages, j & 63);
+          row0 = 2 * (long long)ph * vl.page_stride + (long long)(kv0 % vl.block_size) * kstride;
+        }
+        const char* ks0 = uniform_ptr(kbase + (PG ? row0 : (long long)kv0 * kstride));
+        const char* vs0 = uniform_ptr(vbase + (PG ? row0 : (long long)kv0 * vstride));
+        const uint32_t dst = ring32 + (j % ST) * 2 * KT;
+        const int last = Sk - 1 - kv0;  // keys past the end repeat the last one
+#pragma unroll
+        for (int u = 0; u < DPT / 2; ++u) {
+          const int key = u * KPI + dkey;
+          dma16_asm(ks0, (uint32_t)(min(key, last) * (int)kstride) + ((dpos ^ kswz(key)) << 4), dst + u * 1024);
+        }
+#pragma unroll
+        for (int u = 0; u < DPT / 2; ++u) {
+          const int key = u * KPI + dkey;
+          dma16_asm(vs0, (uint32_t)(min(key, last) * (int)vstride) + ((dpos ^ (vswz(key) << 1)) << 4),
+                    dst + KT + u * 1024);
+        }
+      };
+
+      f32x4 o[RT][DB];
+      float ms[RT], l[RT];
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
-        const float mh = vmax3(vmax3(s[rt][0], s[rt][1], s[rt][2]), s[rt][3], s[rt][3]) * c2;
-        if (__any(mh > ms[rt] + 8.0f)) {
-          const float mt = row4<OpMax>(mh);
-          const bool move = mt > ms[rt] + 8.0f;
-          const float alpha = move ? __builtin_amdgcn_exp2f(ms[rt] - mt) : 1.0f;
-          l[rt] *= alpha;
+        ms[rt] = -__builtin_huge_valf();
+        l[rt] = 0.0f;
 #pragma unroll
-          for (int b = 0; b < DB; ++b) o[rt][b] *= alpha;
-          ms[rt] = move ? mt : ms[rt];
+        for (int b = 0; b < DB; ++b) o[rt][b] = (f32x4){};
+      }
+      const float c2 = p.scale_log2;
+      for (int j = 0; j < ST && j < nloc; ++j) issue(j);
+      for (int i = 0; i < nloc; ++i) {
+        // tile i has landed once at most the later tiles' loads are in flight
+        if (i + ST <= nloc) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((ST - 1) * DPT) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const char* st = ring + (i % ST) * 2 * KT;
+        const int kv0 = lo + DEC_TK * (wave + DEC_WAVES * i);
+        f32x4 s[RT];
+        i32x4 unused;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) s[rt] = (f32x4){};
+#pragma unroll
+        for (int ks = 0; ks < DS; ++ks) {
+          const u32x4 kf = *(const u32x4*)(st + koff[ks]);
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) mfma16_step<F16 ? GEMM_F16 : GEMM_BF16>(kf, qf[rt][ks], s[rt], unused);
         }
-        // rows without a visible key so far: exponent base 0, exp2(-inf) = 0
-        const float mb = (ms[rt] == -__builtin_huge_valf()) ? 0.0f : ms[rt];
-        float pe[4];
+        // keys kv0 + 4 g4 .. + 3 of query row l16
+        const bool mask = kv0 + DEC_TK > Sk || (has_hi && kv0 + DEC_TK - 1 > q0 + hi_off) ||
+                          (has_lo && kv0 < q0 + qn - 1 + lo_off);
+        if (mask) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) pe[e] = __builtin_amdgcn_exp2f(fmaf(s[rt][e], c2, -mb));
-        l[rt] += (pe[0] + pe[1]) + (pe[2] + pe[3]);
-        pf[rt] = (u32x2){pack2(pe[0], pe[1], F16), pack2(pe[2], pe[3], F16)};
+          for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int key = kv0 + 4 * g4 + e;
+              if (key >= Sk || (has_hi && key > qi[rt] + hi_off) || (has_lo && key < qi[rt] + lo_off))
+                s[rt][e] = -__builtin_huge_valf();
+            }
+        }
+        u32x2 pf[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          const float mh = vmax3(vmax3(s[rt][0], s[rt][1], s[rt][2]), s[rt][3], s[rt][3]) * c2;
+          if (__any(mh > ms[rt] + 8.0f)) {
+            const float mt = row4<OpMax>(mh);
+            const bool move = mt > ms[rt] + 8.0f;
+            const float alpha = move ? __builtin_amdgcn_exp2f(ms[rt] - mt) : 1.0f;
+            l[rt] *= alpha;
+#pragma unroll
+            for (int b = 0; b < DB; ++b) o[rt][b] *= alpha;
+            ms[rt] = move ? mt : ms[rt];
+          }
+          // rows without a visible key so far: exponent base 0, exp2(-inf) = 0
+          const float mb = (ms[rt] == -__builtin_huge_valf()) ? 0.0f : ms[rt];
+          float pe[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) pe[e] = __builtin_amdgcn_exp2f(fmaf(s[rt][e], c2, -mb));
+          l[rt] += (pe[0] + pe[1]) + (pe[2] + pe[3]);
+          pf[rt] = (u32x2){pack2(pe[0], pe[1], F16), pack2(pe[2], pe[3], F16)};
+        }
+#pragma unroll
+        for (int b = 0; b < DB; ++b) {
+          typedef short s16x4 __attribute__((ext_vector_type(4)));
+          const s16x4 vf = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (__attribute__((address_space(3))) s16x4*)(st + (voff ^ (b << 5))));
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt)
+            o[rt][b] = mfma16x16x16(__builtin_bit_cast(u32x2, vf), pf[rt], o[rt][b], std::bool_constant<F16>{});
+        }
+        // this tile's LDS reads have returned before its slot is refilled
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (i + ST < nloc) issue(i + ST);
       }
-#pragma unroll
-      for (int b = 0; b < DB; ++b) {
-        typedef short s16x4 __attribute__((ext_vector_type(4)));
-        const s16x4 vf = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4*)(st + (voff ^ (b << 5))));
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-          o[rt][b] = mfma16x16x16(__builtin_bit_cast(u32x2, vf), pf[rt], o[rt][b], std::bool_constant<F16>{});
-      }
-      // this tile's LDS reads have returned before its slot is refilled
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (i + ST < nloc) issue(i + ST);
-    }
 
-    // ---- the four waves' partial rows: O through each wave's own ring
-    // (16-byte chunks XOR-swizzled by the row), maxima and sums beside it
+      // ---- the four waves' partial rows: O through each wave's own ring
+      // (16-byte chunks XOR-swizzled by the row), maxima and sums beside it
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const int r = rt * 16 + l16;
-      const float ls = row4<OpSum>(l[rt]);
+      for (int rt = 0; rt < RT; ++rt) {
+        const int r = rt * 16 + l16;
+        const float ls = row4<OpSum>(l[rt]);
 #pragma unroll
-      for (int b = 0; b < DB; ++b) *(f32x4*)(ring + r * D * 4 + (((4 * b + g4) ^ l16) << 4)) = o[rt][b];
-      if (g4 == 0) {
-        ml[wave][r][0] = ms[rt];
-        ml[wave][r][1] = ls;
+        for (int b = 0; b < DB; ++b) *(f32x4*)(ring + r * D * 4 + (((4 * b + g4) ^ l16) << 4)) = o[rt][b];
+        if (g4 == 0) {
+          ml[wave][r][0] = ms[rt];
+          ml[wave][r][1] = ls;
+        }
       }
-    }
-    __syncthreads();
-    constexpr int CPR = D / 4;  // 16-byte chunks (4 d) per row
-    for (int it = tid; it < qn * G * CPR; it += DEC_WAVES * 64) {
-      const int r = it / CPR, c = it % CPR;
-      float m = ml[0][r][0];
+      __syncthreads();
+    };
+    // chunk c of row r over the four waves: O unnormalised, maximum m, sum lt
+    auto waves = [&](int r, int c, float& m, float& lt) {
+      m = ml[0][r][0];
 #pragma unroll
       for (int w = 1; w < DEC_WAVES; ++w) m = fmaxf(m, ml[w][r][0]);
       f32x4 sum = {};
-      float lt = 0.0f;
+      lt = 0.0f;
 #pragma unroll
       for (int w = 0; w < DEC_WAVES; ++w) {
         const float mw = ml[w][r][0], lw = ml[w][r][1];
         // no finite score: no key of this row (l = 0), or only NaN ones
         const float f = mw == -__builtin_huge_valf() ? 1.0f : __builtin_amdgcn_exp2f(mw - m);
-        lt += f * lw;
-        sum += f * *(const f32x4*)(lds + w * DEC_RING + r * D * 4 + ((c ^ (r & 15)) << 4));
+        lt = fmaf(f, lw, lt);
+        const f32x4 ow = *(const f32x4*)(lds + w * DEC_RING + r * D * 4 + ((c ^ (r & 15)) << 4));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sum[e] = fmaf(f, ow[e], sum[e]);
       }
+      return sum;
+    };
+    auto store = [&](int r, int c, const f32x4& sum, float m, float lt) {
       const int h = hk * G + r % G, q = q0 + r / G;
-      if (whole) {
-        const bool empty = !(lt > 0.0f);  // zero or NaN
-        const float inv = empty ? 1.0f : 1.0f / lt;
-        char* dst = (char*)p.o + 2 * (sg.o_off + (long long)h * p.o_sh + (long long)q * p.o_ss + c * 4);
-        *(u32x2*)dst = (u32x2){pack2(sum[0] * inv, sum[1] * inv, F16), pack2(sum[2] * inv, sum[3] * inv, F16)};
-        if (c == 0)
-          p.lse[sg.lse_off + (long long)h * p.lse_sh + q] =
-              empty ? __builtin_huge_valf() : (m + __log2f(lt)) * 0.69314718055994530942f;
-      } else {
+      const bool empty = !(lt > 0.0f);  // zero or NaN
+      const float inv = empty ? 1.0f : 1.0f / lt;
+      char* dst = (char*)p.o + 2 * (sg.o_off + (long long)h * p.o_sh + (long long)q * p.o_ss + c * 4);
+      *(u32x2*)dst = (u32x2){pack2(sum[0] * inv, sum[1] * inv, F16), pack2(sum[2] * inv, sum[3] * inv, F16)};
+      if (c == 0)
+        p.lse[sg.lse_off + (long long)h * p.lse_sh + q] =
+            empty ? __builtin_huge_valf() : (m + __log2f(lt)) * 0.69314718055994530942f;
+    };
+
+    // range n of the pass: its keys, of the pass's window
+    auto bounds = [&](int n, int& lo, int& hi) {
+      lo = ranged ? max(kbeg, n * g.chunk) : kbeg;
+      hi = ranged && n + 1 < g.splits ? min(kend, (n + 1) * g.chunk) : kend;
+    };
+    constexpr int CPR = D / 4;  // 16-byte chunks (4 d) per row
+    constexpr int NT = DEC_WAVES * 64;
+    int lo, hi;
+    if constexpr (PART) {
+      bounds(split, lo, hi);
+      attend(lo, hi);
+      for (int it = tid; it < qn * G * CPR; it += NT) {
+        const int r = it / CPR, c = it % CPR;
+        float m, lt;
+        const f32x4 sum = waves(r, c, m, lt);
+        if (!ranged) {
+          store(r, c, sum, m, lt);
+          continue;
+        }
         // record (pair, row, split): O unnormalised at the row's D floats,
         // maximum and sum behind all the O rows
         const long long rec = ((long long)pair * g.rows + r) * g.splits + split;
@@ -292,14 +341,43 @@ __device__ __forceinline__ void attn_decode_body(const AttnDecArgs& g) {
           g.ml[2 * rec + 1] = lt;
         }
       }
+      __syncthreads();  // the rings are free for a further pass
+    } else {
+      // thread tid's chunks tid + NT i gather the ranges
+      constexpr int OUT = (ROWS * CPR + NT - 1) / NT;
+      DecRow row[OUT];
+      f32x4 acc[OUT];
+#pragma unroll
+      for (int i = 0; i < OUT; ++i) acc[i] = (f32x4){};
+      for (int n = 0; n < (ranged ? g.splits : 1); ++n) {
+        bounds(n, lo, hi);
+        if (lo >= hi) continue;  // no key: nothing to join
+        attend(lo, hi);
+#pragma unroll
+        for (int i = 0; i < OUT; ++i) {
+          const int it = tid + NT * i;
+          if (it >= qn * G * CPR) continue;
+          float m, lt, was, now;
+          const f32x4 sum = waves(it / CPR, it % CPR, m, lt);
+          if (!row[i].join(m, lt, was, now)) continue;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][e] = fmaf(now, sum[e], was * acc[i][e]);
+        }
+        __syncthreads();  // the rings are free for the next range or pass
+      }
+#pragma unroll
+      for (int i = 0; i < OUT; ++i) {
+        const int it = tid + NT * i;
+        if (it < qn * G * CPR) store(it / CPR, it % CPR, acc[i], row[i].m, row[i].l);
+      }
     }
-    __syncthreads();  // the rings are free for a further pass
   }
 }
 
 // Joins the key ranges of attn_decode_body: one wave per (sequence, head,
-// query), lane s holding range s's maximum and sum, then D / 64 outputs per
-// lane summed over the ranges that saw a key.
+// query), D / 64 outputs per lane.  Lane s holds range s's maximum and sum and
+// works out DecRow's weights at range s (its maximum so far is the greatest
+// of the ranges up to s); they are applied in the ranges' order.
 template <int D, bool F16>
 __device__ __forceinline__ void attn_decode_merge_body(const AttnDecArgs& g) {
   const AttnArgs& p = g.a;
@@ -309,37 +387,56 @@ __device__ __forceinline__ void attn_decode_merge_body(const AttnDecArgs& g) {
   const int pair = item / g.rows, r = item % g.rows;
   const int z = pair / p.Hkv, hk = pair % p.Hkv;
   const int h = hk * p.group + r % p.group, q = r / p.group;
-  const SeqGeom sg = varlen_geom(p, g.v, z);
-  if (q >= sg.q_len) return;
+  // eight records' O in flight, the first of them beside the maxima and sums
+  constexpr int E = D / 64, U = 8;
   const long long rec = (long long)item * g.splits;
+  float v[U][E];
+  auto load = [&](int s0) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < E; ++e) v[u][e] = g.part[(rec + min(s0 + u, g.splits - 1)) * D + lane * E + e];
+  };
+  load(0);
   float m = -__builtin_huge_valf(), l = 0.0f;
   if (lane < g.splits) {
     m = g.ml[2 * (rec + lane)];
     l = g.ml[2 * (rec + lane) + 1];
   }
-  const float mt = wave_reduce<OpMax>(m);
-  const float f = m == -__builtin_huge_valf() ? 1.0f : __builtin_amdgcn_exp2f(m - mt);
-  const float lt = wave_reduce<OpSum>(f * l);
-  constexpr int E = D / 64;
-  float acc[E] = {};
-  const uint64_t live = __ballot(m != -__builtin_huge_valf() || l != 0.0f);
-  const int first = live ? __builtin_ctzll(live) : 0;
-  // eight records in flight; one that saw no key is replaced by the first
-  // that did, at weight 0 (its own O may hold anything)
-  for (int s0 = 0; s0 < g.splits && live; s0 += 8) {
-    float v[8][E], fs[8];
+  const SeqGeom sg = varlen_geom(p, g.v, z);
+  if (q >= sg.q_len) return;
+  // greatest maximum of ranges 0 .. lane (row_shr 1, 2, 4, 8, then across rows)
+  constexpr float none = -__builtin_huge_valf();
+  float to = fmaxf(m, dpp_f32<0x111, 0xF>(none, m));
+  to = fmaxf(to, dpp_f32<0x112, 0xF>(none, to));
+  to = fmaxf(to, dpp_f32<0x114, 0xF>(none, to));
+  to = fmaxf(to, dpp_f32<0x118, 0xF>(none, to));
+  to = fmaxf(to, dpp_f32<0x142, 0xA>(none, to));
+  to = fmaxf(to, dpp_f32<0x143, 0xC>(none, to));
+  const float before = __shfl_up(to, 1);  // by all lanes
+  auto of = [](float x, int s) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), s));
+  };
+  const float mt = of(to, 63);  // (read here, where every lane has worked its part out)
+  DecRow row;
+  row.m = lane ? before : none;
+  float was, now;
+  const bool seen = row.join(m, l, was, now);
+  // a range left out: 0 x -0 + 1 x what was gathered, without a branch
+  const uint64_t live = __ballot(seen);
+  was = seen ? was : 1.0f;
+  now = seen ? now : 0.0f;
+  float acc[E] = {}, lt = 0.0f;
+  for (int s0 = 0; s0 < g.splits; s0 += U) {
+    if (s0) load(s0);
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const bool on = s0 + u < g.splits && (live >> (s0 + u)) & 1;
-      const int s = on ? s0 + u : first;
-      fs[u] = on ? __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), s)) : 0.0f;
+    for (int u = 0; u < U; ++u) {
+      const int s = s0 + u;  // (a lane past the ranges is one left out)
+      const float w = of(was, s), n = of(now, s);
+      lt = fmaf(n, of(l, s), w * lt);
 #pragma unroll
-      for (int e = 0; e < E; ++e) v[u][e] = g.part[(rec + s) * D + lane * E + e];
+      for (int e = 0; e < E; ++e) acc[e] = fmaf(n, (live >> s) & 1 ? v[u][e] : -0.0f, w * acc[e]);
     }
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-#pragma unroll
-      for (int e = 0; e < E; ++e) acc[e] = fmaf(fs[u], v[u][e], acc[e]);
   }
   const bool empty = !(lt > 0.0f);  // zero or NaN
   const float inv = empty ? 1.0f : 1.0f / lt;
@@ -353,21 +450,21 @@ __device__ __forceinline__ void attn_decode_merge_body(const AttnDecArgs& g) {
 
 }  // namespace g950
 
-#define G950_DEC(NAME, D, F16)                                                                             \
-  extern "C" __global__ __launch_bounds__(256) void NAME##_r16(const g950::AttnDecArgs g) {                \
-    g950::attn_decode_body<D, F16, 1, 0>(g);                                                               \
-  }                                                                                                        \
-  extern "C" __global__ __launch_bounds__(256) void NAME##_r16_pg(const g950::AttnDecArgs g) {             \
-    g950::attn_decode_body<D, F16, 1, 1>(g);                                                               \
-  }                                                                                                        \
-  extern "C" __global__ __launch_bounds__(256) void NAME##_r32(const g950::AttnDecArgs g) {                \
-    g950::attn_decode_body<D, F16, 2, 0>(g);                                                               \
-  }                                                                                                        \
-  extern "C" __global__ __launch_bounds__(256) void NAME##_r32_pg(const g950::AttnDecArgs g) {             \
-    g950::attn_decode_body<D, F16, 2, 1>(g);                                                               \
-  }                                                                                                        \
-  extern "C" __global__ __launch_bounds__(256) void NAME##_merge(const g950::AttnDecArgs g) {              \
-    g950::attn_decode_merge_body<D, F16>(g);                                                               \
+// _part: one of a pair's key ranges per workgroup; without it all of them
+#define G950_DEC_BODY(NAME, D, F16, RT, PG)                                                        \
+  extern "C" __global__ __launch_bounds__(256) void NAME(const g950::AttnDecArgs g) {              \
+    g950::attn_decode_body<D, F16, RT, PG, false>(g);                                              \
+  }                                                                                                \
+  extern "C" __global__ __launch_bounds__(256) void NAME##_part(const g950::AttnDecArgs g) {       \
+    g950::attn_decode_body<D, F16, RT, PG, true>(g);                                               \
+  }
+#define G950_DEC(NAME, D, F16)                                                                     \
+  G950_DEC_BODY(NAME##_r16, D, F16, 1, 0)                                                          \
+  G950_DEC_BODY(NAME##_r16_pg, D, F16, 1, 1)                                                       \
+  G950_DEC_BODY(NAME##_r32, D, F16, 2, 0)                                                          \
+  G950_DEC_BODY(NAME##_r32_pg, D, F16, 2, 1)                                                       \
+  extern "C" __global__ __launch_bounds__(256) void NAME##_merge(const g950::AttnDecArgs g) {      \
+    g950::attn_decode_merge_body<D, F16>(g);                                                       \
   }
 G950_DEC(g950_attn_dec_bf16_d128, 128, false)
 G950_DEC(g950_attn_dec_bf16_d64, 64, false)

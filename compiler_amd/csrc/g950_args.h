@@ -147,8 +147,8 @@ struct AttnVarArgs {
 struct AttnDecArgs {
   AttnArgs a;
   VarlenArgs v;
-  float* part;  // splits > 1: [pairs * rows * splits][D] unnormalised O
-  float* ml;    //             [pairs * rows * splits][2] maximum (log2 units), sum
+  float* part;  // _part kernels: [pairs * rows * splits][D] unnormalised O
+  float* ml;    //                [pairs * rows * splits][2] maximum (log2 units), sum
   int splits;   // key ranges per pair
   int chunk;    // keys per range but the last, which takes the rest (multiple of 16)
   int rows;     // seqlen_q * group

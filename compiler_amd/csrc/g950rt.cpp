@@ -1437,6 +1437,14 @@ void* optional_workspace(g950_module* m, void* stream, size_t bytes) {
 // one sequence of 8192 keys 29.5 us against 21.8 (256) and 19.8 (512), one
 // of 1024 keys runs 11.7 against 13.6 with 512.  Up to 512 keys one range and
 // one launch: 40 sequences of 400 keys 21.3 -> 14.5, 2 of 500 11.4 -> 7.4.
+// The ranges are cut from seqlen_k, not from the sequences' device-held
+// lengths: with a seqlen_k of 16384 or more the 32 sequences of 4096..300 fall
+// into range 0 and run 71 against 60.
+// Without the workspace (captured graphs, no-alloc calls, a failed
+// allocation) one workgroup per pair takes the ranges in turn, for the same
+// bits: one sequence of 8192 keys 127 against 13.2, 32 of 4096..300 74 against
+// 60, 64 of 2048 95 against 100.  (One range instead takes 84, 67 and 94, but
+// rounds the probabilities against other maxima.)
 constexpr long long kDecTarget = 4, kDecMinKeys = 256, kDecOneRange = 512;
 
 int launch_attn_decode(g950_module* m, AttnDecArgs& a, uint32_t dt, long long D, bool paged, void* stream) {
@@ -1445,20 +1453,23 @@ int launch_attn_decode(g950_module* m, AttnDecArgs& a, uint32_t dt, long long D,
   long long splits = std::min({(kDecTarget * cus + pairs - 1) / pairs, (long long)(a.a.Sk + kDecMinKeys - 1) / kDecMinKeys,
                                64ll});  // the merge holds a pair's ranges in one wave's lanes
   splits = a.a.Sk <= kDecOneRange ? 1 : std::max(splits, 1ll);
-  if (splits > 1 && m) {
+  a.chunk = (int)(((a.a.Sk + splits - 1) / splits + 63) / 64 * 64);
+  a.splits = (int)splits;
+  bool part = splits > 1;  // a workgroup per range, else one per pair for all of them
+  if (part && m) {
     const long long recs = pairs * a.rows * splits;
     a.part = (float*)optional_workspace(m, stream, (size_t)recs * (size_t)(D + 2) * 4);
     a.ml = a.part + recs * D;
-    if (!a.part) splits = 1;
+    part = a.part != nullptr;
   }
-  a.chunk = (int)(((a.a.Sk + splits - 1) / splits + 63) / 64 * 64);
-  a.splits = (int)splits;
   const char* ty = dt == G950_DTYPE_BFLOAT16 ? "bf16" : "f16";
+  const long long blocks = pairs * (part ? splits : 1);
+  if (blocks > 0x7FFFFFFF) return fail(G950_USAGE, "flash_varlen: grid too large");
   char name[64];
-  snprintf(name, sizeof name, "g950_attn_dec_%s_d%lld_r%d%s", ty, D, a.rows <= 16 ? 16 : 32, paged ? "_pg" : "");
-  if (pairs * splits > 0x7FFFFFFF) return fail(G950_USAGE, "flash_varlen: grid too large");
-  if (int rc = launch(m, name, (unsigned)(pairs * splits), 256u, a, stream)) return rc;
-  if (splits == 1) return G950_OK;
+  snprintf(name, sizeof name, "g950_attn_dec_%s_d%lld_r%d%s%s", ty, D, a.rows <= 16 ? 16 : 32, paged ? "_pg" : "",
+           part ? "_part" : "");
+  if (int rc = launch(m, name, (unsigned)blocks, 256u, a, stream)) return rc;
+  if (!part) return G950_OK;
   snprintf(name, sizeof name, "g950_attn_dec_%s_d%lld_merge", ty, D);
   return launch(m, name, (unsigned)((pairs * a.rows + 3) / 4), 256u, a, stream);
 }

@@ -83,15 +83,20 @@ def test_decode_attention_longer_sequences_than_seqlen_q(seqlen_q, d):
     assert rt.module().last_kernel.endswith("_merge")
 
 
-def test_decode_attention_without_workspace():
-    """No-alloc calls and captured graphs keep to one key range per pair (no
-    workspace) and give the same results within the bar; a graph replayed
-    between other work gives its own result again."""
-    a, meta = inputs.varlen_case(batches=2, max_q=1, max_k=3000, h=8, hk=2, d=128, var_q=False, var_k=False)
+def device_args(a, dt=torch.bfloat16):
     t = {n: torch.from_numpy(np.ascontiguousarray(a[n]).view(np.int64) if a[n].dtype == np.uint64
                              else np.ascontiguousarray(a[n])).to("cuda") for n in ops._VARLEN_VIEWS}
     for n in ("q_ptr", "k_ptr", "v_ptr", "o_ptr"):
-        t[n] = t[n].to(torch.bfloat16)
+        t[n] = t[n].to(dt)
+    return t
+
+
+def test_decode_attention_without_workspace():
+    """No-alloc calls and captured graphs keep to one workgroup per pair (no
+    workspace) and give the same results; a graph replayed between other work
+    gives its own result again."""
+    a, meta = inputs.varlen_case(batches=2, max_q=1, max_k=3000, h=8, hk=2, d=128, var_q=False, var_k=False)
+    t = device_args(a)
     scal = {n: {**a, **meta}[n] for n in ops._VARLEN_SCALARS}
     ops.flash_varlen_fwd_kernel(**t, **scal, sync=True)
     assert rt.module().last_kernel.endswith("_merge")
@@ -121,10 +126,7 @@ def test_decode_attention_leaves_captured_workspace_alone():
     it as it is."""
     stream = torch.cuda.Stream()
     a, meta = inputs.varlen_case(batches=4, max_q=1, max_k=4000, h=32, hk=8, d=128, var_q=False, var_k=False)
-    t = {n: torch.from_numpy(np.ascontiguousarray(a[n]).view(np.int64) if a[n].dtype == np.uint64
-                             else np.ascontiguousarray(a[n])).to("cuda") for n in ops._VARLEN_VIEWS}
-    for n in ("q_ptr", "k_ptr", "v_ptr", "o_ptr"):
-        t[n] = t[n].to(torch.bfloat16)
+    t = device_args(a)
     scal = {n: {**a, **meta}[n] for n in ops._VARLEN_SCALARS}
     x = torch.randn(2, 60000, device="cuda")
     y = torch.zeros_like(x)
@@ -149,3 +151,56 @@ def test_decode_attention_leaves_captured_workspace_alone():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, want)
+
+
+SAME_BITS = {n: CASES[n] for n in ("ranges", "ranges_d64", "rows32", "rows17", "local", "paged16", "paged64", "seqused")}
+SAME_BITS["one_long"] = dict(batches=1, max_q=1, max_k=8000, h=8, hk=1, d=128, causal=True, window_right=0)
+
+
+@pytest.mark.parametrize("case", sorted(SAME_BITS) + ["longer_than_seqlen_q", "climbing", "not_finite"])
+def test_decode_attention_same_bits_without_workspace(case):
+    """A call gives the same bits whether its key ranges run side by side (own
+    workspace), under no_alloc or in a captured graph, on every replay: the
+    ranges are joined by the same operations in the same order.  Also where
+    sequences hold more queries than seqlen_q, where every range moves the
+    maximum, and where keys are inf or NaN."""
+    a, meta = inputs.varlen_case(**SAME_BITS.get(case, dict(batches=2, max_q=5, max_k=2500, h=8, hk=2, d=128, causal=True,
+                                                            window_right=0)))
+    scal = {n: {**a, **meta}[n] for n in ops._VARLEN_SCALARS}
+    t = device_args(a)
+    if case == "longer_than_seqlen_q":
+        scal["seqlen_q"] = 2
+    rows = t["k_ptr"].view(-1, 2, 128) if case in ("climbing", "not_finite") else None
+    if case == "climbing":
+        rows *= (torch.arange(rows.shape[0], device="cuda")[:, None, None] / 40).to(rows.dtype)
+    if case == "not_finite":
+        rows[700, 0], rows[900, 1] = float("inf"), float("nan")
+    out = ("o_ptr", "softmax_lse_ptr")
+
+    def result():
+        torch.cuda.synchronize()
+        return [t[n].view(torch.int16 if n == "o_ptr" else torch.int32).clone() for n in out]
+
+    def poison():
+        for n in out:
+            t[n].fill_(7.0)
+
+    poison()
+    ops.flash_varlen_fwd_kernel(**t, **scal, sync=True)
+    assert rt.module().last_kernel.endswith("_merge")
+    want = result()
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        ops.flash_varlen_fwd_kernel(**t, **scal)
+    for _ in range(3):
+        poison()
+        graph.replay()
+        assert all(torch.equal(g, w) for g, w in zip(result(), want))
+        poison()
+        ops.flash_varlen_fwd_kernel(**t, **scal)
+        assert all(torch.equal(g, w) for g, w in zip(result(), want))
+    poison()
+    with rt.no_alloc():
+        ops.flash_varlen_fwd_kernel(**t, **scal)
+    assert not rt.module().last_kernel.endswith("_merge")
+    assert all(torch.equal(g, w) for g, w in zip(result(), want))
