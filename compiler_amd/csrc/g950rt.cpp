@@ -1178,7 +1178,9 @@ int op_dequant_matmul(g950_module* m, const g950_view* views, uint32_t nviews, c
                   stream);
   }
   g.a_s0 = a.stride[0]; g.a_s1 = a.stride[1];
-  g.b_s0 = b.stride[0]; g.b_s1 = b.stride[1];
+  // B as the caller laid it out, or its K-contiguous copy
+  g.b_s0 = transposed ? 1 : b.stride[0];
+  g.b_s1 = transposed ? bts : b.stride[1];
   g.tiles_n = (int)((N + 63) / 64);
   const long long blocks = ((M + 63) / 64) * g.tiles_n;
   if (blocks > 0x7FFFFFFF) return fail(G950_USAGE, "dequant_matmul: too many tiles");
