@@ -704,13 +704,14 @@ constexpr FewRowsForm kFewRows[2][3][4] = {
     // int8 weights
     {{{1, 8, 4}, {2, 8, 3}, {3, 8, 4}, {4, 4, 4}}, {{1, 4, 4}, {2, 4, 4}, {3, 4, 4}, {}}, {{1, 4, 4}, {2, 4, 4}, {}, {}}}};
 
-// `rows` rows at stride s0 (plus a row's part of a slab) within 32-bit offsets
-bool rows_off32(long long rows, long long s0, int esz) {
-  return (__int128)(rows - 1) * s0 * esz + 256 <= (__int128)0xFFFFFFFFll;
+// The rows of a workgroup's tile -- `tile` of the operand's `rows`, at stride
+// s0 -- plus a row's part of a slab within 32-bit offsets.
+bool rows_off32(long long rows, int tile, long long s0, int esz) {
+  return (__int128)(std::min<long long>(rows, tile) - 1) * s0 * esz + 256 <= (__int128)0xFFFFFFFFll;
 }
 
 bool few_rows_ok(const GemmArgs& g, int a_esz, int b_esz) {
-  return g.M <= 64 && rows_off32(64, g.a_s0, a_esz) && rows_off32(64, g.b_s0, b_esz);
+  return g.M <= 64 && rows_off32(g.M, 64, g.a_s0, a_esz) && rows_off32(g.N, 64, g.b_s0, b_esz);
 }
 
 int launch_few_rows(g950_module* m, const char* name, GemmArgs& g, bool w8, void* stream) {
@@ -825,7 +826,7 @@ int op_matmul(g950_module* m, const g950_view* views, uint32_t nviews, const g95
     g.a_s0 = a.stride[0];
     g.b_s0 = b.stride[0];  // k-row stride of B
     // (the smaller tiles' lanes span a slab's 64 k-rows of B by 32-bit offsets)
-    const int tiles = rows_off32(64, b.stride[0], 2) ? gemm_pick_tile(m, g, (int)(K / 64), TILES_16) : gemm_tiles(g);
+    const int tiles = rows_off32(K, 64, b.stride[0], 2) ? gemm_pick_tile(m, g, (int)(K / 64), TILES_16) : gemm_tiles(g);
     if (tiles < 0) return fail(G950_USAGE, "matmul: too many tiles");
     const char* name = a.v->dtype == G950_DTYPE_BFLOAT16 ? "g950_gemm_bf16_256x256_rb" : "g950_gemm_f16_256x256_rb";
     return launch(m, name, (unsigned)tiles, 512u, g, stream);
@@ -1090,7 +1091,7 @@ int op_dequant_matmul(g950_module* m, const g950_view* views, uint32_t nviews, c
     g.b_s0 = N;  // k-row stride of the copy
     g.bscale = nullptr;
     g.cscale = s.v->data; g.cscale_dtype = (int)s.v->dtype;
-    const int tiles = rows_off32(64, N, 2) ? gemm_pick_tile(m, g, (int)(K / 64), TILES_16) : gemm_tiles(g);
+    const int tiles = rows_off32(K, 64, N, 2) ? gemm_pick_tile(m, g, (int)(K / 64), TILES_16) : gemm_tiles(g);
     if (tiles < 0) return fail(G950_USAGE, "dequant_matmul: too many tiles");
     const char* name = bf16 ? "g950_gemm_bf16_256x256_rb" : "g950_gemm_f16_256x256_rb";
     return launch(m, name, (unsigned)tiles, 512u, g, stream);
@@ -1118,16 +1119,17 @@ int op_dequant_matmul(g950_module* m, const g950_view* views, uint32_t nviews, c
     g.b_s0 = bts;
     g.bscale = nullptr;
     g.cscale = s.v->data; g.cscale_dtype = (int)s.v->dtype;
-    if (few_rows_ok(g, 2, 1)) {
-      const long long blocks32 = (N + 31) / 32;
-      const bool c16 = M <= 16 && (M == 1 || blocks32 < cus || 4 * blocks32 > 5 * cus);
-      char name[48];
-      snprintf(name, sizeof name, "g950_gemm_w8a16_skinny%s_%s", c16 ? "_c16" : M <= 16 ? "" : M <= 32 ? "32" : "64",
-               bf16 ? "bf16" : "f16");
-      return launch_few_rows(m, name, g, true, stream);
+    const char* ty = bf16 ? "bf16" : "f16";
+    const int rows = M <= 16 ? 16 : M <= 32 ? 32 : 64;
+    char name[48];
+    if (!few_rows_ok(g, 2, 1)) {  // the last token of long sequences: 64-bit offsets
+      snprintf(name, sizeof name, "g950_gemm_w8a16_far%d_%s", rows, ty);
+      return launch(m, name, (unsigned)((N + 31) / 32), rows == 16 ? 512u : 256u, g, stream);
     }
-    g.cscale = nullptr;
-    g.bscale = s.v->data;
+    const long long blocks32 = (N + 31) / 32;
+    const bool c16 = M <= 16 && (M == 1 || blocks32 < cus || 4 * blocks32 > 5 * cus);
+    snprintf(name, sizeof name, "g950_gemm_w8a16_skinny%s_%s", c16 ? "_c16" : M <= 16 ? "" : M <= 32 ? "32" : "64", ty);
+    return launch_few_rows(m, name, g, true, stream);
   }
   // Many output tiles: widen B once into an exact bf16 / f16 copy in the
   // workspace and run the 256x256 GEMM with the column scale in its epilogue.
@@ -1167,20 +1169,20 @@ int op_dequant_matmul(g950_module* m, const g950_view* views, uint32_t nviews, c
       return launch(m, name, (unsigned)tiles, (unsigned)kernel_threads(m, name, 512), g, stream);
     }
   }
-  if (fast && rows_off32(128, a.stride[0], 2) && rows_off32(128, bts, 1)) {
+  if (fast) {
+    const bool near = rows_off32(M, 128, a.stride[0], 2) && rows_off32(N, 128, bts, 1);
     g.a_s0 = a.stride[0];
     g.b_s0 = bts;  // Bt row (n) stride
     g.bscale = nullptr;
     g.cscale = s.v->data; g.cscale_dtype = (int)s.v->dtype;
     const int tiles = gemm_pick_tile(m, g, (int)((K + 127) / 128), TILES_W8);
     if (tiles < 0) return fail(G950_USAGE, "dequant_matmul: too many tiles");
-    return launch(m, bf16 ? "g950_gemm_w8a16_bf16_128x128" : "g950_gemm_w8a16_f16_128x128", (unsigned)tiles, 512u, g,
-                  stream);
+    char name[48];
+    snprintf(name, sizeof name, "g950_gemm_w8a16_%s%s_128x128", near ? "" : "far_", bf16 ? "bf16" : "f16");
+    return launch(m, name, (unsigned)tiles, 512u, g, stream);
   }
   g.a_s0 = a.stride[0]; g.a_s1 = a.stride[1];
-  // B as the caller laid it out, or its K-contiguous copy
-  g.b_s0 = transposed ? 1 : b.stride[0];
-  g.b_s1 = transposed ? bts : b.stride[1];
+  g.b_s0 = b.stride[0]; g.b_s1 = b.stride[1];
   g.tiles_n = (int)((N + 63) / 64);
   const long long blocks = ((M + 63) / 64) * g.tiles_n;
   if (blocks > 0x7FFFFFFF) return fail(G950_USAGE, "dequant_matmul: too many tiles");

@@ -49,6 +49,7 @@
 // the no-alloc entry when a copy of B would not fit its scratch array.
 #include "g950_common.h"
 
+#include <type_traits>
 #include <utility>
 
 namespace g950 {
@@ -84,6 +85,13 @@ __device__ __forceinline__ void dma16_asm(const char* sbase, uint32_t voff, uint
   const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_dst);
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(m0) : "memory");
 }
+// the same from a 64-bit lane offset (rows too far apart for 32 bits)
+__device__ __forceinline__ void dma16_asm(const char* sbase, long long voff, uint32_t lds_dst) {
+  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_dst);
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(sbase + voff), "{m0}"(m0) : "memory");
+}
+template <bool FAR>
+using DmaOff = std::conditional_t<FAR, long long, uint32_t>;
 
 // Map the linear workgroup id to a (tile_m, tile_n): XCD-contiguous, then
 // grouped by 4 tile-rows.  The hardware deals workgroups round-robin over
@@ -766,7 +774,10 @@ constexpr int W8_LDS = 144 * 1024;  // of the tiled int8-weight kernels
 // computes the TN columns ending there and stores its own.  bf16 512 x 4096 x
 // 4096 97.6 -> 34 us, 300 x 2048 x 2048 41.8 -> 11.7, 1024 x 8192 x 8192 183 ->
 // 152, against the 256 x 256 form; 8192^3 as before.
-template <int MODE, int TM, int TN, int UMASK, int NST, bool W8 = false, bool BROW = false>
+//
+// FAR: 64-bit lane offsets, for rows of A or Bt that lie too far apart (or
+// at negative strides) for 32 bits within a tile.
+template <int MODE, int TM, int TN, int UMASK, int NST, bool W8 = false, bool BROW = false, bool FAR = false>
 __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
   constexpr int AROW = W8 ? 256 : SLAB;            // bytes of an A row per slab
   constexpr int STAGE = TM * AROW + TN * SLAB;
@@ -792,7 +803,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
   // group t of this wave: 8 rows of A or B (rows past the edge repeat the
   // last one; their outputs are not stored), the 16-byte chunks XOR-swizzled
   // by (row >> 1) & 7 as in the 256 x 256 kernels
-  uint32_t doff[DPW];
+  DmaOff<FAR> doff[DPW];
   const uint32_t lds32 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char*)lds;
   // this lane's 16-byte chunk of DMA instruction grp
   auto chunk = [&](int grp) {
@@ -815,7 +826,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
       continue;
     }
     const int src = min(row, (is_a ? p.M - m0 : p.N - n0) - 1);
-    doff[t] = (uint32_t)((long long)src * (is_a ? lda : ldb) + (chunk(grp) << 4));
+    doff[t] = (DmaOff<FAR>)((long long)src * (is_a ? lda : ldb) + (chunk(grp) << 4));
   }
   auto issue = [&](int slab) {
     const uint32_t dst = lds32 + (uint32_t)(slab % NST) * STAGE;
@@ -824,7 +835,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, char* lds) {
     for (int t = 0; t < DPW; ++t) {
       const int grp = wave * DPW + t;
       const bool is_a = grp < AG;
-      uint32_t off = doff[t];
+      DmaOff<FAR> off = doff[t];
       if (tail) off -= max(0, (chunk(grp) << 4) + 16 - (is_a ? 2 * tb : tb));
       dma16_asm((is_a ? abase : bbase) + (long long)slab * (is_a ? AROW : bstep), off, dst + grp * 1024);
     }
@@ -1341,13 +1352,13 @@ __device__ __forceinline__ void i8_sums_body(const I8SumArgs& p) {
 // matmul.py:21-37).  int8 values are exact in bf16/fp16, so A.B accumulates
 // exactly as the unfused pair would from exact weights; the scale multiplies
 // the fp32 accumulator and the result rounds once at the store.
-template <int MODE>
+template <int MODE, bool FAR = false>
 __device__ __forceinline__ void gemm_w8a16_tiles(const GemmArgs& p) {
   __shared__ __attribute__((aligned(1024))) char lds[W8_LDS];
   if (blockDim.x != 512) return;  // launch shape must match the kernel
-  if (p.tile == GEMM_TILE_128x128) gemm_tile_body<MODE, 128, 128, 0, 3, true>(p, lds);
-  else if (p.tile == GEMM_TILE_64x128) gemm_tile_body<MODE, 64, 128, 0, 4, true>(p, lds);
-  else gemm_tile_body<MODE, 64, 64, 0, 6, true>(p, lds);
+  if (p.tile == GEMM_TILE_128x128) gemm_tile_body<MODE, 128, 128, 0, 3, true, false, FAR>(p, lds);
+  else if (p.tile == GEMM_TILE_64x128) gemm_tile_body<MODE, 64, 128, 0, 4, true, false, FAR>(p, lds);
+  else gemm_tile_body<MODE, 64, 64, 0, 6, true, false, FAR>(p, lds);
 }
 
 // Exact copy of an int8 weight matrix Bt[N, K] (row stride b_s0 bytes, K a
@@ -1388,9 +1399,10 @@ __device__ __forceinline__ void widen_i8_body(const GemmArgs& p) {
 // FEW: M <= 8 (W8: 4), one DMA instruction brings all of A's unit; the other
 // rows of the operand hold whatever LDS holds and feed outputs that are not
 // stored (an output row depends on its own row of A alone).
+// FAR: 64-bit lane offsets (gemm_tile_body's notes).
 constexpr int FEW_LDS = 160 * 1024;
 
-template <int MODE, bool W8, int R, int T, int W, int NS, bool FEW = false>
+template <int MODE, bool W8, int R, int T, int W, int NS, bool FEW = false, bool FAR = false>
 __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
   constexpr int ES = W8 ? 1 : (MODE == GEMM_I8) ? 1 : (MODE == GEMM_F32) ? 4 : 2;  // bytes of a B element
   constexpr int AROW = W8 ? 256 : 128;       // bytes of an A row's unit
@@ -1414,7 +1426,7 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
   // DMA instruction u: 8 rows x 128 bytes (W8's A: 4 rows x 256 bytes), the
   // 16-byte chunks XOR-swizzled by the row.  Rows past M repeat row M - 1 and
   // columns past N column N - 1: their outputs are never stored.
-  uint32_t aoff[DA], boff[DB];
+  DmaOff<FAR> aoff[DA], boff[DB];
   auto achunk = [&](int u) {
     const int row = W8 ? u * 4 + (lane >> 4) : u * 8 + (lane >> 3);
     return W8 ? (lane & 15) ^ (row & 15) : (lane & 7) ^ ((row >> 1) & 7);
@@ -1423,10 +1435,11 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
 #pragma unroll
   for (int u = 0; u < DA; ++u) {
     const int row = W8 ? u * 4 + (lane >> 4) : u * 8 + (lane >> 3);
-    aoff[u] = (uint32_t)((long long)min(row, p.M - 1) * lda) + (achunk(u) << 4);
+    aoff[u] = (DmaOff<FAR>)((long long)min(row, p.M - 1) * lda) + (achunk(u) << 4);
   }
 #pragma unroll
-  for (int u = 0; u < DB; ++u) boff[u] = (uint32_t)((long long)min(u * 8 + (lane >> 3), p.N - 1 - n0) * ldb) + (bchunk(u) << 4);
+  for (int u = 0; u < DB; ++u)
+    boff[u] = (DmaOff<FAR>)((long long)min(u * 8 + (lane >> 3), p.N - 1 - n0) * ldb) + (bchunk(u) << 4);
   auto issue = [&](int j) {
     const int unit = wave + W * j;
     const char* as = abase + (long long)unit * AROW;
@@ -1681,6 +1694,24 @@ G950_GEMM_SKINNY(i8, g950::GEMM_I8)
   G950_FEW_ROWS(g950_gemm_w8a16_skinny64_##TY, MODE, true, 4)
 G950_W8A16_SKINNY(bf16, g950::GEMM_BF16)
 G950_W8A16_SKINNY(f16, g950::GEMM_F16)
+// int8 weights, rows out of 32-bit reach (the last token of long sequences):
+// 32 columns per workgroup up to 64 rows of A, and the tiles.  The address
+// arithmetic is hidden: 16 x 4096 x 8192 with A's rows 2^28 elements apart
+// 11.0 us (10.5 at 2^26, in reach), 64 x 8192 x 8192 46, 512 x 4096 x 4096 36.
+#define G950_W8A16_FAR(TY, MODE, ROWS, R, W, NS)                                                    \
+  extern "C" __global__ __launch_bounds__(W * 64) void g950_gemm_w8a16_far##ROWS##_##TY(const g950::GemmArgs p) { \
+    __shared__ __attribute__((aligned(1024))) char lds[g950::FEW_LDS];                              \
+    g950::gemm_stream_body<MODE, true, R, 2, W, NS, false, true>(p, lds);                           \
+  }
+#define G950_W8A16_FARS(TY, MODE)              \
+  G950_W8A16_FAR(TY, MODE, 16, 1, 8, 2)        \
+  G950_W8A16_FAR(TY, MODE, 32, 2, 4, 3)        \
+  G950_W8A16_FAR(TY, MODE, 64, 4, 4, 2)        \
+  extern "C" __global__ __launch_bounds__(512) void g950_gemm_w8a16_far_##TY##_128x128(const g950::GemmArgs p) { \
+    g950::gemm_w8a16_tiles<MODE, true>(p);     \
+  }
+G950_W8A16_FARS(bf16, g950::GEMM_BF16)
+G950_W8A16_FARS(f16, g950::GEMM_F16)
 extern "C" __global__ __launch_bounds__(256) void g950_transpose_b16(const g950::GemmArgs p) {
   g950::transpose16_body(p);
 }

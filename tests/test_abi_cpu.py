@@ -703,3 +703,43 @@ def test_dequant_matmul_k0_never_takes_the_widened_route():
     assert rc == 0, err
     assert name != "g950_gemm_bf16_256x256"
     assert name == "g950_gemm_w8a16_bf16_128x128"
+
+
+def test_gemm_row_reach_counts_the_rows_a_call_has():
+    """32-bit row offsets span the rows of one workgroup's tile that exist:
+    one row at any stride and 16 rows 2^26 elements apart stay on the few-row
+    kernels; rows past the reach keep to MFMA kernels (64-bit offsets), also
+    with row-major weights (transposed first)."""
+    def w8(m, stride, col_b=True, n=4096, k=4096, bstride=None):
+        b = [1, bstride or k] if col_b else [bstride or n, 1]
+        a = (Args().view([m, k], rt.DT_BF16, strides=[stride, 1]).view([k, n], rt.DT_INT8, strides=b)
+             .view([n], rt.DT_BF16).view([m, n], rt.DT_BF16, output=True))
+        rc, name, err = validate(rt.OP_DEQUANT_MATMUL, a, [k, m, n])
+        assert rc == 0, err
+        return name
+    far = "g950_gemm_w8a16_far"
+    for col_b in (True, False):
+        assert w8(1, 1 << 33, col_b) == "g950_gemm_w8a16_skinny_c16_bf16"
+        assert w8(16, 1 << 26, col_b) == "g950_gemm_w8a16_skinny_c16_bf16"
+        assert w8(16, 1 << 28, col_b) == far + "16_bf16"
+        assert w8(64, 1 << 25, col_b) == "g950_gemm_w8a16_skinny64_bf16"
+        assert w8(64, 1 << 26, col_b) == far + "64_bf16"
+        assert w8(20, 1 << 28, col_b) == far + "32_bf16"
+        assert w8(65, 1 << 24, col_b) == "g950_gemm_w8a16_bf16_128x128"
+        assert w8(100, 1 << 25, col_b) == far + "_bf16_128x128"
+        assert w8(300, 1 << 25, col_b) == far + "_bf16_128x128"
+    # Bt rows far apart: 64 (few rows of A) and 128 of them
+    assert w8(8, 4096, n=4096, bstride=1 << 26) == "g950_gemm_w8a16_skinny_c16_bf16"
+    assert w8(8, 4096, n=4096, bstride=3 << 25) == far + "16_bf16"
+    assert w8(8, 4096, n=32, bstride=3 << 25) == "g950_gemm_w8a16_skinny_c16_bf16"
+    assert w8(100, 4096, n=4096, bstride=3 << 24) == far + "_bf16_128x128"
+
+    def mm(m, stride, n=4096, k=4096):
+        a = (Args().view([m, k], rt.DT_BF16, strides=[stride, 1]).view([k, n], rt.DT_BF16, strides=[1, k])
+             .view([m, n], rt.DT_BF16, output=True))
+        rc, name, err = validate(rt.OP_MATMUL, a, [k, m, n])
+        assert rc == 0, err
+        return name
+    assert mm(1, 1 << 33) == "g950_gemm_skinny16_bf16"
+    assert mm(16, 1 << 26) == "g950_gemm_skinny16_bf16"
+    assert mm(64, 1 << 26) == "g950_gemm_bf16_256x256_kt"  # 64-bit offsets, as whole-matrix reach past 4 GiB
