@@ -137,3 +137,41 @@ def test_long_rows_packed(rows, cols):
     assert np.array_equal(np.isnan(lse), np.isnan(want)) and np.isposinf(lse[1]) and np.isneginf(lse[3])
     ok, err = ref.isclose_verdict(lse[5:], want[5:], 3e-5, 3e-6)
     assert ok, err
+
+
+# the most columns a row may have, at two 16-byte phases, and (y one element
+# off x's phase) by element loads
+@pytest.mark.parametrize("offset,y_offset", [(0, 0), (3, 3), (0, 1)])
+def test_split_rows_of_the_most_columns(offset, y_offset):
+    """Columns up to 2^31 - 1: the last chunk counts (its values alone set the
+    variance and the logsumexp) and no vector past the row is read.  Four
+    buffers of 4.3 GB.  LayerNorm bf16: the statistics within 1e-4 (fp32 sums of 2^31
+    terms in chunks), y within bf16 rounding."""
+    n, pad, tail, big = 2**31 - 1, 16, 4000, 1024.0
+    g = torch.Generator(device="cuda").manual_seed(1)
+    xs = torch.empty(n + pad, dtype=torch.bfloat16, device="cuda")
+    for c in xs.split(1 << 28):
+        c.normal_(generator=g)
+    x = xs[offset:offset + n].view(1, n)
+    x[0, -tail:] = big
+    mean = sum(c.double().sum().item() for c in x[0].split(1 << 27)) / n
+    var = sum((c.double() - mean).square().sum().item() for c in x[0].split(1 << 27)) / n
+    ys = torch.full((n + pad,), 7.0, dtype=torch.bfloat16, device="cuda")
+    y = ys[y_offset:y_offset + n].view(1, n)
+    w = torch.ones(n, dtype=torch.bfloat16, device="cuda")
+    b = torch.zeros(n, dtype=torch.bfloat16, device="cuda")
+    _, m, r = ops.layernorm(x, w, b, 1e-5, out=y, sync=True)
+    assert rt.module().last_kernel == "g950_rs_final_layernorm_bf16_v1"
+    rstd = (var + 1e-5) ** -0.5
+    assert abs(m.item() - mean) < 1e-4 and abs(r.item() / rstd - 1) < 1e-4
+    for xc, yc in zip(x[0].split(1 << 27), y[0].split(1 << 27)):
+        want = (xc.float() - mean) * rstd
+        assert bool(((want - yc.float()).abs() <= 2**-8 * want.abs() + 1e-3).all())
+    assert bool((ys[:y_offset] == 7.0).all()) and bool((ys[y_offset + n:] == 7.0).all())
+    if y_offset == offset:
+        del y, ys
+        x[0, -tail:] = 0.0
+        x[0, -1] = 40.0
+        lse = ops.logsumexp(x, sync=True)
+        assert rt.module().last_kernel == "g950_rs_final_logsumexp_bf16_v1"
+        assert abs(lse.item() - 40.0) < 1e-3  # log(e^40 + 2^31 e^0.5): 1.5e-8 past 40
