@@ -646,6 +646,14 @@ int gemm_tiles(GemmArgs& g, int bm = 256, int bn = 256) {
   return (int)(tm * tn);
 }
 
+// The rows of a workgroup's tile -- `tile` of the operand's `rows`, at stride
+// s0 -- plus a row's `part` bytes of a slab within 32-bit unsigned offsets
+// (so no negative stride unless there is one row).
+bool rows_off32(long long rows, int tile, long long s0, int esz, int part = 256) {
+  const long long n = std::min<long long>(rows, tile) - 1;
+  return n <= 0 || (s0 >= 0 && (__int128)n * s0 * esz + part <= (__int128)0xFFFFFFFFll);
+}
+
 // Workgroup tile of a whole-slab MFMA GEMM (GemmArgs::tile) and its tile
 // count: the least of rounds x (slabs x slab time + fixed time), a round
 // being one workgroup per CU.  Smaller tiles cost more per output (a CU's
@@ -704,12 +712,6 @@ constexpr FewRowsForm kFewRows[2][3][4] = {
     // int8 weights
     {{{1, 8, 4}, {2, 8, 3}, {3, 8, 4}, {4, 4, 4}}, {{1, 4, 4}, {2, 4, 4}, {3, 4, 4}, {}}, {{1, 4, 4}, {2, 4, 4}, {}, {}}}};
 
-// The rows of a workgroup's tile -- `tile` of the operand's `rows`, at stride
-// s0 -- plus a row's part of a slab within 32-bit offsets.
-bool rows_off32(long long rows, int tile, long long s0, int esz) {
-  return (__int128)(std::min<long long>(rows, tile) - 1) * s0 * esz + 256 <= (__int128)0xFFFFFFFFll;
-}
-
 bool few_rows_ok(const GemmArgs& g, int a_esz, int b_esz) {
   return g.M <= 64 && rows_off32(g.M, 64, g.a_s0, a_esz) && rows_off32(g.N, 64, g.b_s0, b_esz);
 }
@@ -744,10 +746,7 @@ bool gemm_ktail(int K, int esz) { return (K * esz) % 128 != 0; }
 // either operand can reach plus a slab's last 16-byte chunk must lie below
 // 4 GiB, or the _kt kernels (64-bit addresses) serve the call.
 bool gemm_off32(const GemmArgs& g, int esz) {
-  auto fits = [esz](long long rows, long long s0) {
-    return (__int128)(rows - 1) * s0 * esz + 128 <= (__int128)0xFFFFFFFFll;
-  };
-  return fits(g.M, g.a_s0) && fits(g.N, g.b_s0);
+  return rows_off32(g.M, 0x7FFFFFFF, g.a_s0, esz, 128) && rows_off32(g.N, 0x7FFFFFFF, g.b_s0, esz, 128);
 }
 
 // Row-major B[K,N] (N-contiguous, the reference matmul's layout,
@@ -819,10 +818,10 @@ int op_matmul(g950_module* m, const g950_view* views, uint32_t nviews, const g95
   const bool rowb_ok = same16 && out16 && gemm_rowb_ok(a, b, (int)K, (int)N, esz);
   // Row-major B read directly by the 16x16 MFMA kernel (transposing LDS
   // reads): 16-bit operands, at least one 256 tile each way, whole 64-k
-  // slabs, A's farthest DMA row within a 32-bit offset (B's lane offsets
-  // span 16 k-rows of one slab)
+  // slabs, A's farthest DMA row and the 16 k-rows of one slab that B's lane
+  // offsets span within 32-bit offsets
   if (rowb_ok && esz == 2 && M >= 256 && N >= 256 && K % 64 == 0 &&
-      (__int128)(M - 1) * a.stride[0] * 2 + 128 <= (__int128)0xFFFFFFFFll) {
+      rows_off32(M, 0x7FFFFFFF, a.stride[0], 2, 128) && rows_off32(K, 16, b.stride[0], 2)) {
     g.a_s0 = a.stride[0];
     g.b_s0 = b.stride[0];  // k-row stride of B
     // (the smaller tiles' lanes span a slab's 64 k-rows of B by 32-bit offsets)
@@ -1075,7 +1074,7 @@ int op_dequant_matmul(g950_module* m, const g950_view* views, uint32_t nviews, c
     return bytes <= (1ull << 31) && !(t_scratch && bytes > kScratchWorkspace);
   };
   if (nrow && M >= 256 && N >= 256 && K % 64 == 0 && fits((unsigned long long)K * N * 2) &&
-      (__int128)(M - 1) * a.stride[0] * 2 + 128 <= (__int128)0xFFFFFFFFll) {
+      rows_off32(M, 0x7FFFFFFF, a.stride[0], 2, 128)) {
     void* wide = nullptr;
     if (m)
       if (int rc = workspace(m, stream, (size_t)(K * N * 2), &wide)) return rc;

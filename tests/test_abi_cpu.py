@@ -743,3 +743,42 @@ def test_gemm_row_reach_counts_the_rows_a_call_has():
     assert mm(1, 1 << 33) == "g950_gemm_skinny16_bf16"
     assert mm(16, 1 << 26) == "g950_gemm_skinny16_bf16"
     assert mm(64, 1 << 26) == "g950_gemm_bf16_256x256_kt"  # 64-bit offsets, as whole-matrix reach past 4 GiB
+
+
+def test_gemm_negative_row_strides_leave_the_32_bit_kernels():
+    """The C ABI takes negative strides; unsigned 32-bit lane offsets cannot.
+    Such calls run kernels with 64-bit offsets, the transposed copy of B or
+    the general kernels."""
+    def reversed_rows(args, shape, dtype, stride):
+        far = (shape[0] - 1) * stride
+        return args.view(shape, dtype, strides=[-stride, 1], offset=far, storage_extra=2 * args.ITEM[dtype] * far)
+
+    def kernel(op, m, n, k, dt=rt.DT_BF16, rev="a", col_b=True):
+        w8, i8 = op == rt.OP_DEQUANT_MATMUL, dt == rt.DT_INT8
+        a = Args()
+        a = reversed_rows(a, [m, k], dt, k) if "a" in rev else a.view([m, k], dt)
+        bdt = rt.DT_INT8 if w8 else dt
+        if "b" in rev and not col_b:
+            a = reversed_rows(a, [k, n], bdt, n)
+        elif "b" in rev:
+            a = a.view([k, n], bdt, strides=[1, -k], offset=(n - 1) * k, storage_extra=8 * n * k)
+        else:
+            a = a.view([k, n], bdt, strides=[1, k] if col_b else None)
+        if w8:
+            a = a.view([n], dt)
+        rc, name, err = validate(op, a.view([m, n], rt.DT_INT32 if i8 else dt, output=True), [k, m, n])
+        assert rc == 0, err
+        return name
+    mm, w8 = rt.OP_MATMUL, rt.OP_DEQUANT_MATMUL
+    for rev in ("a", "b", "ab"):
+        assert kernel(mm, 16, 512, 1024, rev=rev) == "g950_gemm_bf16_256x256_kt"
+        assert kernel(mm, 16, 512, 1032, rev=rev) == "g950_gemm_bf16_256x256_kt"
+        assert kernel(mm, 300, 512, 1024, rev=rev) == "g950_gemm_bf16_256x256_kt"
+        assert kernel(rt.OP_MATMUL_I8, 16, 512, 1024, rt.DT_INT8, rev) == "g950_gemm_i8_256x256_kt"
+        assert kernel(w8, 16, 512, 1024, rev=rev) == "g950_gemm_w8a16_far16_bf16"
+        assert kernel(w8, 100, 512, 1024, rev=rev) == "g950_gemm_w8a16_far_bf16_128x128"
+    assert kernel(mm, 1, 512, 1024) == "g950_gemm_skinny16_bf16"   # one row: its stride is not used
+    assert kernel(mm, 300, 512, 1024, rev="a", col_b=False) == "g950_gemm_bf16_256x256_kt"
+    assert kernel(mm, 300, 512, 1024, rev="b", col_b=False) == "g950_gemm_bf16_256x256"   # the copy's rows
+    assert kernel(w8, 300, 512, 1024, rev="a", col_b=False) == "g950_gemm_w8a16_far_bf16_128x128"
+    assert kernel(w8, 300, 512, 1024, rev="b", col_b=False) == "g950_gemm_bf16_256x256_rb"  # the copy's rows
