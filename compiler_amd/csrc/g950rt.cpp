@@ -704,13 +704,15 @@ int gemm_pick_tile(const g950_module* m, GemmArgs& g, int slabs, TileClass cls) 
 // 19.4; with int8 weights 16x4096x4096 9.1 / 8.8 / 9.9 / 11.7, 16x6144x4096
 // 14.0 / 9.4 / 10.6, 16x8192x8192 23.9 / 20.4 / 18.8 / 20.9 (T = 2 at exactly
 // one workgroup per CU loses to T = 3 on two thirds of them, so it ends at
-// three quarters).
+// three quarters; up to 4 rows, where the workgroups start apart in K, it
+// wins: 1x8192x8192 14.6 against 15.5).
 struct FewRowsForm { int t, waves, quarters; };  // taken up to quarters / 4 workgroups per CU
-constexpr FewRowsForm kFewRows[2][3][4] = {
+constexpr FewRowsForm kFewRows[2][4][4] = {
     // 16-bit, int8 and fp32 operands: up to 16, 32, 64 rows
-    {{{1, 8, 4}, {3, 8, 4}, {4, 8, 4}, {}}, {{1, 8, 4}, {2, 8, 4}, {4, 4, 4}, {}}, {{1, 8, 4}, {2, 4, 4}, {4, 4, 4}, {}}},
-    // int8 weights
-    {{{1, 8, 4}, {2, 8, 3}, {3, 8, 4}, {4, 4, 4}}, {{1, 4, 4}, {2, 4, 4}, {3, 4, 4}, {}}, {{1, 4, 4}, {2, 4, 4}, {}, {}}}};
+    {{{1, 8, 4}, {3, 8, 4}, {4, 8, 4}, {}}, {{1, 8, 4}, {2, 8, 4}, {4, 4, 4}, {}}, {{1, 8, 4}, {2, 4, 4}, {4, 4, 4}, {}}, {}},
+    // int8 weights, and up to 4 rows
+    {{{1, 8, 4}, {2, 8, 3}, {3, 8, 4}, {4, 4, 4}}, {{1, 4, 4}, {2, 4, 4}, {3, 4, 4}, {}}, {{1, 4, 4}, {2, 4, 4}, {}, {}},
+     {{1, 8, 4}, {2, 8, 4}, {3, 8, 4}, {4, 4, 4}}}};
 
 bool few_rows_ok(const GemmArgs& g, int a_esz, int b_esz) {
   return g.M <= 64 && rows_off32(g.M, 64, g.a_s0, a_esz) && rows_off32(g.N, 64, g.b_s0, b_esz);
@@ -718,7 +720,7 @@ bool few_rows_ok(const GemmArgs& g, int a_esz, int b_esz) {
 
 int launch_few_rows(g950_module* m, const char* name, GemmArgs& g, bool w8, void* stream) {
   const long long cus = m ? m->cus : 256;
-  const FewRowsForm* form = kFewRows[w8][g.M <= 16 ? 0 : g.M <= 32 ? 1 : 2];
+  const FewRowsForm* form = kFewRows[w8][g.M <= 4 && w8 ? 3 : g.M <= 16 ? 0 : g.M <= 32 ? 1 : 2];
   long long blocks = 0;
   for (int i = 0; i < 4 && form[i].t; ++i) {
     blocks = (g.N + 16ll * form[i].t - 1) / (16 * form[i].t);
@@ -1126,6 +1128,10 @@ int op_dequant_matmul(g950_module* m, const g950_view* views, uint32_t nviews, c
       return launch(m, name, (unsigned)((N + 31) / 32), rows == 16 ? 512u : 256u, g, stream);
     }
     const long long blocks32 = (N + 31) / 32;
+    if (M <= 4 && N > 64 * cus) {  // past one round of the widest form (gemm.hip G950_W8A16_FEW)
+      snprintf(name, sizeof name, "g950_gemm_w8a16_few_%s", ty);
+      return launch(m, name, (unsigned)blocks32, 512u, g, stream);
+    }
     const bool c16 = M <= 16 && (M == 1 || blocks32 < cus || 4 * blocks32 > 5 * cus);
     snprintf(name, sizeof name, "g950_gemm_w8a16_skinny%s_%s", c16 ? "_c16" : M <= 16 ? "" : M <= 32 ? "32" : "64", ty);
     return launch_few_rows(m, name, g, true, stream);

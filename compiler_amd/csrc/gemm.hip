@@ -1400,13 +1400,24 @@ __device__ __forceinline__ void widen_i8_body(const GemmArgs& p) {
 // rows of the operand hold whatever LDS holds and feed outputs that are not
 // stored (an output row depends on its own row of A alone).
 // FAR: 64-bit lane offsets (gemm_tile_body's notes).
+// With int8 weights and FEW each workgroup starts at its own place in K (the
+// golden ratio's multiples spread them evenly) and wraps round: where all
+// workgroups walk K in step, rows of 8 KiB or so keep them on the same few
+// HBM channels.  One row of A, from 0 -> spread (us; the kernel that loaded
+// operands into registers, each wave its own part of K): 4096 x 11008 14.5 ->
+// 12.0 (13.1), 8192 x 22016 43.4 -> 32.6 (38.0), 16384 x 8192 29.9 -> 25.8
+// (26.4), 4096 x 8192 10.0 -> 9.8 (9.0).
+// A4: the unit holds FEW's four rows of A alone, so that two workgroups fit a
+// CU: for grids of more than one round (gemm_w8a16_few).
 constexpr int FEW_LDS = 160 * 1024;
 
-template <int MODE, bool W8, int R, int T, int W, int NS, bool FEW = false, bool FAR = false>
+template <int MODE, bool W8, int R, int T, int W, int NS, bool FEW = false, bool FAR = false, bool A4 = false>
 __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
   constexpr int ES = W8 ? 1 : (MODE == GEMM_I8) ? 1 : (MODE == GEMM_F32) ? 4 : 2;  // bytes of a B element
   constexpr int AROW = W8 ? 256 : 128;       // bytes of an A row's unit
-  constexpr int AU = 16 * R * AROW, BU = 16 * T * 128, UNIT = AU + BU;
+  static_assert(!A4 || (W8 && FEW && R == 1), "four rows of A");
+  constexpr bool SPREAD = W8 && FEW;
+  constexpr int AU = A4 ? 1024 : 16 * R * AROW, BU = 16 * T * 128, UNIT = AU + BU;
   constexpr int DA = FEW ? 1 : AU / 1024, DB = BU / 1024, DPU = DA + DB;
   static_assert(W * NS * UNIT <= FEW_LDS && NS >= 2 && R * T * 1024 <= NS * UNIT, "the rings fit LDS");
   if (blockDim.x != W * 64) return;  // launch shape must match the kernel
@@ -1440,8 +1451,13 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
 #pragma unroll
   for (int u = 0; u < DB; ++u)
     boff[u] = (DmaOff<FAR>)((long long)min(u * 8 + (lane >> 3), p.N - 1 - n0) * ldb) + (bchunk(u) << 4);
+  const int start = SPREAD ? (int)(((uint64_t)(blockIdx.x * 2654435769u) * (uint32_t)units) >> 32) : 0;
+  auto unit_of = [&](int j) {  // this wave's j-th unit of K
+    const int u = start + wave + W * j;
+    return SPREAD && u >= units ? u - units : u;
+  };
   auto issue = [&](int j) {
-    const int unit = wave + W * j;
+    const int unit = unit_of(j);
     const char* as = abase + (long long)unit * AROW;
     const char* bs = bbase + (long long)unit * 128;
     const uint32_t dst = ring32 + (uint32_t)(j % NS) * UNIT;
@@ -1474,7 +1490,7 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
     if (j + NS <= nloc) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * DPU) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const char* st = ring + (j % NS) * UNIT;
-    const bool tail = wave + W * j == units - 1 && tb != 128;
+    const bool tail = unit_of(j) == units - 1 && tb != 128;
     u32x4 av[2][R][W8 ? 2 : 1], bv[2][T];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -1484,8 +1500,9 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         if constexpr (W8) {
-          av[h][r][0] = *(const u32x4*)(st + (16 * r + l16) * 256 + (((2 * c) ^ l16) << 4));
-          av[h][r][1] = *(const u32x4*)(st + (16 * r + l16) * 256 + (((2 * c + 1) ^ l16) << 4));
+          const int row = A4 ? l16 & 3 : l16;
+          av[h][r][0] = *(const u32x4*)(st + (16 * r + row) * 256 + (((2 * c) ^ row) << 4));
+          av[h][r][1] = *(const u32x4*)(st + (16 * r + row) * 256 + (((2 * c + 1) ^ row) << 4));
         } else {
           av[h][r][0] = *(const u32x4*)(st + (16 * r + l16) * 128 + ((c ^ ((l16 >> 1) & 7)) << 4));
         }
@@ -1694,6 +1711,18 @@ G950_GEMM_SKINNY(i8, g950::GEMM_I8)
   G950_FEW_ROWS(g950_gemm_w8a16_skinny64_##TY, MODE, true, 4)
 G950_W8A16_SKINNY(bf16, g950::GEMM_BF16)
 G950_W8A16_SKINNY(f16, g950::GEMM_F16)
+// int8 weights, up to four rows of A, more columns than one round of the CUs
+// holds: 32 columns per workgroup, two workgroups per CU.  One row of A (us;
+// 64 columns and one workgroup per CU -> this; the register-loading kernel):
+// 100000 x 4096 93.1 -> 65.7 (84.6), 50000 x 8192 92.9 -> 69.4 (74.5), 20000 x
+// 4096 25.3 -> 17.5 (21.9).
+#define G950_W8A16_FEW(TY, MODE)                                                                       \
+  extern "C" __global__ __launch_bounds__(512) void g950_gemm_w8a16_few_##TY(const g950::GemmArgs p) { \
+    __shared__ __attribute__((aligned(1024))) char lds[80 * 1024];                                     \
+    g950::gemm_stream_body<MODE, true, 1, 2, 8, 2, true, false, true>(p, lds);                         \
+  }
+G950_W8A16_FEW(bf16, g950::GEMM_BF16)
+G950_W8A16_FEW(f16, g950::GEMM_F16)
 // int8 weights, rows out of 32-bit reach (the last token of long sequences):
 // 32 columns per workgroup up to 64 rows of A, and the tiles.  The address
 // arithmetic is hidden: 16 x 4096 x 8192 with A's rows 2^28 elements apart

@@ -83,3 +83,26 @@ def test_few_rows_keep_nan_to_their_own_row():
     bt = torch.randn(40, 1024, device=DEV).to(torch.bfloat16)
     y = ops.matmul(a, bt.t(), sync=True)
     assert bool(y[2].isnan().all()) and not bool(y[[0, 1, 3, 4]].isnan().any())
+
+
+@pytest.mark.parametrize("dt", ["bfloat16", "float16"])
+@pytest.mark.parametrize("m,n,chunks", [(1, 16385, 1), (4, 16415, 9), (3, 20001, 69), (2, 16390, 64), (1, 16400, 127),
+                                        (4, 33000, 17)])
+def test_few_rows_int8_weights_past_one_round(m, n, chunks, dt):
+    """Up to four rows of A against more columns than one round of the widest
+    form holds: the two-workgroups-per-CU kernel, whose workgroups start at
+    different units of K and wrap round (fewer units than waves, tails)."""
+    rng = np.random.default_rng(m + n + chunks)
+    k = 16 * chunks
+    a = torch.from_numpy(rng.standard_normal((m, k)).astype(np.float32) * 0.5).to(DEV).to(TD[dt])
+    bt = rng.integers(-127, 128, (n, k)).astype(np.int8)
+    s = torch.from_numpy((rng.random(n) / 64).astype(np.float32)).to(DEV).to(TD[dt])
+    full = torch.full((m + 2, n + 5), 7.0, dtype=TD[dt], device=DEV)
+    y = torch.as_strided(full, (m, n), (n + 5, 1), (n + 5) // 8 * 8)
+    ops.dequant_matmul_kernel(a, torch.from_numpy(bt).to(DEV).t(), s, y, m, n, k, sync=True)
+    assert rt.module().last_kernel == f"g950_gemm_w8a16_few_{'bf16' if dt == 'bfloat16' else 'f16'}"
+    expect = ref.matmul(a.float().cpu().numpy(), ref.dequantize(bt.T, s.float().cpu().numpy()))
+    ok, err = ref.isclose_verdict(y.float().cpu().numpy(), expect, 2e-2, 2e-2)
+    assert ok, err
+    y.fill_(7.0)
+    assert bool((full == 7.0).all())
