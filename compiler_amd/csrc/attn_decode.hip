@@ -450,13 +450,18 @@ __device__ __forceinline__ void attn_decode_merge_body(const AttnDecArgs& g) {
 
 }  // namespace g950
 
-// _part: one of a pair's key ranges per workgroup; without it all of them
-#define G950_DEC_BODY(NAME, D, F16, RT, PG)                                                        \
-  extern "C" __global__ __launch_bounds__(256) void NAME(const g950::AttnDecArgs g) {              \
-    g950::attn_decode_body<D, F16, RT, PG, false>(g);                                              \
-  }                                                                                                \
-  extern "C" __global__ __launch_bounds__(256) void NAME##_part(const g950::AttnDecArgs g) {       \
-    g950::attn_decode_body<D, F16, RT, PG, true>(g);                                               \
+// _part: one of a pair's key ranges per workgroup; without it all of them.
+// Two waves per SIMD (256 registers), so that two workgroups share a CU: left
+// to itself the compiler gave the paged 32-row form at d = 128 264 and the
+// forms that gather all ranges up to 305; bounded they take 185 to 233 without
+// a spill.  Groups of 8, 4 queries, 64-key pages: 64 sequences of 2048 keys
+// (32/4 heads) 72.3 -> 58.2 us, 64 of 4096..300 (8/1) 40.9 -> 29.6.
+#define G950_DEC_BODY(NAME, D, F16, RT, PG)                                                     \
+  extern "C" __global__ __launch_bounds__(256, 2) void NAME(const g950::AttnDecArgs g) {        \
+    g950::attn_decode_body<D, F16, RT, PG, false>(g);                                           \
+  }                                                                                             \
+  extern "C" __global__ __launch_bounds__(256, 2) void NAME##_part(const g950::AttnDecArgs g) { \
+    g950::attn_decode_body<D, F16, RT, PG, true>(g);                                            \
   }
 #define G950_DEC(NAME, D, F16)                                                                     \
   G950_DEC_BODY(NAME##_r16, D, F16, 1, 0)                                                          \

@@ -34,6 +34,8 @@ CASES = {
                     causal=True, window_right=0),
     "paged64": dict(batches=2, max_q=4, max_k=4500, h=8, hk=1, d=64, paged=True, block_size=64, causal=True,
                     window_right=0),
+    "paged_rows32": dict(batches=2, max_q=4, max_k=1300, h=8, hk=1, d=128, paged=True, block_size=32, causal=True,
+                         window_right=0),
     "paged48": dict(batches=2, max_q=1, max_k=400, h=4, hk=4, d=128, var_q=False, paged=True, block_size=48),
     "fewer_keys_than_queries": dict(batches=1, max_q=8, max_k=5, h=2, hk=1, d=64, causal=True, window_right=0),
     "seqused": dict(batches=3, max_q=1, max_k=520, h=8, hk=8, d=128, var_q=False, seqused_trim=37),
@@ -153,7 +155,8 @@ def test_decode_attention_leaves_captured_workspace_alone():
         assert torch.equal(y, want)
 
 
-SAME_BITS = {n: CASES[n] for n in ("ranges", "ranges_d64", "rows32", "rows17", "local", "paged16", "paged64", "seqused")}
+SAME_BITS = {n: CASES[n] for n in ("ranges", "ranges_d64", "rows32", "rows17", "local", "paged16", "paged64",
+                                 "paged_rows32", "seqused")}
 SAME_BITS["one_long"] = dict(batches=1, max_q=1, max_k=8000, h=8, hk=1, d=128, causal=True, window_right=0)
 
 
