@@ -1417,9 +1417,10 @@ long long rows_held(long long n, long long rs, long long nh, long long hs, long 
 // streams as long as their routes leave it alone.  Not under stream capture:
 // nothing can be allocated there, and a graph would keep an address that a
 // later, larger call frees.  A capture on another stream is left undisturbed
-// (relaxed mode around the allocation).
+// (relaxed mode around the allocation).  Not on hipStreamPerThread: that one
+// handle names a stream of every thread, whose calls nothing orders.
 void* optional_workspace(g950_module* m, void* stream, size_t bytes) {
-  if (t_scratch) return nullptr;
+  if (t_scratch || (hipStream_t)stream == hipStreamPerThread) return nullptr;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
     (void)hipGetLastError();

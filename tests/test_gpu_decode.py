@@ -207,3 +207,32 @@ def test_decode_attention_same_bits_without_workspace(case):
         ops.flash_varlen_fwd_kernel(**t, **scal)
     assert not rt.module().last_kernel.endswith("_merge")
     assert all(torch.equal(g, w) for g, w in zip(result(), want))
+
+
+def test_decode_attention_per_thread_streams_share_no_workspace():
+    """hipStreamPerThread (handle 2) is one handle for a stream of every
+    thread: calls on it take no workspace, and give the same bits, also from
+    two threads at once."""
+    import threading
+    a, meta = inputs.varlen_case(batches=2, max_q=1, max_k=3000, h=8, hk=2, d=128, var_q=False, var_k=False)
+    scal = {n: {**a, **meta}[n] for n in ops._VARLEN_SCALARS}
+    t = [device_args(a) for _ in range(2)]
+    ops.flash_varlen_fwd_kernel(**t[0], **scal, sync=True)
+    want = t[0]["o_ptr"].clone()
+    t[0]["o_ptr"].zero_()
+    torch.cuda.synchronize()
+    names, held = [], rt.module().workspace_bytes(2)
+
+    def calls(args):
+        for _ in range(20):
+            ops.flash_varlen_fwd_kernel(**args, **scal, stream=2)
+        rt.load_library().g950_sync(2)
+        names.append(rt.load_library().g950_last_kernel().decode())
+    threads = [threading.Thread(target=calls, args=(x,)) for x in t]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    assert names == ["g950_attn_dec_bf16_d128_r16"] * 2 and rt.module().workspace_bytes(2) == held == 0
+    assert all(torch.equal(x["o_ptr"], want) for x in t)
