@@ -11,6 +11,7 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <cstring>
 
@@ -151,4 +152,9 @@ PyModuleDef def = {PyModuleDef_HEAD_INIT, "g950_py", nullptr, -1, methods, nullp
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_g950_py(void) { return PyModule_Create(&def); }
+PyMODINIT_FUNC PyInit_g950_py(void) {
+  PyObject* m = PyModule_Create(&def);
+  // launch() reads tensors by this torch's layouts: the loader compares
+  if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION)) Py_CLEAR(m);
+  return m;
+}

@@ -188,8 +188,9 @@ _packer = None
 
 
 def _load_packer():
-    """g950_py.so (native packing of a call's arguments); torch must be
-    importable.  No fallback: a missing library is an error."""
+    """g950_py.so (native packing of a call's arguments), which belongs to the
+    torch it was built against.  No fallback: a missing library, or one of
+    another torch, is an error."""
     global _packer
     with _lib_lock:
         if _packer is None:
@@ -201,8 +202,16 @@ def _load_packer():
             import torch  # noqa: F401  (the extension resolves against torch's libraries)
             loader = importlib.machinery.ExtensionFileLoader("g950_py", str(PYLIB_PATH))
             spec = importlib.util.spec_from_file_location("g950_py", str(PYLIB_PATH), loader=loader)
-            mod = importlib.util.module_from_spec(spec)
-            loader.exec_module(mod)
+            try:
+                mod = importlib.util.module_from_spec(spec)
+                loader.exec_module(mod)
+                built = mod.torch_version
+            except (ImportError, AttributeError) as e:
+                raise G950Error(RESOURCE, f"{PYLIB_PATH} does not load with torch {torch.__version__}: {e} "
+                                "(run __graft_entry__.build() with the torch that is used)") from e
+            if not torch.__version__.startswith(built):
+                raise G950Error(RESOURCE, f"{PYLIB_PATH} was built against torch {built}, not {torch.__version__} "
+                                "(run __graft_entry__.build() with the torch that is used)")
             mod.init(Scalar, np.float32)
             _packer = mod
         return _packer
