@@ -63,6 +63,9 @@ namespace {
 
 thread_local std::string t_error;
 thread_local std::string t_kernel;
+// The form of the last launch (g950_last_form) and of the one to come: set
+// where a form is picked, taken over by launch().
+thread_local std::string t_form, t_next_form;
 // Set while a g950_launch_noalloc call is dispatched on this thread: the
 // device address of the module's scratch array, which then serves every
 // workspace request instead of hipMalloc.
@@ -225,6 +228,8 @@ hipFunction_t function(g950_module* m, const std::string& name) {
 template <class Args>
 int launch(g950_module* m, const std::string& name, unsigned grid, unsigned block, Args& args,
            void* stream) {
+  t_form.swap(t_next_form);
+  t_next_form.clear();
   if (!m) {  // validation only (g950_validate): report the choice, launch nothing
     t_kernel = name;
     return G950_OK;
@@ -690,6 +695,7 @@ int gemm_pick_tile(const g950_module* m, GemmArgs& g, int slabs, TileClass cls) 
     }
   }
   g.tile = pick->tile;
+  t_next_form = std::to_string(pick->bm) + "x" + std::to_string(pick->bn);
   return gemm_tiles(g, pick->bm, pick->bn);
 }
 
@@ -729,6 +735,7 @@ int launch_few_rows(g950_module* m, const char* name, GemmArgs& g, bool w8, void
   }
   form += g.tile;
   g.tile = form->t;
+  t_next_form = std::to_string(g.M <= 16 ? 16 : g.M <= 32 ? 32 : 64) + "x" + std::to_string(16 * form->t);
   return launch(m, name, (unsigned)blocks, (unsigned)(64 * form->waves), g, stream);
 }
 
@@ -1702,6 +1709,7 @@ int g950_open(const char* path, g950_module** out) {
 namespace {
 int dispatch(g950_module* m, uint32_t op, const g950_view* views, uint32_t nviews,
              const g950_scalar* scalars, uint32_t nscalars, void* stream) {
+  t_next_form.clear();
   t_kernel.clear();
   if ((!views && nviews) || (!scalars && nscalars)) return fail(G950_USAGE, "null argument");
   try {
@@ -1757,6 +1765,8 @@ int g950_validate(uint32_t op, const g950_view* views, uint32_t nviews, const g9
 }
 
 const char* g950_last_kernel(void) { return t_kernel.c_str(); }
+
+const char* g950_last_form(void) { return t_form.c_str(); }
 
 size_t g950_workspace_bytes(g950_module* m, void* stream) {
   if (!m) return 0;

@@ -43,7 +43,7 @@ DT_BOOL, DT_INT8, DT_UINT8, DT_INT16, DT_UINT16, DT_INT32 = 1, 2, 3, 4, 5, 6
 DT_UINT32, DT_INT64, DT_UINT64, DT_F16, DT_BF16, DT_F32, DT_F64 = 7, 8, 9, 10, 11, 12, 13
 
 EXPORTS = ("g950_open", "g950_launch", "g950_launch_noalloc", "g950_workspace_bytes", "g950_validate",
-           "g950_last_kernel", "g950_sync", "g950_strerror",
+           "g950_last_kernel", "g950_last_form", "g950_sync", "g950_strerror",
            "g950_last_error", "g950_close", "g950_bundle_open", "g950_bundle_check", "g950_bundle_reason",
            "g950_bundle_count", "g950_bundle_view", "g950_bundle_scalar", "g950_bundle_exec",
            "g950_bundle_close")
@@ -119,6 +119,7 @@ def load_library():
                                       ctypes.POINTER(Scalar), ctypes.c_uint32]
         lib.g950_validate.restype = ctypes.c_int
         lib.g950_last_kernel.restype = ctypes.c_char_p
+        lib.g950_last_form.restype = ctypes.c_char_p
         lib.g950_sync.argtypes = [ctypes.c_void_p]
         lib.g950_sync.restype = ctypes.c_int
         lib.g950_strerror.argtypes = [ctypes.c_int]

@@ -782,3 +782,33 @@ def test_gemm_negative_row_strides_leave_the_32_bit_kernels():
     assert kernel(mm, 300, 512, 1024, rev="b", col_b=False) == "g950_gemm_bf16_256x256"   # the copy's rows
     assert kernel(w8, 300, 512, 1024, rev="a", col_b=False) == "g950_gemm_w8a16_far_bf16_128x128"
     assert kernel(w8, 300, 512, 1024, rev="b", col_b=False) == "g950_gemm_bf16_256x256_rb"  # the copy's rows
+
+
+def test_gemm_tests_reach_every_form():
+    """The shapes that the GPU tests of the few-row and tiled GEMM kernels run
+    reach every form that one kernel symbol holds (256 CUs): rows x columns
+    per workgroup, with and without the one-instruction A of up to 8 (int8
+    weights: 4) rows."""
+    import test_gpu_few_rows as few
+    import test_gpu_gemm_tiles as tiles
+    lib = rt.load_library()
+
+    def form(op, dt, m, n, k, rb=False):
+        w8 = op == rt.OP_DEQUANT_MATMUL
+        a = Args().view([m, k], dt).view([k, n], rt.DT_INT8 if w8 else dt, strides=None if rb else [1, k])
+        if w8:
+            a = a.view([n], dt)
+        rc, _, err = validate(op, a.view([m, n], rt.DT_INT32 if dt == rt.DT_INT8 else dt, output=True), [k, m, n])
+        assert rc == 0, err
+        return lib.g950_last_form().decode()
+
+    for op, dt, per16 in ((rt.OP_MATMUL, rt.DT_BF16, 8), (rt.OP_MATMUL, rt.DT_F32, 4), (rt.OP_MATMUL_I8, rt.DT_INT8, 16)):
+        got = {(m <= 8, form(op, dt, m, n, per16 * c)) for m, n, c in few.SHAPES + few.SHAPES_FEW}
+        assert got == {(True, f"16x{16 * t}") for t in (1, 3, 4)} | {(False, f"16x{16 * t}") for t in (1, 3, 4)} | {
+            (False, f"{r}x{16 * t}") for r in (32, 64) for t in (1, 2, 4)}
+        got = {form(op, dt, m, n, k * (2 if per16 == 16 else 1)) for m, n, k in tiles.SHAPES if m > 64}
+        assert got == {"64x64", "64x128", "128x128", "256x256"}
+    got = {(m <= 4, form(rt.OP_DEQUANT_MATMUL, rt.DT_BF16, m, n, 16 * c)) for m, n, c in few.SHAPES + few.SHAPES_W8}
+    assert got == {(f, f"16x{16 * t}") for f in (True, False) for t in (1, 2, 3, 4)} | {
+        (False, f"32x{16 * t}") for t in (1, 2, 3)} | {(False, f"64x{16 * t}") for t in (1, 2)}
+    assert form(rt.OP_MATMUL, rt.DT_BF16, 256, 256, 96) == ""  # one form

@@ -23,9 +23,13 @@ TD = {"float32": torch.float32, "bfloat16": torch.bfloat16, "float16": torch.flo
 SHAPES = [(1, 1, 64), (4, 33, 65), (5, 47, 127), (8, 4097, 64), (9, 12300, 72), (16, 100, 300), (16, 6200, 70),
           (17, 70, 64), (32, 4100, 81), (31, 8200, 64), (33, 130, 90), (64, 4098, 64), (64, 8208, 73)]
 
+# the widest column groups with one DMA instruction of A (8 rows; int8 weights: 4)
+SHAPES_FEW = [(7, 12300, 72)]
+SHAPES_W8 = [(3, 20, 1), (16, 14400, 9), (32, 12300, 20), (4, 6200, 70), (2, 10000, 33), (3, 14400, 9), (1, 8192, 130)]
+
 
 @pytest.mark.parametrize("dt", ["bfloat16", "float16", "float32", "int8"])
-@pytest.mark.parametrize("m,n,chunks", SHAPES)
+@pytest.mark.parametrize("m,n,chunks", SHAPES + SHAPES_FEW)
 def test_few_rows(m, n, chunks, dt):
     rng = np.random.default_rng(m + 3 * n + 7 * chunks)
     k = chunks * {"float32": 4, "int8": 16}.get(dt, 8)
@@ -57,7 +61,7 @@ def test_few_rows(m, n, chunks, dt):
 
 
 @pytest.mark.parametrize("dt", ["bfloat16", "float16"])
-@pytest.mark.parametrize("m,n,chunks", SHAPES + [(3, 20, 1), (16, 14400, 9), (32, 12300, 20)])
+@pytest.mark.parametrize("m,n,chunks", SHAPES + SHAPES_W8)
 def test_few_rows_int8_weights(m, n, chunks, dt):
     rng = np.random.default_rng(m + n + chunks)
     k = 16 * chunks
