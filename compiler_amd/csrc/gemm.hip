@@ -748,9 +748,11 @@ constexpr int W8_LDS = 144 * 1024;  // of the tiled int8-weight kernels
 // tiles).  The slabs run through a ring of NST stages filled by direct DMA,
 // every wave issuing its share: NST - 1 slabs are in flight, since with few
 // MFMAs per slab the latency of a load, not its issue, is what a two-stage
-// ring would show.  What bounds it is the CU's load path (16, 24 or 32 KB per
-// slab at about 70 bytes per ns): bf16 512 x 4096 x 4096 68 -> 26 us (64 x 128
-// tiles, one per CU), 256 x 4096 x 4096 68 -> 16, 1000 x 4096 x 4096 68 -> 39,
+// ring would show.  What bounds it is loading 16, 24 or 32 KB per slab: all
+// three tiles run at about 70 bytes per ns and CU with about 100 KB in flight,
+// which a latency of 1.4 us explains as well as a limit of the path (the two
+// were not told apart).  bf16 512 x 4096 x 4096 68 -> 26 us (64 x 128 tiles,
+// one per CU), 256 x 4096 x 4096 68 -> 16, 1000 x 4096 x 4096 68 -> 39,
 // int8 512 x 8192 x 8192 70 -> 40, fp32 512 x 2048 x 2048 452 -> 40 (operands
 // in the MALL).  fp32 sums in two chains: error against 64 bits at 512 x 2048
 // x 4096 1.14e-6 -> 8.1e-7.  Iteration kt multiplies slab kt from registers while slab
@@ -761,10 +763,10 @@ constexpr int W8_LDS = 144 * 1024;  // of the tiled int8-weight kernels
 //
 // W8 (int8 weights under 16-bit A): a slab is 128 k -- 256 bytes of an A row,
 // 128 of a B row -- and a lane's 16 weights are widened as they leave LDS,
-// for two MFMAs; B then costs half the load path's bytes.  K need only be a
+// for two MFMAs; B then costs half the bytes.  K need only be a
 // multiple of 16: the last slab's chunks past K repeat the row's last one and
 // are zeroed in registers.  The column scale is the epilogue's.  It is bound
-// by the load path like the others: 512 x 4096 x 4096 30 us, 256 x 4096 x
+// by its loads like the others: 512 x 4096 x 4096 30 us, 256 x 4096 x
 // 4096 22 and 1024 x 8192 x 8192 153, against 102, 102 and 186 for the 128 x
 // 128 kernel it replaced (operands staged through registers, one slab ahead).
 //
@@ -1456,11 +1458,11 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
     const int u = start + wave + W * j;
     return SPREAD && u >= units ? u - units : u;
   };
-  auto issue = [&](int j) {
+  auto issue = [&](int j, int slot) {
     const int unit = unit_of(j);
     const char* as = abase + (long long)unit * AROW;
     const char* bs = bbase + (long long)unit * 128;
-    const uint32_t dst = ring32 + (uint32_t)(j % NS) * UNIT;
+    const uint32_t dst = ring32 + (uint32_t)slot * UNIT;
     if (unit == units - 1 && tb != 128) {
       // chunks past K repeat the row's last one (zeroed as they are used)
 #pragma unroll
@@ -1484,12 +1486,14 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
       if constexpr (MODE == GEMM_I8) aci[r][t] = (i32x4){};
       else acf[r][t] = (f32x4){};
     }
-  for (int j = 0; j < NS && j < nloc; ++j) issue(j);
-  for (int j = 0; j < nloc; ++j) {
+  for (int j = 0; j < NS && j < nloc; ++j) issue(j, j);
+  // unit j lies in slot j % NS, counted along (the remainder by 3 cost one row
+  // of A with int8 weights up to a fifth: 432 x 28672 21.2 -> 17.1 us)
+  for (int j = 0, slot = 0; j < nloc; ++j, slot = slot + 1 == NS ? 0 : slot + 1) {
     // unit j has landed once at most the later units' loads are in flight
     if (j + NS <= nloc) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * DPU) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const char* st = ring + (j % NS) * UNIT;
+    const char* st = ring + slot * UNIT;
     const bool tail = unit_of(j) == units - 1 && tb != 128;
     u32x4 av[2][R][W8 ? 2 : 1], bv[2][T];
 #pragma unroll
@@ -1518,7 +1522,7 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, char* lds) {
     }
     // the unit's reads have returned before its slot is refilled
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    if (j + NS < nloc) issue(j + NS);
+    if (j + NS < nloc) issue(j + NS, slot);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
