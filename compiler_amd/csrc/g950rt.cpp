@@ -346,6 +346,7 @@ int launch_split_rows(g950_module* m, const char* op, RowArgs& a, uint32_t dt, i
   snprintf(name, sizeof name, "g950_rs_part_%s_%s_v%d", op, rr_dtype(dt), v);
   if (int rc = launch(m, name, (unsigned)blocks, 256u, a, stream)) return rc;
   snprintf(name, sizeof name, "g950_rs_final_%s_%s_v%d", op, rr_dtype(dt), v);
+  if (v == 1) t_next_form = a.masked ? "vectors" : "elements";
   const bool lse = strcmp(op, "logsumexp") == 0;
   return launch(m, name, (unsigned)(lse ? a.rows : blocks), 256u, a, stream);
 }
@@ -418,7 +419,14 @@ int launch_rows(g950_module* m, const char* op, RowArgs& a, uint32_t dt, const V
     return launch(m, name, row_grid(m, a.rows, pick->block, pick->waves), (unsigned)pick->block, a,
                   stream);
   }
-  a.masked = !vec && phase;
+  // masked vectors or elements (chunks of 1024 either way): a few elements per
+  // thread spread a small call over more workgroups, so vectors only past four
+  // workgroups of elements per CU, six where a weight and a bias come with
+  // them.  Measured on MI355X (us, vectors / elements): bf16 softmax 4 x 68389
+  // 7.4 / 6.3, 20 x 50001 7.4 / 7.1, 40 x 50001 7.8 / 9.1; LayerNorm 4 x 68389
+  // 8.9 / 6.7, 120 x 10111 9.5 / 7.8, 40 x 50001 10.3 / 10.6, 80 x 50001 11.6 /
+  // 16.7; fp32 softmax 40 x 50001 8.1 / 9.2.
+  a.masked = !vec && phase && (long long)a.rows * ((a.cols + 1023ll) / 1024) > (p1 ? 6 : 4) * cus;
   return launch_split_rows(m, op, a, dt, v, stream);
 }
 
@@ -661,10 +669,10 @@ bool rows_off32(long long rows, int tile, long long s0, int esz, int part = 256)
 
 // Workgroup tile of a whole-slab MFMA GEMM (GemmArgs::tile) and its tile
 // count: the least of rounds x (slabs x slab time + fixed time), a round
-// being one workgroup per CU.  Smaller tiles cost more per output (a CU's
-// load path moves 70 bytes per ns whatever the tile, and a 64 x 64 tile needs
-// four times the bytes of a 256 x 256 one per output) but fill the chip where
-// the larger would leave CUs idle.  Slab times in us, measured on MI355X with
+// being one workgroup per CU.  Smaller tiles cost more per output (a CU takes
+// in about 70 bytes per ns whatever the tile, and a 64 x 64 tile needs four
+// times the bytes of a 256 x 256 one per output) but fill the chip where the
+// larger would leave CUs idle.  Slab times in us, measured on MI355X with
 // operands from HBM: bf16 M x 4096 x 4096 (64 slabs, each CU at most one
 // tile) 256x256 92-95 us, 128x128 40-43, 64x128 31, 64x64 22; 4096 x 11008 x
 // 512 to 8192 x 8192 x 1536 follow within 10%.  Both sides of a line, bf16:

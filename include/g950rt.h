@@ -253,9 +253,10 @@ int g950_validate(uint32_t op, const g950_view *views, uint32_t nviews,
  * ran (for profiling and tests); empty string if none. */
 const char *g950_last_kernel(void);
 
-/* Outputs per workgroup, "rows x columns" (as "64x128"), of that launch where
- * one kernel symbol holds several forms: the tiled GEMM kernels of whole
- * slabs and the few-row ones.  Empty string for all others. */
+/* The form of that launch where one kernel symbol holds several: outputs per
+ * workgroup, "rows x columns" (as "64x128"), for the tiled GEMM kernels of
+ * whole slabs and the few-row ones; "vectors" or "elements" for the _v1 split
+ * row kernels.  Empty string for all others. */
 const char *g950_last_form(void);
 
 /* Wait for all work on `stream`. */

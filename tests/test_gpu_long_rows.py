@@ -42,9 +42,11 @@ def host(t):
 
 SHAPES = {  # rows, cols, extra stride, kernel prefix
     "float32": [(130, 2049, 1, "rl"), (140, 4089, 0, "rl"), (129, 4097, 3, "rl"), (128, 8191, 0, "rl"),
-                (131, 32761, 2, "rl"), (3, 20001, 1, "rs"), (2, 70001, 0, "rs")],
+                (131, 32761, 2, "rl"), (3, 20001, 1, "rs"), (2, 70001, 0, "rs"), (101, 17001, 1, "rs"),
+                (2, 800001, 0, "rs")],
     "bfloat16": [(5, 4097, 0, "rl"), (130, 8185, 1, "rl"), (128, 8193, 6, "rl"), (129, 16379, 0, "rl"),
-                 (128, 50001, 0, "rl"), (128, 65521, 3, "rl"), (3, 40001, 1, "rs"), (2, 140001, 0, "rs")],
+                 (128, 50001, 0, "rl"), (128, 65521, 3, "rl"), (3, 40001, 1, "rs"), (2, 140001, 0, "rs"),
+                 (61, 40001, 0, "rs"), (2, 800001, 1, "rs")],
 }
 SHAPES["float16"] = SHAPES["bfloat16"][1::2]
 
@@ -62,6 +64,10 @@ def test_long_odd_rows(dt, shape):
         assert ok, (rt.module().last_kernel, err)
         name = rt.module().last_kernel
         assert name.startswith(f"g950_{kind}_") and "_v1" in name, name
+        if kind == "rs":
+            limit = 256 * (6 if "layernorm" in name else 4)
+            many = rows * -(-cols // 1024) > limit
+            assert rt.load_library().g950_last_form() == (b"vectors" if many else b"elements"), name
 
     full, y = guarded(rows, cols, stride, dt)
     ops.softmax_kernel(x, y, cols, sync=True)
@@ -89,10 +95,12 @@ def test_long_odd_rows(dt, shape):
 # rows whose vectors fill their chunks exactly at some phases and reach one
 # vector further at others (chunks of 1024 vectors): the last chunk is empty
 # for part of the rows
-@pytest.mark.parametrize("dt,cols", [("bfloat16", 8186), ("bfloat16", 8190), ("bfloat16", 16383), ("float16", 8192),
-                                     ("float32", 4095), ("float32", 4094), ("float32", 12287)])
-def test_split_rows_last_chunk_empty(dt, cols):
-    rows, stride = 9, cols + 1
+@pytest.mark.parametrize("dt,cols,rows", [("bfloat16", 8186, 9), ("bfloat16", 8190, 9), ("bfloat16", 16383, 9),
+                                          ("float16", 8192, 9), ("float32", 4095, 9), ("float32", 4094, 9),
+                                          ("float32", 12287, 9), ("bfloat16", 16378, 126), ("bfloat16", 16383, 126),
+                                          ("float16", 24575, 126), ("float32", 16381, 126), ("float32", 16383, 126)])
+def test_split_rows_last_chunk_empty(dt, cols, rows):
+    stride = cols + 1
     x, w, b = case(rows, cols, stride, dt, cols)
     _, y = guarded(rows, cols, stride, dt)
     xr, wr, br = host(x), host(w), host(b)
@@ -100,6 +108,8 @@ def test_split_rows_last_chunk_empty(dt, cols):
     mean, rstd = torch.empty(rows, device=DEV), torch.empty(rows, device=DEV)
     ops.layernorm_kernel(x, y, w, b, mean, rstd, stride, cols, 1e-5, sync=True)
     assert rt.module().last_kernel.startswith("g950_rs_final_layernorm") and "_v1" in rt.module().last_kernel
+    # (few rows run by elements; only vectors can leave a chunk empty)
+    assert rt.load_library().g950_last_form() == (b"elements" if rows == 9 else b"vectors")
     want = ref.layernorm(xr, wr, br, 1e-5)
     ln_bar = bar if dt != "float32" else (1e-5, 1e-5)
     for got, exp, (rtol, atol) in zip((host(y), mean.cpu().numpy(), rstd.cpu().numpy()), want,
