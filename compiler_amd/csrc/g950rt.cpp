@@ -425,8 +425,10 @@ int launch_rows(g950_module* m, const char* op, RowArgs& a, uint32_t dt, const V
   // them.  Measured on MI355X (us, vectors / elements): bf16 softmax 4 x 68389
   // 7.4 / 6.3, 20 x 50001 7.4 / 7.1, 40 x 50001 7.8 / 9.1; LayerNorm 4 x 68389
   // 8.9 / 6.7, 120 x 10111 9.5 / 7.8, 40 x 50001 10.3 / 10.6, 80 x 50001 11.6 /
-  // 16.7; fp32 softmax 40 x 50001 8.1 / 9.2.
-  a.masked = !vec && phase && (long long)a.rows * ((a.cols + 1023ll) / 1024) > (p1 ? 6 : 4) * cus;
+  // 16.7; fp32 softmax 40 x 50001 8.1 / 9.2.  Not up to the last of 2^31
+  // columns, where a vector's position past the row's end would overflow.
+  a.masked = !vec && phase && a.cols <= 0x7FFFFFFF - 16384 &&
+             (long long)a.rows * ((a.cols + 1023ll) / 1024) > (p1 ? 6 : 4) * cus;
   return launch_split_rows(m, op, a, dt, v, stream);
 }
 

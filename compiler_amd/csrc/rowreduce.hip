@@ -757,8 +757,10 @@ __device__ __forceinline__ void rm_body(const RowArgs& a) {
 // How a masked kernel's vectors meet a row of `cols` elements whose start
 // lies ph elements past a 16-byte boundary: vector j holds columns j*VEC - ph
 // .. + VEC - 1.  (The rules of rm_body, for vectors spread over a workgroup.)
-// Positions from that boundary count unsigned: a row may hold 2^31 - 1
-// columns, and the last chunk's vectors lie up to 8192 elements past its end.
+// Positions are 32-bit: the last chunk's vectors lie up to 8192 elements past
+// the row's end, so the host gives masked rows at most 2^31 - 16385 columns
+// (positions that reach further cost registers: rl softmax of 16 vectors a
+// thread spilled and ran 663 x 61856 fp32 in 70.5 us for 65.4).
 template <typename T, int VEC>
 struct MaskedRow {
   using IO = RawIO<T, VEC>;
@@ -771,13 +773,10 @@ struct MaskedRow {
     lo = (char*)(at & ~(uintptr_t)15);
     cols = n;
   }
-  __device__ __forceinline__ uint32_t at(int j) const { return (uint32_t)j * VEC; }
-  __device__ __forceinline__ uint32_t end() const { return (uint32_t)cols + (uint32_t)ph; }
-  __device__ __forceinline__ long long col(int j) const { return (long long)at(j) - ph; }
-  __device__ __forceinline__ bool live(int j) const { return at(j) < end(); }
-  __device__ __forceinline__ bool whole(int j) const { return at(j) >= (uint32_t)ph && at(j) + VEC <= end(); }
-  // (an element before the row wraps to past its end)
-  __device__ __forceinline__ bool ok(int j, int e) const { return at(j) + e - (uint32_t)ph < (uint32_t)cols; }
+  __device__ __forceinline__ int col(int j) const { return j * VEC - ph; }
+  __device__ __forceinline__ bool live(int j) const { return col(j) < cols; }
+  __device__ __forceinline__ bool whole(int j) const { return col(j) >= 0 && col(j) + VEC <= cols; }
+  __device__ __forceinline__ bool ok(int j, int e) const { return col(j) + e >= 0 && col(j) + e < cols; }
   // elements of a live vector, those outside the row as `ident`
   __device__ __forceinline__ void unpack(const R& r, int j, float ident, float* v) const {
     IO::unpack(r, v);
@@ -800,7 +799,7 @@ struct MaskedRow {
   __device__ __forceinline__ void params(const void* base, int j, float* w) const {
     typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
     if (whole(j)) {
-      const u32x4_any t = *(const u32x4_any*)((const char*)base + col(j) * (long long)sizeof(T));
+      const u32x4_any t = *(const u32x4_any*)((const char*)base + (long long)col(j) * (long long)sizeof(T));
       IO::unpack(__builtin_bit_cast(R, (u32x4){t[0], t[1], t[2], t[3]}), w);
     } else {
 #pragma unroll
@@ -1037,10 +1036,11 @@ __device__ __forceinline__ void rs_part_body(const RowArgs& a, float* scratch) {
     p[0] = block_reduce<OpSum, RS_BLOCK>(s, scratch);
     p[1] = block_reduce<OpSum, RS_BLOCK>(q, scratch);
   } else {
-    const long long first = (long long)split * (RS_BLOCK * RS_ITEMS * VEC) - (MASKED ? x.ph : 0);
+    const int first = split * (RS_BLOCK * RS_ITEMS * VEC) - (MASKED ? x.ph : 0);
     // (the host counts a masked row's vectors at its worst phase, so the last
     // chunk may hold no element: weight 0 and, not 0 / 0, mean 0)
-    const float n = (float)max(min(first + RS_BLOCK * RS_ITEMS * VEC, (long long)a.cols) - max(first, 0ll), 0ll);
+    // (a.cols - first, not first + chunk: no overflow at the most columns)
+    const float n = (float)max(min(RS_BLOCK * RS_ITEMS * VEC, a.cols - first) - max(-first, 0), 0);
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < RS_ITEMS; ++i)

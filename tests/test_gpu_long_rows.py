@@ -149,15 +149,17 @@ def test_long_rows_packed(rows, cols):
     assert ok, err
 
 
-# the most columns a row may have, at two 16-byte phases, and (y one element
-# off x's phase) by element loads
-@pytest.mark.parametrize("offset,y_offset", [(0, 0), (3, 3), (0, 1)])
-def test_split_rows_of_the_most_columns(offset, y_offset):
+# the most columns a row may have, and the most that vectors take (at two
+# 16-byte phases; y one element off x's phase: elements)
+@pytest.mark.parametrize("n,offset,y_offset", [(2**31 - 1, 3, 3), (2**31 - 16385, 0, 0), (2**31 - 16385, 3, 3),
+                                               (2**31 - 16385, 0, 1), (2**31 - 9001, 0, 0)])
+def test_split_rows_of_the_most_columns(n, offset, y_offset):
     """Columns up to 2^31 - 1: the last chunk counts (its values alone set the
     variance and the logsumexp) and no vector past the row is read.  Four
     buffers of 4.3 GB.  LayerNorm bf16: the statistics within 1e-4 (fp32 sums of 2^31
     terms in chunks), y within bf16 rounding."""
-    n, pad, tail, big = 2**31 - 1, 16, 4000, 1024.0
+    pad, tail, big = 16, 4000, 1024.0
+    vectors = n <= 2**31 - 16385 and offset == y_offset
     g = torch.Generator(device="cuda").manual_seed(1)
     xs = torch.empty(n + pad, dtype=torch.bfloat16, device="cuda")
     for c in xs.split(1 << 28):
@@ -172,6 +174,7 @@ def test_split_rows_of_the_most_columns(offset, y_offset):
     b = torch.zeros(n, dtype=torch.bfloat16, device="cuda")
     _, m, r = ops.layernorm(x, w, b, 1e-5, out=y, sync=True)
     assert rt.module().last_kernel == "g950_rs_final_layernorm_bf16_v1"
+    assert rt.load_library().g950_last_form() == (b"vectors" if vectors else b"elements")
     rstd = (var + 1e-5) ** -0.5
     assert abs(m.item() - mean) < 1e-4 and abs(r.item() / rstd - 1) < 1e-4
     for xc, yc in zip(x[0].split(1 << 27), y[0].split(1 << 27)):
