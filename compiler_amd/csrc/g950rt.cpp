@@ -395,12 +395,26 @@ int launch_rows(g950_module* m, const char* op, RowArgs& a, uint32_t dt, const V
   // against the split pair (us): softmax bf16 [256, 50001] 41.9 -> 14.1,
   // aligned [512, 65536] 33.5 -> 30.2, LayerNorm bf16 [4555, 5001] 79.3 ->
   // 27.3; logsumexp bf16 [512, 100000] 21.1 split, 30.0 as one workgroup.
+  // Workgroups of 1024 threads run one per CU, so past one round a last round
+  // that leaves too many CUs idle costs more than reading x twice: at least
+  // 7/8 (softmax and LayerNorm of 16 bits) or 3/4 (fp32 and RMSNorm) of the
+  // rounds must be filled.  Time against the split pair at 262 / 400 / 450 / 512 / 700 / 786 rows: softmax bf16 x
+  // 50000 1.47 / 1.02 / 0.95 / 0.92 / 1.00 / 1.13, LayerNorm bf16 x 33024 1.41
+  // / 1.15 / 1.03 / 0.97 / 1.05 / 1.21, softmax fp32 x 25000 1.28 / 0.93 / 0.88
+  // / 0.87 / 0.90 / 1.02, RMSNorm bf16 x 50000 1.20 / 0.89 / 0.84 / 0.86 / 0.89
+  // / 0.97.  Within the first round it stays ahead down to 128 rows (0.82 to
+  // 1.08) but for softmax past 8192 vectors (x 100000: 1.33 at 128 rows, 0.98
+  // at 180).
+  const long long rounds = (a.rows + cus - 1) / cus;
+  const bool lean = isz == 4 || !strcmp(op, "rmsnorm");
+  const bool filled = rounds == 1 || 8ll * a.rows >= (lean ? 6 : 7) * rounds * cus;
   if (phase && !few && (!vec || !pick)) {
     static const struct { int items, block; } kRl[] = {{4, 256}, {8, 256}, {8, 1024}, {16, 1024}};
     const int forms = !strcmp(op, "softmax") ? 4 : !strcmp(op, "logsumexp") ? 2 : 3;
     for (int f = 0; f < forms; ++f) {
       const auto& c = kRl[f];
       if (mvec > (long long)c.items * c.block) continue;
+      if (c.block == 1024 && !filled) break;
       snprintf(name, sizeof name, "g950_rl_%s_%s_v1_i%d_b%d", op, rr_dtype(dt), c.items, c.block);
       return launch(m, name, (unsigned)a.rows, (unsigned)c.block, a, stream);
     }

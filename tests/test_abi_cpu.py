@@ -812,3 +812,25 @@ def test_gemm_tests_reach_every_form():
     assert got == {(f, f"16x{16 * t}") for f in (True, False) for t in (1, 2, 3, 4)} | {
         (False, f"32x{16 * t}") for t in (1, 2, 3)} | {(False, f"64x{16 * t}") for t in (1, 2)}
     assert form(rt.OP_MATMUL, rt.DT_BF16, 256, 256, 96) == ""  # one form
+
+
+@pytest.mark.parametrize("rows,cols,dtype,op,kernel", [
+    (256, 50000, rt.DT_BF16, "softmax", "g950_rl_softmax_bf16_v1_i8_b1024"),     # one full round of the CUs
+    (262, 50000, rt.DT_BF16, "softmax", "g950_rs_final_softmax_bf16_v8"),        # a second round of 6
+    (447, 50000, rt.DT_BF16, "softmax", "g950_rs_final_softmax_bf16_v8"),
+    (448, 50000, rt.DT_BF16, "softmax", "g950_rl_softmax_bf16_v1_i8_b1024"),     # 7/8 of two rounds
+    (300, 50001, rt.DT_F16, "softmax", "g950_rs_final_softmax_f16_v1"),          # odd rows alike
+    (383, 32768, rt.DT_F32, "softmax", "g950_rs_final_softmax_f32_v4"),
+    (384, 32768, rt.DT_F32, "softmax", "g950_rl_softmax_f32_v1_i8_b1024"),       # 3/4 in fp32
+    (786, 56688, rt.DT_BF16, "layernorm", "g950_rs_final_layernorm_bf16_v8"),
+    (1000, 56688, rt.DT_BF16, "layernorm", "g950_rl_layernorm_bf16_v1_i8_b1024"),
+    (300, 15001, rt.DT_BF16, "softmax", "g950_rl_softmax_bf16_v1_i8_b256"),      # several per CU: no rounds
+])
+def test_long_rows_fill_their_last_round(rows, cols, dtype, op, kernel):
+    if op == "softmax":
+        rc, name, err = validate(rt.OP_SOFTMAX, softmax_args(rows, cols, dtype), [cols])
+    else:
+        a = (Args().view([cols], dtype).view([rows], rt.DT_F32, output=True).view([rows], rt.DT_F32, output=True)
+             .view([cols], dtype).view([rows, cols], dtype).view([rows, cols], dtype, output=True))
+        rc, name, err = validate(rt.OP_LAYERNORM, a, [cols, (1e-5, "float32"), cols])
+    assert rc == 0 and name == kernel, err

@@ -43,10 +43,10 @@ def host(t):
 SHAPES = {  # rows, cols, extra stride, kernel prefix
     "float32": [(130, 2049, 1, "rl"), (140, 4089, 0, "rl"), (129, 4097, 3, "rl"), (128, 8191, 0, "rl"),
                 (131, 32761, 2, "rl"), (3, 20001, 1, "rs"), (2, 70001, 0, "rs"), (101, 17001, 1, "rs"),
-                (2, 800001, 0, "rs")],
+                (2, 800001, 0, "rs"), (262, 9001, 0, "rs"), (390, 8201, 1, "rl")],
     "bfloat16": [(5, 4097, 0, "rl"), (130, 8185, 1, "rl"), (128, 8193, 6, "rl"), (129, 16379, 0, "rl"),
                  (128, 50001, 0, "rl"), (128, 65521, 3, "rl"), (3, 40001, 1, "rs"), (2, 140001, 0, "rs"),
-                 (61, 40001, 0, "rs"), (2, 800001, 1, "rs")],
+                 (61, 40001, 0, "rs"), (262, 17001, 1, "rs"), (2, 800001, 1, "rs"), (449, 16401, 0, "rl")],
 }
 SHAPES["float16"] = SHAPES["bfloat16"][1::2]
 
