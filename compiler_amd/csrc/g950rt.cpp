@@ -65,7 +65,7 @@ thread_local std::string t_error;
 thread_local std::string t_kernel;
 // The form of the last launch (g950_last_form) and of the one to come: set
 // where a form is picked, taken over by launch().
-thread_local std::string t_form, t_next_form;
+thread_local const char *t_form = "", *t_next_form = "";
 // Set while a g950_launch_noalloc call is dispatched on this thread: the
 // device address of the module's scratch array, which then serves every
 // workspace request instead of hipMalloc.
@@ -228,8 +228,8 @@ hipFunction_t function(g950_module* m, const std::string& name) {
 template <class Args>
 int launch(g950_module* m, const std::string& name, unsigned grid, unsigned block, Args& args,
            void* stream) {
-  t_form.swap(t_next_form);
-  t_next_form.clear();
+  t_form = t_next_form;
+  t_next_form = "";
   if (!m) {  // validation only (g950_validate): report the choice, launch nothing
     t_kernel = name;
     return G950_OK;
@@ -702,11 +702,11 @@ enum TileClass { TILES_16 = 0, TILES_F32 = 1, TILES_W8 = 2 };
 
 int gemm_pick_tile(const g950_module* m, GemmArgs& g, int slabs, TileClass cls) {
   const long long cus = m ? m->cus : 256;
-  static const struct { int tile, bm, bn; double slab[3], fixed; } kTiles[] = {
-      {GEMM_TILE_256x256, 256, 256, {1.42, 7.0, 0.0}, 4.0},  // (no such tile for int8 weights)
-      {GEMM_TILE_128x128, 128, 128, {0.59, 1.95, 1.25}, 3.0},
-      {GEMM_TILE_64x128, 64, 128, {0.44, 1.06, 0.86}, 3.0},
-      {GEMM_TILE_64x64, 64, 64, {0.31, 0.58, 0.60}, 2.5}};
+  static const struct { int tile, bm, bn; const char* form; double slab[3], fixed; } kTiles[] = {
+      {GEMM_TILE_256x256, 256, 256, "256x256", {1.42, 7.0, 0.0}, 4.0},  // (no such tile for int8 weights)
+      {GEMM_TILE_128x128, 128, 128, "128x128", {0.59, 1.95, 1.25}, 3.0},
+      {GEMM_TILE_64x128, 64, 128, "64x128", {0.44, 1.06, 0.86}, 3.0},
+      {GEMM_TILE_64x64, 64, 64, "64x64", {0.31, 0.58, 0.60}, 2.5}};
   const auto* pick = &kTiles[1];
   double best = HUGE_VAL;
   for (const auto& t : kTiles) {
@@ -719,7 +719,7 @@ int gemm_pick_tile(const g950_module* m, GemmArgs& g, int slabs, TileClass cls) 
     }
   }
   g.tile = pick->tile;
-  t_next_form = std::to_string(pick->bm) + "x" + std::to_string(pick->bn);
+  t_next_form = pick->form;
   return gemm_tiles(g, pick->bm, pick->bn);
 }
 
@@ -759,7 +759,10 @@ int launch_few_rows(g950_module* m, const char* name, GemmArgs& g, bool w8, void
   }
   form += g.tile;
   g.tile = form->t;
-  t_next_form = std::to_string(g.M <= 16 ? 16 : g.M <= 32 ? 32 : 64) + "x" + std::to_string(16 * form->t);
+  static const char* const kForms[3][4] = {{"16x16", "16x32", "16x48", "16x64"},
+                                           {"32x16", "32x32", "32x48", "32x64"},
+                                           {"64x16", "64x32", "64x48", "64x64"}};
+  t_next_form = kForms[g.M <= 16 ? 0 : g.M <= 32 ? 1 : 2][form->t - 1];
   return launch(m, name, (unsigned)blocks, (unsigned)(64 * form->waves), g, stream);
 }
 
@@ -1733,7 +1736,7 @@ int g950_open(const char* path, g950_module** out) {
 namespace {
 int dispatch(g950_module* m, uint32_t op, const g950_view* views, uint32_t nviews,
              const g950_scalar* scalars, uint32_t nscalars, void* stream) {
-  t_next_form.clear();
+  t_next_form = "";
   t_kernel.clear();
   if ((!views && nviews) || (!scalars && nscalars)) return fail(G950_USAGE, "null argument");
   try {
@@ -1790,7 +1793,7 @@ int g950_validate(uint32_t op, const g950_view* views, uint32_t nviews, const g9
 
 const char* g950_last_kernel(void) { return t_kernel.c_str(); }
 
-const char* g950_last_form(void) { return t_form.c_str(); }
+const char* g950_last_form(void) { return t_form; }
 
 size_t g950_workspace_bytes(g950_module* m, void* stream) {
   if (!m) return 0;
