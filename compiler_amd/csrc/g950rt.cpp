@@ -322,6 +322,24 @@ int workspace(g950_module* m, void* stream, size_t bytes, void** out, bool optio
   return G950_OK;
 }
 
+// Whether workspace() can serve `bytes` on `stream`: a stream under capture
+// cannot allocate, so it has what it holds.
+bool workspace_at_hand(g950_module* m, void* stream, size_t bytes) {
+  if (!m) return true;
+  if (t_scratch) return bytes <= kScratchWorkspace;
+  {
+    std::lock_guard<std::mutex> lock(m->ws_mu);
+    const auto it = m->ws.find(stream);
+    if (it != m->ws.end() && it->second.second >= bytes) return true;
+  }
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st == hipStreamCaptureStatusNone;
+}
+
 template <class Args>
 int launch(g950_module* m, const std::string& name, unsigned grid, unsigned block, Args& args, void* stream);
 
@@ -404,7 +422,8 @@ int launch_rows(g950_module* m, const char* op, RowArgs& a, uint32_t dt, const V
   // / 0.87 / 0.90 / 1.02, RMSNorm bf16 x 50000 1.20 / 0.89 / 0.84 / 0.86 / 0.89
   // / 0.97.  Within the first round it stays ahead down to 128 rows (0.82 to
   // 1.08) but for softmax past 8192 vectors (x 100000: 1.33 at 128 rows, 0.98
-  // at 180).
+  // at 180).  A stream under capture that has no room for the split pair's
+  // records takes one workgroup per row, which needs none.
   const long long rounds = (a.rows + cus - 1) / cus;
   const bool lean = isz == 4 || !strcmp(op, "rmsnorm");
   const bool filled = rounds == 1 || 8ll * a.rows >= (lean ? 6 : 7) * rounds * cus;
@@ -414,7 +433,7 @@ int launch_rows(g950_module* m, const char* op, RowArgs& a, uint32_t dt, const V
     for (int f = 0; f < forms; ++f) {
       const auto& c = kRl[f];
       if (mvec > (long long)c.items * c.block) continue;
-      if (c.block == 1024 && !filled) break;
+      if (c.block == 1024 && !filled && workspace_at_hand(m, stream, (size_t)a.rows * ((mvec + 1023) / 1024) * 16)) break;
       snprintf(name, sizeof name, "g950_rl_%s_%s_v1_i%d_b%d", op, rr_dtype(dt), c.items, c.block);
       return launch(m, name, (unsigned)a.rows, (unsigned)c.block, a, stream);
     }

@@ -188,3 +188,34 @@ def test_split_rows_of_the_most_columns(n, offset, y_offset):
         lse = ops.logsumexp(x, sync=True)
         assert rt.module().last_kernel == "g950_rs_final_logsumexp_bf16_v1"
         assert abs(lse.item() - 40.0) < 1e-3  # log(e^40 + 2^31 e^0.5): 1.5e-8 past 40
+
+
+def test_poorly_filled_rounds_under_capture():
+    """262 rows run the split pair; captured on a stream that holds no
+    workspace (nothing can be allocated there) one workgroup per row, on one
+    that does the split pair again.  Every replay gives the eager result (fp32
+    exponentials and sums in another order: 2e-5)."""
+    x = torch.randn(262, 33000, device=DEV)
+    want = torch.softmax(x, -1)
+    y = torch.empty_like(x)
+    torch.cuda.synchronize()
+    for warm in (False, True):
+        stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        if warm:
+            with torch.cuda.stream(stream):
+                ops.softmax_kernel(x, y, 33000, sync=True)
+            assert rt.module().last_kernel == "g950_rs_final_softmax_f32_v4"
+        held = rt.module().workspace_bytes(stream)
+        with torch.cuda.graph(graph, stream=stream):
+            ops.softmax_kernel(x, y, 33000)
+        if held:
+            assert rt.module().last_kernel == "g950_rs_final_softmax_f32_v4"
+        else:
+            assert rt.module().last_kernel == "g950_rl_softmax_f32_v1_i16_b1024"
+        assert rt.module().workspace_bytes(stream) == held
+        for _ in range(3):
+            y.fill_(7.0)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.allclose(y, want, rtol=2e-5, atol=0)
