@@ -1505,8 +1505,8 @@ void* optional_workspace(g950_module* m, void* stream, size_t bytes) {
 // into range 0 and run 71 against 60.
 // Without the workspace (captured graphs, no-alloc calls, a failed
 // allocation) one workgroup per pair takes the ranges in turn, for the same
-// bits: one sequence of 8192 keys 127 against 13.2, 32 of 4096..300 74 against
-// 60, 64 of 2048 95 against 100.  (One range instead takes 84, 67 and 94, but
+// bits: one sequence of 8192 keys 121 against 13.2, 32 of 4096..300 72 against
+// 61, 64 of 2048 95 against 100.  (One range instead takes 84, 67 and 94, but
 // rounds the probabilities against other maxima.)
 constexpr long long kDecTarget = 4, kDecMinKeys = 256, kDecOneRange = 512;
 

@@ -1406,9 +1406,10 @@ __device__ __forceinline__ void widen_i8_body(const GemmArgs& p) {
 // golden ratio's multiples spread them evenly) and wraps round: where all
 // workgroups walk K in step, rows of 8 KiB or so keep them on the same few
 // HBM channels.  One row of A, from 0 -> spread (us; the kernel that loaded
-// operands into registers, each wave its own part of K): 4096 x 11008 14.5 ->
-// 12.0 (13.1), 8192 x 22016 43.4 -> 32.6 (38.0), 16384 x 8192 29.9 -> 25.8
-// (26.4), 4096 x 8192 10.0 -> 9.8 (9.0).
+// operands into registers, each wave its own part of K): 4096 x 11008 14.4 ->
+// 11.4 (13.2), 8192 x 22016 42.8 -> 32.6 (38.2), 16384 x 8192 30.0 -> 25.6
+// (26.4), 4096 x 8192 9.7 -> 9.4 (9.1); at K = 14336, 112 whole units, it is
+// 3% behind walking in step (16384 columns 42.4 -> 43.7; 45.3).
 // A4: the unit holds FEW's four rows of A alone, so that two workgroups fit a
 // CU: for grids of more than one round (gemm_w8a16_few).
 constexpr int FEW_LDS = 160 * 1024;
@@ -1719,8 +1720,8 @@ G950_W8A16_SKINNY(f16, g950::GEMM_F16)
 // int8 weights, up to four rows of A, more columns than one round of the CUs
 // holds: 32 columns per workgroup, two workgroups per CU.  One row of A (us;
 // 64 columns and one workgroup per CU -> this; the register-loading kernel):
-// 100000 x 4096 93.1 -> 65.7 (84.6), 50000 x 8192 92.9 -> 69.4 (74.5), 20000 x
-// 4096 25.3 -> 17.5 (21.9).
+// 100000 x 4096 93.6 -> 65.3 (84.5), 50000 x 8192 93.8 -> 69.8 (74.5), 20000 x
+// 4096 25.2 -> 17.6 (22.0).
 #define G950_W8A16_FEW(TY, MODE)                                                                       \
   extern "C" __global__ __launch_bounds__(512) void g950_gemm_w8a16_few_##TY(const g950::GemmArgs p) { \
     __shared__ __attribute__((aligned(1024))) char lds[80 * 1024];                                     \
